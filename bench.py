@@ -42,7 +42,7 @@ RH_NEAR_FLOPS_PER_QP = 65
 # other sources or another launch shape is not reported.
 TRAFFIC_SOURCE = 'profiles/far_p2p_H_two_surface_442k_pmc_traffic.md'
 TRAFFIC_KERNEL_SOURCES = {
-    'far_p2p_f32_kernel<H>': ('tectosaur_amd/csrc/far_p2p.hip', 'tectosaur_amd/csrc/far_pair.h'),
+    'far_tri_kernel<H>': ('tectosaur_amd/csrc/far_tri.h', 'tectosaur_amd/csrc/far_pair.h'),
     'bsr9_kernel': ('tectosaur_amd/csrc/sparse.hip',)}
 
 
@@ -629,10 +629,12 @@ def main():
             steps = args.steps if (K == 'elasticH3' and prec == 'f32') else 1
             dt, out, k_dt = time_matvec(op, v_dev, prec, steps, args.warmup if steps > 1 else 1)
             outs[prec] = out.cpu().numpy()
-            tc = op.engine.tile_cfg[prec]
+            # 256 lanes (64 observation triangles, four source tiles at a
+            # time), points per triangle, source chunks
+            chunks = op.tri.plan.chunks[op.tri.prec_id(prec)]
             res[prec] = {'pair_evals_per_s': pe / dt, 'ms_per_matvec': dt * 1e3,
                          'nbody_ms': k_dt * 1e3,
-                         'tile': [tc.block, tc.obs_per_lane, tc.src_chunks, tc.flags]}
+                         'tile': [256, op.nq, chunks]}
             print('# %s %s: %.3f ms/matvec, %.3e pair-evals/s' % (K, prec, dt * 1e3, pe / dt),
                   flush=True)
         res['f32_vs_f64_rel_l2'] = float(np.linalg.norm(outs['f32'] - outs['f64']) /
@@ -652,7 +654,7 @@ def main():
     flops = 102.0 * pe
     achieved = flops / kt / 1e12
     H_tile = per_kernel['elasticH3']['f32']['tile']
-    traffic, traffic_src = profiled_traffic('far_p2p_f32_kernel<H>', H_tile)
+    traffic, traffic_src = profiled_traffic('far_tri_kernel<H>', H_tile)
     line = {
         'metric': 'H-kernel pair-evals/s + served-solve p50/p99 vs plain FP64, at 1e-8 residual',
         'value': pe / H_dt,
@@ -674,8 +676,9 @@ def main():
         'roofline': {'bound': 'valu', 'achieved': achieved, 'peak': PEAK_FP32_TFLOPS,
                      'unit': 'TFLOP/s', 'frac': achieved / PEAK_FP32_TFLOPS,
                      'traffic': traffic, 'traffic_source': traffic_src,
-                     'algorithmic_bytes': int(n * 3 * (24 + 48 + 24 * H_tile[2])),
-                     'kernel': 'far_p2p_f32_kernel<H>', 'kernel_ms': kt * 1e3,
+                     # observation points and origins, source records, partial sums
+                     'algorithmic_bytes': int(n * (48 + 24 + 112 + 72 * H_tile[2])),
+                     'kernel': 'far_tri_kernel<H>', 'kernel_ms': kt * 1e3,
                      'kernel_timing': 'HIP events around the N-body launch inside the %d '
                                       'timed matvecs' % args.steps,
                      'tile': H_tile, 'flops_per_pair': 102},

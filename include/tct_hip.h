@@ -190,6 +190,72 @@ typedef struct {
 int tct_far_p2p_batched(int kernel, const double *params_host, int block, int obs_per_lane,
                         int n_seg, const tct_far_segment *segs, void *stream);
 
+/* ---------------- Triangle-to-triangle farfield ---------------------------
+ * farfield_tris_to_tris{K} (tectosaur/matrix_free.cl:19-107) for rules of 3
+ * (equal weights) or 4 points, all seven kernels: one lane holds the points
+ * of one observation triangle and walks whole source triangles, so what is
+ * constant over a flat triangle is formed once (far_tri.h).  A plan holds one
+ * operator's layout; every pointer is dev memory of the caller.
+ *   n_obs, n_obs_pad: observation triangles, padded to a multiple of 64;
+ *   n_src, n_tiles:   source triangles, tiles of TCT_TRI_TILE of them;
+ *   qw, phi:          rule weights [nq] and basis values [nq][3];
+ *   eps2, group_extent: as tct_far_p2p, with one origin per observation
+ *                     triangle and one per source tile;
+ *   chunks[prec]:     source chunks (1 <= chunks <= n_tiles) of each
+ *                     precision: partial[prec] is [chunks][out][n_obs_pad],
+ *                     out = 3 nq (U, T, A, H, RT), 9 (RH) or 3 + 3 nq (RA);
+ *   flags:            bit 0 keeps the r2 test on every tile;
+ *   obs32/64 [3 nq + 3][n_obs_pad], obs_org [3][n_obs_pad],
+ *   rec32/64 [n_tiles TCT_TRI_TILE][words], src_org [n_tiles][3]: written by
+ *                     tct_tri_pack (words = tct_tri_words(kernel, nq));
+ *   obs_tri, src_tri: DOF-space triangle of each packed position;
+ *   obs_jac, src_jac: Jacobian (2 area) of each packed position;
+ *   obs_curl, src_curl [.][9]: basis surface curls by DOF-space triangle
+ *                     (RA, RH: obs; RT, RH: src; else NULL). */
+#define TCT_TRI_TILE 16
+
+typedef struct {
+    int32_t kernel, nq;
+    double params[2];
+    double qw[4];
+    double phi[12];
+    int64_t n_obs, n_obs_pad, n_src, n_tiles;
+    double eps2, group_extent;
+    int32_t chunks[2];
+    int32_t flags, reserved;
+    float *obs32;
+    double *obs64;
+    double *obs_org;
+    float *rec32;
+    double *rec64;
+    double *src_org;
+    const int32_t *obs_tri, *src_tri;
+    const double *obs_jac, *src_jac;
+    const double *obs_curl, *src_curl;
+    double *partial[2];
+} tct_tri_plan;
+
+/* Words of a source triangle's record, and outputs per observation triangle
+ * (0 for a kernel or rule without this form). */
+int tct_tri_words(int kernel, int nq);
+int tct_tri_outputs(int kernel, int nq);
+/* Workgroups of the N-body (64 observation triangles by one chunk) that a CU
+ * holds at once: a property of the compiled kernel, for the choice of chunks. */
+int tct_tri_resident(int kernel, int nq, int prec, int *blocks);
+/* Geometry into the plan's layout: quadrature points [n][nq][3] and unit
+ * normals [n][3] of both sides in packed order. */
+int tct_tri_pack(const tct_tri_plan *plan, const double *obs_pts, const double *obs_ns,
+                 const double *src_pts, const double *src_ns, void *stream);
+/* The three steps of a matvec out = K v (v, out: dev, 9 doubles a triangle):
+ * strengths into the records, the N-bodies of n plans (one kernel, rule and
+ * constants) in one launch per 16, and the Galerkin scatter of the sums. */
+int tct_tri_gather(const tct_tri_plan *plan, int prec, const double *v, void *stream);
+int tct_tri_nbody(int n, const tct_tri_plan *const *plans, int prec, void *stream);
+int tct_tri_scatter(const tct_tri_plan *plan, int prec, double *out, void *stream);
+/* All three. */
+int tct_tri_matvec(const tct_tri_plan *plan, int prec, const double *v, double *out,
+                   void *stream);
+
 /* Sum of the chunk partials: out [n][3] f64 (point order of the packing). */
 int tct_far_reduce_pts(int64_t n, int64_t n_obs_pad, int chunks, const double *partial,
                        double *out, void *stream);

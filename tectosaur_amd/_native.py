@@ -22,6 +22,7 @@ KERNEL_IDS = {
 F32, F64 = 0, 1
 GROUP = 64
 REC = 12
+TRI_TILE = 16
 
 
 class TctError(RuntimeError):
@@ -41,6 +42,20 @@ class FarSegment(ctypes.Structure):
 class TileCfg(ctypes.Structure):
     _fields_ = [('block', ctypes.c_int32), ('obs_per_lane', ctypes.c_int32),
                 ('src_chunks', ctypes.c_int32), ('flags', ctypes.c_int32)]
+
+
+class TriPlan(ctypes.Structure):
+    """tct_tri_plan: the layout of one triangle-to-triangle operator."""
+    _fields_ = [('kernel', ctypes.c_int32), ('nq', ctypes.c_int32),
+                ('params', ctypes.c_double * 2), ('qw', ctypes.c_double * 4),
+                ('phi', ctypes.c_double * 12), ('n_obs', ctypes.c_int64),
+                ('n_obs_pad', ctypes.c_int64), ('n_src', ctypes.c_int64),
+                ('n_tiles', ctypes.c_int64), ('eps2', ctypes.c_double),
+                ('group_extent', ctypes.c_double), ('chunks', ctypes.c_int32 * 2),
+                ('flags', ctypes.c_int32), ('reserved', ctypes.c_int32)] + \
+        [(k, ctypes.c_void_p) for k in
+         ('obs32', 'obs64', 'obs_org', 'rec32', 'rec64', 'src_org', 'obs_tri', 'src_tri',
+          'obs_jac', 'src_jac', 'obs_curl', 'src_curl')] + [('partial', ctypes.c_void_p * 2)]
 
 
 _vp = ctypes.c_void_p
@@ -63,6 +78,14 @@ SIGNATURES = {
     'tct_far_p2p': [_int, _int, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _dbl, _dbl, _vp, _vp,
                     _vp],
     'tct_far_p2p_batched': [_int, _vp, _int, _int, _int, _vp, _vp],
+    'tct_tri_words': [_int, _int],
+    'tct_tri_outputs': [_int, _int],
+    'tct_tri_resident': [_int, _int, _int, _vp],
+    'tct_tri_pack': [_vp, _vp, _vp, _vp, _vp, _vp],
+    'tct_tri_gather': [_vp, _int, _vp, _vp],
+    'tct_tri_nbody': [_int, _vp, _int, _vp],
+    'tct_tri_scatter': [_vp, _int, _vp, _vp],
+    'tct_tri_matvec': [_vp, _int, _vp, _vp, _vp],
     'tct_far_reduce_pts': [_i64, _i64, _int, _vp, _vp, _vp],
     'tct_tree_p2m': [_int, _int, _int, _i64, _i64, _vp, _vp, _vp, _vp, _vp],
     'tct_tree_m2m': [_int, _int, _int, _int, _int, _int, _int, _vp, _vp, _vp],

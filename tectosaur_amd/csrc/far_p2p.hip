@@ -480,24 +480,6 @@ __global__ void pack_src_kernel(int64_t n, const double *__restrict__ pts,
     }
 }
 
-// Strength scale and per-source extras for the point kernels.
-struct StrengthConsts {
-    double scale;     // multiplies the raw strength
-    double x0, x1;    // e0 = x0 (n.s'), e1 = x1 (n.s')
-};
-
-inline StrengthConsts strength_consts(int kid, const double *params) {
-    ElasticConsts c = elastic_consts(params);
-    StrengthConsts s{1.0, 0.0, 0.0};
-    switch (kid) {
-    case TCT_U: s.scale = c.CsU1; break;
-    case TCT_T: s.scale = c.CsT1; s.x0 = 1.0; break;
-    case TCT_A: s.scale = c.CsT1; break;
-    case TCT_H: s.scale = c.CsH0; s.x0 = c.CsH2; s.x1 = 3.0 * c.CsH1; break;
-    }
-    return s;
-}
-
 template <typename T>
 __device__ __forceinline__ void write_strength(T *r, double s0, double s1, double s2,
                                                const StrengthConsts &sc) {
@@ -540,8 +522,6 @@ __global__ void gather_tris_kernel(int64_t n_pts, int64_t n_pad, int nq,
     }
     write_strength<T>(rec + i * R, s[0], s[1], s[2], sc);
 }
-
-__device__ __forceinline__ int levi3(int i, int j, int k) { return (i - j) * (j - k) * (k - i) / 2; }
 
 // Surface-curl kernels: per source point the record fields that carry the
 // source triangle's surface curl S[d][I] = sum_b curl[b][I] v[9t+3b+d]

@@ -282,4 +282,25 @@ inline KConst<T> kernel_consts(int kid, const double *params, double eps2) {
     return k;
 }
 
+// Strength scale and per-source extras for the point kernels.
+struct StrengthConsts {
+    double scale;     // multiplies the raw strength
+    double x0, x1;    // e0 = x0 (n.s'), e1 = x1 (n.s')
+};
+
+inline StrengthConsts strength_consts(int kid, const double *params) {
+    ElasticConsts c = elastic_consts(params);
+    StrengthConsts s{1.0, 0.0, 0.0};
+    switch (kid) {
+    case TCT_U: s.scale = c.CsU1; break;
+    case TCT_T: s.scale = c.CsT1; s.x0 = 1.0; break;
+    case TCT_A: s.scale = c.CsT1; break;
+    case TCT_H: s.scale = c.CsH0; s.x0 = c.CsH2; s.x1 = 3.0 * c.CsH1; break;
+    }
+    return s;
+}
+
+// Levi-Civita symbol of (i, j, k) in {0, 1, 2}^3.
+__device__ __forceinline__ int levi3(int i, int j, int k) { return (i - j) * (j - k) * (k - i) / 2; }
+
 }  // namespace tct

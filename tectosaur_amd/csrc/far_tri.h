@@ -1,0 +1,600 @@
+// Triangle-to-triangle farfield N-body: the pair body of one (observation
+// triangle, source triangle) pair, shared by the FP32 and FP64 units
+// far_tri_f32.hip and far_tri_f64.hip.
+//
+// Reference semantics: farfield_tris_to_tris{K} (tectosaur/matrix_free.cl:
+// 19-107) with the kernel bodies of tectosaur/kernels/kernels.cl: every
+// quadrature point of one triangle against every one of the other, pairs at
+// r2 == 0 skipped.
+//
+// What bounds it: VALU issue.  The point N-body (far_p2p.hip) evaluates every
+// pair of points by itself; here a lane holds the NQ points of one
+// observation triangle and walks whole source triangles, so what is constant
+// over a flat triangle is formed once per triangle pair or once per point:
+//   * n . D is the same for the NQ points of a source triangle, m . D for
+//     those of an observation triangle, m . n for the pair, m . s for the
+//     source point (T, A, H, RT, RA);
+//   * terms along n are summed as scalars over the source triangle (T, H);
+//   * the surface curls of RH are constant on both triangles, so a triangle
+//     pair needs only 7 moments, sum 1/r and sum D_k D_l / r^3, and one
+//     contraction with the source curl (RH); RT's 1/r term likewise;
+//   * U keeps its two terms in separate sums, scaled once per tile.
+// VALU instructions per point pair with a three-point rule, point form ->
+// this: H 54 -> 39, RH 40 -> 23, T 31 -> 27, A 30 -> 26, RT 27 -> 24,
+// RA 26 -> 23, U 20 -> 19.
+#pragma once
+#include "far_pair.h"
+
+namespace tct {
+
+constexpr int TT = TCT_TRI_TILE;   // source triangles per tile (one origin)
+
+// Rules of NQ = 3 points have equal weights.
+template <int NQ>
+constexpr bool equal_w() { return NQ == 3; }
+
+// Record of one source triangle: a block of SW words per point, so that a
+// point is read with whole 16-byte vectors, and the words of the triangle in
+// the blocks' spare words or after them:
+//   U, A, RA: [y s - -]              T: [y s e0 n_j]        H: [y s e0 e1] .. n
+//   RT:       [y s n_j e_j]          RH: [y G_j] .. G_3 to G_8
+// (n_j: component j of the normal, in the blocks of the first three points).
+template <int KID>
+constexpr int tri_sw() { return KID == TCT_RH ? 4 : 8; }
+template <int KID, int NQ>
+constexpr int tri_words() {
+    return tri_sw<KID>() * NQ + (KID == TCT_H ? 4 : (KID == TCT_RH ? 8 : 0));
+}
+template <int KID, int NQ>
+constexpr int tri_n_word(int d) {
+    return KID == TCT_T ? 8 * d + 7 : (KID == TCT_RT ? 8 * d + 6 : 8 * NQ + d);
+}
+constexpr int tri_e_word(int d) { return 8 * d + 7; }                  // RT
+template <int NQ>
+constexpr int tri_g_word(int a) { return a < 3 ? 4 * a + 3 : 4 * NQ + a - 3; }   // RH
+// Outputs per observation triangle: NQ 3-vectors; RH the 9 sums weighted by
+// the observation rule; RA one weighted 3-vector and NQ 3-vectors.
+template <int KID, int NQ>
+constexpr int tri_out() { return KID == TCT_RH ? 9 : (KID == TCT_RA ? 3 + 3 * NQ : 3 * NQ); }
+// Accumulators kept through a tile.
+template <int KID, int NQ>
+constexpr int tri_acc() {
+    return KID == TCT_U ? 6 * NQ
+           : KID == TCT_A ? 4 * NQ
+           : KID == TCT_H ? 5 * NQ
+           : KID == TCT_RA ? 6 + 3 * NQ
+           : KID == TCT_RH ? 18
+                           : 3 * NQ;
+}
+template <int KID>
+constexpr bool tri_obs_normal() { return KID == TCT_A || KID == TCT_H || KID == TCT_RA; }
+template <int KID>
+constexpr bool tri_src_normal() { return KID == TCT_T || KID == TCT_H || KID == TCT_RT; }
+
+// Kernel constants, and the rule weights relative to the last one: rw[q] for
+// one rule, ww[p NQ + q] for products.
+template <typename T, int NQ>
+struct TriConst {
+    T c0, c1, c2, c3, c4, eps2;
+    T rw[NQ], ww[NQ * NQ];
+};
+
+// Words [w, w + SW) of a record (w a multiple of the vector length).
+template <int SW, typename T>
+__device__ __forceinline__ void tri_load(const T *r, int w, T (&q)[SW]) {
+    constexpr int VW = 16 / sizeof(T);
+    typedef T vec __attribute__((ext_vector_type(VW)));
+#pragma unroll
+    for (int v = 0; v < SW / VW; ++v) {
+        const vec f = *(const vec *)(r + w + v * VW);
+#pragma unroll
+        for (int c = 0; c < VW; ++c) q[v * VW + c] = f[c];
+    }
+}
+
+// What a triangle pair starts from: the first point's block, the normal and
+// RT's curl term of the source triangle.
+template <int KID, typename T>
+struct TriHead {
+    T q[tri_sw<KID>()], n[3], e[3];
+};
+template <int KID, int NQ, typename T>
+__device__ __forceinline__ void tri_head(const T *r, TriHead<KID, T> &h) {
+    tri_load<tri_sw<KID>(), T>(r, 0, h.q);
+    if constexpr (tri_src_normal<KID>())
+#pragma unroll
+        for (int d = 0; d < 3; ++d) h.n[d] = r[tri_n_word<KID, NQ>(d)];
+    if constexpr (KID == TCT_RT)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) h.e[d] = r[tri_e_word(d)];
+}
+
+// One observation triangle (points x, normal m) against one source triangle
+// (record r, in LDS, its head already in h): acc += its terms, and h becomes
+// the head of the record `next`.  The source points come one after another,
+// fenced from each other, so few of them are in registers at a time; each
+// one's words are read while the point before it computes.  Every fused
+// multiply-add is written out, as in pair_eval, so every copy of the body
+// performs the same operations.
+template <int KID, int NQ, typename T, bool MASK>
+__device__ __forceinline__ void tri_pair(const T (&x)[NQ][3], const T (&m)[3], const T *r,
+                                         const T *next, const TriConst<T, NQ> &k,
+                                         TriHead<KID, T> &h, T *acc) {
+#pragma clang fp contract(off)
+    constexpr bool EQ = equal_w<NQ>();
+    constexpr int SW = tri_sw<KID>();
+    T an[NQ], nt[NQ], s0 = T(0), s2[6], G[9];
+    const T n[3] = {h.n[0], h.n[1], h.n[2]}, e[3] = {h.e[0], h.e[1], h.e[2]};
+    T mn0 = T(0), mn1 = T(0);
+    if constexpr (KID == TCT_H) {
+        const T mn = dot3(m[0], m[1], m[2], n[0], n[1], n[2]);
+        mn0 = k.c0 * mn;
+        mn1 = k.c1 * mn;
+    }
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) {
+        T q[SW];
+#pragma unroll
+        for (int w = 0; w < SW; ++w) q[w] = h.q[w];
+        if (j + 1 < NQ) {
+            tri_load<SW, T>(r, SW * (j + 1), h.q);
+        } else {
+            if constexpr (KID == TCT_RH)
+#pragma unroll
+                for (int a = 0; a < 9; ++a) G[a] = r[tri_g_word<NQ>(a)];
+            tri_head<KID, NQ, T>(next, h);
+        }
+        const T *s = q + 3;
+        // the same for every observation point: m . D, m . s and products
+        T bm = T(0), sm = T(0), sm4 = T(0), e1b = T(0), b4 = T(0), si = T(0);
+        if constexpr (tri_obs_normal<KID>())
+            bm = dot3(m[0], m[1], m[2], q[0] - x[0][0], q[1] - x[0][1], q[2] - x[0][2]);
+        if constexpr (KID == TCT_H || KID == TCT_A)
+            sm = dot3(m[0], m[1], m[2], s[0], s[1], s[2]);
+        if constexpr (KID == TCT_H) {
+            sm4 = k.c4 * sm;
+            sm = k.c0 * sm;
+            e1b = q[7] * bm;
+            b4 = k.c4 * bm;
+        }
+#pragma unroll
+        for (int p = 0; p < NQ; ++p) {
+            const T D[3] = {q[0] - x[p][0], q[1] - x[p][1], q[2] - x[p][2]};
+            const T r2 = dot3(D[0], D[1], D[2], D[0], D[1], D[2]);
+            const T invr = MASK ? rsq_masked(r2, k.eps2) : rsq_plain(r2);
+            const T w = invr * invr;
+            // n . D, the same for every source point
+            if constexpr (tri_src_normal<KID>())
+                if (j == 0) an[p] = dot3(n[0], n[1], n[2], D[0], D[1], D[2]);
+            if constexpr (KID == TCT_RH) {
+                const T iw = EQ ? invr : invr * k.ww[p * NQ + j];
+                const T i3 = iw * w;
+                const T e0 = i3 * D[0], e1 = i3 * D[1], e2 = i3 * D[2];
+                if (p == 0 && j == 0) {
+                    s0 = iw;
+                    s2[0] = e0 * D[0];
+                    s2[1] = e0 * D[1];
+                    s2[2] = e0 * D[2];
+                    s2[3] = e1 * D[1];
+                    s2[4] = e1 * D[2];
+                    s2[5] = e2 * D[2];
+                } else {
+                    s0 = s0 + iw;
+                    s2[0] = fma_t(e0, D[0], s2[0]);
+                    s2[1] = fma_t(e0, D[1], s2[1]);
+                    s2[2] = fma_t(e0, D[2], s2[2]);
+                    s2[3] = fma_t(e1, D[1], s2[3]);
+                    s2[4] = fma_t(e1, D[2], s2[4]);
+                    s2[5] = fma_t(e2, D[2], s2[5]);
+                }
+                continue;
+            }
+            const T i3 = invr * w;
+            if constexpr (KID == TCT_U) {
+                const T b = i3 * dot3(D[0], D[1], D[2], s[0], s[1], s[2]);
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    acc[6 * p + d] = fma_t(invr, s[d], acc[6 * p + d]);
+                    acc[6 * p + 3 + d] = fma_t(b, D[d], acc[6 * p + 3 + d]);
+                }
+            } else if constexpr (KID == TCT_T) {
+                const T ds = dot3(D[0], D[1], D[2], s[0], s[1], s[2]);
+                const T al = k.c0 * i3;
+                const T be = -al * an[p];
+                const T g = ((i3 * w) * an[p]) * ds;
+                const T de = fma_t(al, q[6], -g);
+                nt[p] = j == 0 ? al * ds : fma_t(al, ds, nt[p]);
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    acc[3 * p + d] = fma_t(be, s[d], acc[3 * p + d]);
+                    acc[3 * p + d] = fma_t(de, D[d], acc[3 * p + d]);
+                }
+            } else if constexpr (KID == TCT_A) {
+                const T ds = dot3(D[0], D[1], D[2], s[0], s[1], s[2]);
+                const T al = k.c0 * i3;
+                const T be = al * bm;
+                const T de = fma_t(al, sm, ((i3 * w) * bm) * ds);
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    acc[4 * p + d] = fma_t(be, s[d], acc[4 * p + d]);
+                    acc[4 * p + d] = fma_t(de, D[d], acc[4 * p + d]);
+                }
+                acc[4 * p + 3] = fma_t(i3, ds, acc[4 * p + 3]);
+            } else if constexpr (KID == TCT_H) {
+                const T c = dot3(s[0], s[1], s[2], D[0], D[1], D[2]);
+                const T wa = w * an[p];
+                const T wbc = (w * bm) * c;
+                acc[5 * p + 3] = fma_t(i3, q[6], acc[5 * p + 3]);
+                acc[5 * p + 4] = fma_t(i3, wa * c, acc[5 * p + 4]);
+                const T ni = fma_t(k.c1, wbc, sm);
+                nt[p] = j == 0 ? i3 * ni : fma_t(i3, ni, nt[p]);
+                const T inner = fma_t(T(-15), wbc, sm4);
+                const T DT = (i3 * w) * fma_t(an[p], inner, fma_t(c, mn1, e1b));
+                const T ST = i3 * fma_t(wa, b4, mn0);
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    acc[5 * p + d] = fma_t(D[d], DT, acc[5 * p + d]);
+                    acc[5 * p + d] = fma_t(s[d], ST, acc[5 * p + d]);
+                }
+            } else if constexpr (KID == TCT_RT) {
+                const T iw = EQ ? invr : invr * k.rw[j];
+                const T iw3 = EQ ? i3 : iw * w;
+                const T cd = (k.c0 * iw3) * dot3(D[0], D[1], D[2], e[0], e[1], e[2]);
+                const T cs = i3 * an[p];
+                nt[p] = j == 0 ? iw : nt[p] + iw;
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    acc[3 * p + d] = fma_t(cd, D[d], acc[3 * p + d]);
+                    acc[3 * p + d] = fma_t(cs, s[d], acc[3 * p + d]);
+                }
+            } else {
+                // RA: acc = [sum w_p s/r (3), sum w_p (D.s) D/r^3 (3),
+                // per point sum (m.D) s/r^3 (3 NQ)]
+                const T iw = EQ ? invr : invr * k.rw[p];
+                const T iw3 = EQ ? i3 : iw * w;
+                const T cd = iw3 * dot3(D[0], D[1], D[2], s[0], s[1], s[2]);
+                const T cs = i3 * bm;
+                si = p == 0 ? iw : si + iw;
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    acc[3 + d] = fma_t(cd, D[d], acc[3 + d]);
+                    acc[6 + 3 * p + d] = fma_t(cs, s[d], acc[6 + 3 * p + d]);
+                }
+            }
+        }
+        if constexpr (KID == TCT_RA)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) acc[d] = fma_t(si, s[d], acc[d]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (KID == TCT_RH) {
+        // acc[0..9) += s0 G; acc[9..18) += S2 G
+#pragma unroll
+        for (int a = 0; a < 9; ++a) acc[a] = fma_t(s0, G[a], acc[a]);
+        const T S[3][3] = {{s2[0], s2[1], s2[2]}, {s2[1], s2[3], s2[4]}, {s2[2], s2[4], s2[5]}};
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+#pragma unroll
+            for (int b = 0; b < 3; ++b)
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+                    acc[9 + 3 * a + c] = fma_t(S[a][b], G[3 * b + c], acc[9 + 3 * a + c]);
+    } else if constexpr (tri_src_normal<KID>()) {
+        // the sums along n (T, H) or of 1/r (RT)
+        constexpr int A = KID == TCT_H ? 5 : 3;
+#pragma unroll
+        for (int p = 0; p < NQ; ++p)
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+                acc[A * p + d] = fma_t(KID == TCT_T ? -nt[p] : nt[p],
+                                       KID == TCT_RT ? e[d] : n[d], acc[A * p + d]);
+    }
+}
+
+// The outputs of a tile's accumulators.
+template <int KID, int NQ, typename T>
+__device__ __forceinline__ void tri_fold(const T (&m)[3], const TriConst<T, NQ> &k, const T *acc,
+                                         T (&o)[tri_out<KID, NQ>()]) {
+#pragma clang fp contract(off)
+    if constexpr (KID == TCT_RH) {
+        const T tr = (acc[0] + acc[4]) + acc[8];
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+#pragma unroll
+            for (int b = 0; b < 3; ++b) {
+                T v = T(-2) * (acc[9 + 3 * a + b] + acc[3 * a + b]);
+                v = fma_t(k.c1, acc[3 * b + a], v);
+                if (a == b) v = fma_t(k.c0, tr, v);
+                o[3 * a + b] = v;
+            }
+    } else if constexpr (KID == TCT_RA) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) o[d] = fma_t(k.c0, acc[d], k.c1 * acc[3 + d]);
+#pragma unroll
+        for (int a = 0; a < 3 * NQ; ++a) o[3 + a] = acc[6 + a];
+    } else {
+#pragma unroll
+        for (int p = 0; p < NQ; ++p)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                if constexpr (KID == TCT_U) {
+                    o[3 * p + d] = fma_t(k.c0, acc[6 * p + d], acc[6 * p + 3 + d]);
+                } else if constexpr (KID == TCT_A) {
+                    o[3 * p + d] = fma_t(m[d], -k.c0 * acc[4 * p + 3], acc[4 * p + d]);
+                } else if constexpr (KID == TCT_H) {
+                    const T f = fma_t(k.c2, acc[5 * p + 4], acc[5 * p + 3]);
+                    o[3 * p + d] = fma_t(m[d], f, acc[5 * p + d]);
+                } else {
+                    o[3 * p + d] = acc[3 * p + d];
+                }
+            }
+    }
+}
+
+// One problem of a launch; several problems' N-bodies share one launch
+// through a table passed by value (segment s owns workgroups [blk0, next
+// blk0), observation block fastest, then chunk).
+template <typename T>
+struct TriSeg {
+    const T *obs;            // [3 NQ + 3][n_obs_pad]: points (FP32: local), normal
+    const double *obs_org;   // [3][n_obs_pad]
+    const T *rec;            // [n_tiles * TT][tri_words]
+    const double *src_org;   // [n_tiles][3]
+    double *partial;         // [chunks][tri_out][n_obs_pad]
+    double sep2;
+    float eps2;
+    int n_obs_pad, n_tiles, chunks, blk0;
+};
+constexpr int TRI_SEG_MAX = 16;
+template <typename T>
+struct TriSegTable {
+    int n;
+    TriSeg<T> s[TRI_SEG_MAX];
+};
+
+constexpr int TRI_WAVES = 4;   // waves of a workgroup, one source tile each at a time
+
+// Bytes of LDS: every wave's sums and its current source tile.
+template <int KID, int NQ, typename T>
+constexpr size_t tri_lds_bytes() {
+    return TRI_WAVES * (sizeof(double) * 64 * tri_out<KID, NQ>() +
+                        sizeof(T) * TT * tri_words<KID, NQ>());
+}
+
+// N-body.  A workgroup of four waves holds 64 observation triangles (one per
+// lane, the same in every wave) and one chunk of the source tiles; wave w
+// takes the chunk's tiles w, w + 4, ...  A wave stages its tile in LDS (the
+// next tile's words are loaded a tile ahead) and reads the records back with
+// broadcast reads, so they are VGPR operands.  The four waves' sums are added
+// in wave order through LDS, so a chunk has one partial sum whatever its
+// number of waves: a quarter of the partial sums that one wave per chunk
+// would write and the scatter would read.
+// FP32: points are stored relative to an FP64 origin, one per observation
+// triangle and one per source tile; a tile's sums are FP32, the sums over
+// tiles FP64.  Tiles whose origin is farther than sqrt(sep2) from every
+// lane's origin hold no pair with r2 <= eps2 and run without the test (the
+// last tile, which holds padding, keeps it).
+template <int KID, int NQ, typename T>
+__global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> segs,
+                                                               TriConst<T, NQ> kc) {
+    constexpr bool F32 = sizeof(T) == 4;
+    constexpr int RW = tri_words<KID, NQ>();
+    constexpr int NO = tri_out<KID, NQ>();
+    constexpr int NA = tri_acc<KID, NQ>();
+    constexpr int VW = 16 / sizeof(T);                  // words per 16-byte vector
+    constexpr int NVEC = TT * RW / VW;                  // vectors per tile
+    constexpr int NV = (NVEC + 63) / 64;                // per lane
+    typedef T vec __attribute__((ext_vector_type(VW)));
+    extern __shared__ double lds_raw[];
+    const int L = (int)blockIdx.x;
+    int si = 0;
+    while (si + 1 < segs.n && L >= segs.s[si + 1].blk0) ++si;
+    const TriSeg<T> &g = segs.s[si];
+    const int n_obs_pad = g.n_obs_pad, n_tiles = g.n_tiles, chunks = g.chunks;
+    const int obs_blocks = n_obs_pad / 64;
+    const int l = L - g.blk0;
+    const int ob = l % obs_blocks, ch = l / obs_blocks;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int lane = (int)threadIdx.x & 63;
+    const int t0 = (int)((int64_t)n_tiles * ch / chunks);
+    const int t1 = (int)((int64_t)n_tiles * (ch + 1) / chunks);
+    const int i = ob * 64 + lane;
+
+    // FP32 reads its points again for every tile (coalesced, and in cache by
+    // then), so they hold registers only in the tile's frame
+    T x[NQ][3], m[3];
+    if constexpr (!F32)
+#pragma unroll
+        for (int p = 0; p < NQ; ++p)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) x[p][d] = g.obs[(size_t)(3 * p + d) * n_obs_pad + i];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+        m[d] = tri_obs_normal<KID>() ? g.obs[(size_t)(3 * NQ + d) * n_obs_pad + i] : T(0);
+    TriConst<T, NQ> k = kc;
+    k.eps2 = F32 ? (T)g.eps2 : T(0);
+    if constexpr (F32) {
+        // an instruction that reads an SGPR is never dual-issued
+        asm volatile("" : "+v"(k.c0), "+v"(k.c1), "+v"(k.c2), "+v"(k.c4), "+v"(k.eps2));
+    }
+    // the wave's FP64 sums: in LDS, read and written once per tile
+    double *out = lds_raw + (size_t)wave * NO * 64 + lane;
+#pragma unroll
+    for (int a = 0; a < NO; ++a) out[a * 64] = 0.0;
+    T acc[NA];
+#pragma unroll
+    for (int a = 0; a < NA; ++a) acc[a] = T(0);
+
+    vec *tile = (vec *)(lds_raw + TRI_WAVES * NO * 64) + wave * NVEC;
+    const T *tw = (const T *)tile;
+    vec pre[NV];
+    const int tf = t0 + wave < t1 ? t0 + wave : t0;      // a chunk holds a tile
+    {
+        const vec *src = (const vec *)(g.rec + (size_t)tf * TT * RW);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int e = v * 64 + lane;
+            pre[v] = src[e < NVEC ? e : NVEC - 1];
+        }
+    }
+    for (int t = t0 + wave; t < t1; t += TRI_WAVES) {
+        // the previous tile's LDS reads were issued before these writes, and
+        // a wave's LDS operations complete in order
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int e = v * 64 + lane;
+            if (e < NVEC) tile[e] = pre[v];
+        }
+        {
+            const int tn = t + TRI_WAVES < t1 ? t + TRI_WAVES : t;
+            const vec *src = (const vec *)(g.rec + (size_t)tn * TT * RW);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                const int e = v * 64 + lane;
+                pre[v] = src[e < NVEC ? e : NVEC - 1];
+            }
+        }
+        // an index the compiler cannot see through: it would otherwise move
+        // these loads out of the loop and hold their registers through it
+        int ii = i;
+        asm volatile("" : "+v"(ii));
+        double dd[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            dd[d] = g.src_org[3 * t + d] - g.obs_org[(size_t)d * n_obs_pad + ii];
+        const bool close =
+            t == n_tiles - 1 || dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2] <= g.sep2;
+        if constexpr (F32)
+#pragma unroll
+            for (int p = 0; p < NQ; ++p)
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+                    x[p][d] = g.obs[(size_t)(3 * p + d) * n_obs_pad + ii] - (T)dd[d];
+        const bool mask = __any(close);
+        TriHead<KID, T> h;
+        tri_head<KID, NQ, T>(tw, h);
+        // one triangle per step: two (no register copies between a record's
+        // head and the next one's) measured 2-9% slower
+        if (mask) {
+#pragma unroll 1
+            for (int j = 0; j < TT; ++j)
+                tri_pair<KID, NQ, T, true>(x, m, tw + j * RW, tw + min(j + 1, TT - 1) * RW, k, h,
+                                           acc);
+        } else {
+#pragma unroll 1
+            for (int j = 0; j < TT; ++j)
+                tri_pair<KID, NQ, T, false>(x, m, tw + j * RW, tw + min(j + 1, TT - 1) * RW, k,
+                                            h, acc);
+        }
+        if constexpr (F32) {
+            T o[NO];
+            tri_fold<KID, NQ, T>(m, k, acc, o);
+#pragma unroll
+            for (int a = 0; a < NO; ++a) out[a * 64] += (double)o[a];
+#pragma unroll
+            for (int a = 0; a < NA; ++a) acc[a] = T(0);
+        }
+    }
+    if constexpr (!F32) {
+        T o[NO];
+        tri_fold<KID, NQ, T>(m, k, acc, o);
+#pragma unroll
+        for (int a = 0; a < NO; ++a) out[a * 64] = o[a];
+    }
+    __syncthreads();
+    const double *red = lds_raw;
+    double *po = g.partial + (size_t)ch * NO * n_obs_pad + ob * 64;
+    for (int e = (int)threadIdx.x; e < NO * 64; e += 64 * TRI_WAVES) {
+        double s = red[e];
+#pragma unroll
+        for (int w = 1; w < TRI_WAVES; ++w) s += red[w * NO * 64 + e];
+        po[(size_t)(e >> 6) * n_obs_pad + (e & 63)] = s;
+    }
+}
+
+// Launches the N-bodies of the problems of a table (one kernel, rule and
+// precision), and the workgroups of such a launch that a CU holds (defined
+// in far_tri_f32.hip and far_tri_f64.hip).
+template <typename T>
+int far_tri_launch(int kernel, int nq, const double *params, const double *qw,
+                   const TriSegTable<T> &t, unsigned blocks, hipStream_t st);
+template <typename T>
+int far_tri_resident(int kernel, int nq, int *blocks);
+
+template <int KID, int NQ, typename T>
+inline hipError_t far_tri_occ(int *blocks) {
+    const size_t lds = tri_lds_bytes<KID, NQ, T>();
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        blocks, (const void *)far_tri_kernel<KID, NQ, T>, 64 * TRI_WAVES, lds);
+}
+
+template <int KID, int NQ, typename T>
+inline void far_tri_go(const double *params, const double *qw, const TriSegTable<T> &t,
+                       unsigned blocks, hipStream_t st) {
+    const KConst<T> kc = kernel_consts<T>(KID, params, 0.0);
+    TriConst<T, NQ> k{kc.c0, kc.c1, kc.c2, kc.c3, kc.c4, T(0), {}, {}};
+    if (KID == TCT_RA) {
+        const ElasticConsts c = elastic_consts(params);
+        k.c0 = (T)c.CsRT1;
+        k.c1 = (T)c.CsRT0;
+    }
+    for (int p = 0; p < NQ; ++p) {
+        k.rw[p] = (T)(qw[p] / qw[NQ - 1]);
+        for (int j = 0; j < NQ; ++j)
+            k.ww[p * NQ + j] = (T)(qw[p] / qw[NQ - 1] * (qw[j] / qw[NQ - 1]));
+    }
+    const unsigned lds = (unsigned)tri_lds_bytes<KID, NQ, T>();
+    hipLaunchKernelGGL((far_tri_kernel<KID, NQ, T>), dim3(blocks), dim3(64 * TRI_WAVES), lds, st,
+                       t, k);
+}
+
+template <int NQ, typename T>
+inline void far_tri_kid(int kernel, const double *params, const double *qw,
+                        const TriSegTable<T> &t, unsigned blocks, hipStream_t st) {
+    switch (kernel) {
+    case TCT_U: far_tri_go<TCT_U, NQ, T>(params, qw, t, blocks, st); break;
+    case TCT_T: far_tri_go<TCT_T, NQ, T>(params, qw, t, blocks, st); break;
+    case TCT_A: far_tri_go<TCT_A, NQ, T>(params, qw, t, blocks, st); break;
+    case TCT_H: far_tri_go<TCT_H, NQ, T>(params, qw, t, blocks, st); break;
+    case TCT_RT: far_tri_go<TCT_RT, NQ, T>(params, qw, t, blocks, st); break;
+    case TCT_RA: far_tri_go<TCT_RA, NQ, T>(params, qw, t, blocks, st); break;
+    default: far_tri_go<TCT_RH, NQ, T>(params, qw, t, blocks, st); break;
+    }
+}
+
+template <int NQ, typename T>
+inline hipError_t far_tri_occ_kid(int kernel, int *blocks) {
+    switch (kernel) {
+    case TCT_U: return far_tri_occ<TCT_U, NQ, T>(blocks);
+    case TCT_T: return far_tri_occ<TCT_T, NQ, T>(blocks);
+    case TCT_A: return far_tri_occ<TCT_A, NQ, T>(blocks);
+    case TCT_H: return far_tri_occ<TCT_H, NQ, T>(blocks);
+    case TCT_RT: return far_tri_occ<TCT_RT, NQ, T>(blocks);
+    case TCT_RA: return far_tri_occ<TCT_RA, NQ, T>(blocks);
+    default: return far_tri_occ<TCT_RH, NQ, T>(blocks);
+    }
+}
+
+template <typename T>
+inline int far_tri_occ_nq(int kernel, int nq, int *blocks) {
+    const hipError_t e = nq == 3 ? far_tri_occ_kid<3, T>(kernel, blocks)
+                                 : far_tri_occ_kid<4, T>(kernel, blocks);
+    if (e != hipSuccess)
+        return set_error(TCT_EHIP, "far_tri: occupancy: %s", hipGetErrorString(e));
+    return TCT_OK;
+}
+
+template <typename T>
+inline int far_tri_nq(int kernel, int nq, const double *params, const double *qw,
+                      const TriSegTable<T> &t, unsigned blocks, hipStream_t st) {
+    if (nq == 3)
+        far_tri_kid<3, T>(kernel, params, qw, t, blocks, st);
+    else if (nq == 4)
+        far_tri_kid<4, T>(kernel, params, qw, t, blocks, st);
+    else
+        return set_error(TCT_EUNSUPPORTED, "far_tri: rule of %d points (3 or 4)", nq);
+    TCT_CHECK_LAUNCH("far_tri");
+    return TCT_OK;
+}
+
+}  // namespace tct

@@ -216,9 +216,21 @@ def run_batched(engines, block=256, obs_per_lane=1):
     """One launch for the FP32 N-bodies of several engines (same kernel and
     constants), each with its own layout and source chunks; every engine's
     partial-sum buffer gets what its own ``run('f32')`` would write.
+    Operators on the triangle layout (``tri_farfield.TriFarfield``) share a
+    launch of theirs; ``block`` and ``obs_per_lane`` are the point N-body's.
     Returns the partial-sum buffers."""
     if not engines:
         return []
+    tri = [e for e in engines if not isinstance(e, FarfieldEngine)]
+    if tri:
+        from . import tri_farfield
+        done = {}
+        for nq in sorted({t.nq for t in tri}):
+            group = [t for t in tri if t.nq == nq]
+            done.update(zip(map(id, group), tri_farfield.run_batched(group, 'f32')))
+        pts = [e for e in engines if id(e) not in done]
+        done.update(zip(map(id, pts), run_batched(pts, block, obs_per_lane)))
+        return [done[id(e)] for e in engines]
     e0 = engines[0]
     for e in engines[1:]:
         if e.kid != e0.kid or not np.array_equal(e.params, e0.params):

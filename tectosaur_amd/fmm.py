@@ -314,6 +314,8 @@ class FMMFarfieldOpImpl(TriToTriDirectFarfieldOp):
     FP64 arithmetic; ``dot_dev(..., prec='f64')`` also evaluates directly
     in FP64 (the exact operator) for residuals."""
 
+    _direct = False
+
     def __init__(self, nq_far, K_name, params, pts, tris, float_type, obs_subset, src_subset,
                  mac, pts_per_cell, order, plan=None, precisions=None):
         if K_name not in TREE_KERNELS:

@@ -105,7 +105,7 @@ class ConstrainedOperator:
         its result bit for bit.  The farfield must be the direct N-body
         (TriToTriDirectFarfieldOp)."""
         ff = getattr(self.A, 'farfield', None)
-        if ff is None or not hasattr(ff, '_gather') or not hasattr(ff, 'engine'):
+        if ff is None or not hasattr(ff, 'nbody_gather'):
             raise ValueError('split graphs need a direct farfield operator')
         n = self.shape[0]
         if self._gx is None:
@@ -135,11 +135,11 @@ class ConstrainedOperator:
 
     def _split_pre(self, prec):
         self.cm.dot_dev(self._gx, self._u)
-        self.A.farfield._gather(self._u, prec)
+        self.A.farfield.nbody_gather(self._u, prec)
 
     def _split_post(self, prec):
         ff = self.A.farfield
-        ff._scatter(prec, self._y)
+        ff.nbody_scatter(prec, self._y)
         self.A.nearfield.dot_dev(self._u, self._y, accumulate=True, prec=prec)
         self.cmT.dot_dev(self._y, self._gy)
 
@@ -156,7 +156,7 @@ class ConstrainedOperator:
 
     @property
     def nbody_engine(self):
-        return self.A.farfield.engine
+        return self.A.farfield.nbody_engine
 
     def has_graph(self, prec):
         return prec in self._graphs

@@ -25,6 +25,7 @@ import numpy as np
 import torch
 
 from . import _native as N
+from . import tri_farfield
 from .farfield import FarfieldEngine, morton_order, prec_of
 from .kernels import kernels as KERNELS
 from .quadrature import gauss2d_tri
@@ -81,6 +82,10 @@ def farfield_plan(nq_far, pts, tris, obs_subset, src_subset, curl):
 
 
 class TriToTriDirectFarfieldOp:
+    # whether the operator itself is evaluated by the direct N-body (the
+    # treecode operator only uses the point layout)
+    _direct = True
+
     def __init__(self, nq_far, K_name, params, pts, tris, float_type, obs_subset, src_subset,
                  tile_cfg=None, precisions=None, plan=None):
         K = KERNELS[K_name]
@@ -103,20 +108,40 @@ class TriToTriDirectFarfieldOp:
         self.device = dev
         if precisions is None:
             precisions = (self.prec,)
-        self.engine = FarfieldEngine(K_name, params, plan['o_pts'], plan['o_ns'], plan['s_pts'],
-                                     plan['s_ns'], precisions=precisions, device=dev,
-                                     tile_cfg=tile_cfg, extents=plan['extents'])
-        # source point k belongs to DOF-space triangle tri_of_pt[k]
-        self.tri_of_pt = N.upload(plan['tri_of_pt'], torch.int32, dev)
-        self.pt_of_tri = N.upload(plan['pt_of_tri'], torch.int32, dev)
-        self.qphi = N.upload(plan['phi'], torch.float64, dev)
-        self.wj_src = N.upload(plan['s_wj'], torch.float64, dev)
-        self.wj_obs = N.upload(plan['o_wj'], torch.float64, dev)
-        if self.curl:
-            self.curl_src = N.upload(plan['curl_src'], torch.float64, dev)
-            self.curl_obs = N.upload(plan['curl_obs'], torch.float64, dev)
+        self._args = (params, precisions, tile_cfg)
+        self._plan = plan
         self._plan_pts = (plan['o_pts'], plan['s_pts'])
+        self._engine = None
+        self.tri = None
         self.tree = None
+        # rules of three and four points run over whole triangles
+        # (far_tri.h); a caller's launch shape is one of the point N-body's
+        if self._direct and tile_cfg is None and tri_farfield.supports(self.q[1]):
+            self.tri = tri_farfield.TriFarfield(K_name, params, plan, dev)
+        else:
+            self.engine
+
+    @property
+    def engine(self):
+        """The point layout and N-body of this operator (built when first
+        used: the treecode, rules without a triangle form, and callers that
+        drive the point N-body themselves)."""
+        if self._engine is None:
+            params, precisions, tile_cfg = self._args
+            plan, dev = self._plan, self.device
+            self._engine = FarfieldEngine(self.K_name, params, plan['o_pts'], plan['o_ns'],
+                                          plan['s_pts'], plan['s_ns'], precisions=precisions,
+                                          device=dev, tile_cfg=tile_cfg, extents=plan['extents'])
+            # source point k belongs to DOF-space triangle tri_of_pt[k]
+            self.tri_of_pt = N.upload(plan['tri_of_pt'], torch.int32, dev)
+            self.pt_of_tri = N.upload(plan['pt_of_tri'], torch.int32, dev)
+            self.qphi = N.upload(plan['phi'], torch.float64, dev)
+            self.wj_src = N.upload(plan['s_wj'], torch.float64, dev)
+            self.wj_obs = N.upload(plan['o_wj'], torch.float64, dev)
+            if self.curl:
+                self.curl_src = N.upload(plan['curl_src'], torch.float64, dev)
+                self.curl_obs = N.upload(plan['curl_obs'], torch.float64, dev)
+        return self._engine
 
     def attach_tree(self, order=4, mac=3.0, pts_per_cell=64, plan=None, n_waves=None):
         """Add a treecode evaluation of this operator (kernels U3, RT3, RA3,
@@ -141,6 +166,24 @@ class TriToTriDirectFarfieldOp:
         self._scatter(prec, out_dev, part, self.tree.chunks)
         return out_dev
 
+    # one matvec in three steps: strengths, N-body, scatter.  A server runs
+    # the N-bodies of many operators in one launch between the other two.
+    @property
+    def nbody_engine(self):
+        return self.tri if self.tri is not None else self.engine
+
+    def nbody_gather(self, v_dev, prec):
+        if self.tri is not None:
+            self.tri.gather(v_dev, prec)
+        else:
+            self._gather(v_dev, prec)
+
+    def nbody_scatter(self, prec, out_dev):
+        if self.tri is not None:
+            self.tri.scatter(prec, out_dev)
+        else:
+            self._scatter(prec, out_dev)
+
     def _gather(self, v_dev, prec):
         e = self.engine
         if self.curl:
@@ -160,7 +203,7 @@ class TriToTriDirectFarfieldOp:
 
     @property
     def pair_evals(self):
-        return self.engine.pair_evals
+        return self.nbody_engine.pair_evals
 
     def dot_dev(self, v_dev, out_dev=None, prec=None, nbody_events=None):
         """Device matvec: v_dev float64 [n_src*9] -> float64 [n_obs*9].
@@ -175,13 +218,15 @@ class TriToTriDirectFarfieldOp:
             prec = 'f32'
         if out_dev is None:
             out_dev = torch.empty(self.shape[0], dtype=torch.float64, device=self.device)
-        self._gather(v_dev, prec)
+        if nbody_events is None and self.tri is not None:
+            return self.tri.matvec(v_dev, out_dev, prec)
+        self.nbody_gather(v_dev, prec)
         if nbody_events is not None:
             nbody_events[0].record()
-        self.engine.run(prec)
+        self.nbody_engine.run(prec)
         if nbody_events is not None:
             nbody_events[1].record()
-        self._scatter(prec, out_dev)
+        self.nbody_scatter(prec, out_dev)
         return out_dev
 
     def prepare(self, prec):
@@ -191,7 +236,7 @@ class TriToTriDirectFarfieldOp:
             self.tree.moments('f32')
             self.tree.partial
         else:
-            self.engine.partial('f32' if prec == 'tree' else prec)
+            self.nbody_engine.partial('f32' if prec == 'tree' else prec)
 
     def dot(self, v):
         v_dev = torch.as_tensor(np.ascontiguousarray(v, dtype=np.float64), device=self.device)

@@ -1,0 +1,183 @@
+"""Triangle-to-triangle farfield on the device (far_tri.h): the layout of one
+operator and the launches of a matvec.
+
+``TriFarfield`` packs whole triangles instead of single points: a lane of the
+N-body holds one observation triangle and walks source triangles, so what is
+constant over a flat triangle (normals, surface curls) is used once per
+triangle pair.  It serves rules of three points (equal weights) and four
+points; other rules keep the point layout of ``farfield.FarfieldEngine``.
+"""
+import ctypes
+
+import numpy as np
+import torch
+
+from . import _native as N
+from .kernels import kernels as KERNELS
+
+TILE = N.TRI_TILE
+LANES = 64
+# points of the rules with a triangle form: a lane keeps every point of its
+# triangle, its accumulators and a source triangle's record in registers,
+# and with seven points they no longer fit
+RULE_POINTS = (3, 4)
+
+
+def supports(qw):
+    """Whether a triangle rule with weights ``qw`` has a triangle form."""
+    return qw.shape[0] in RULE_POINTS and (qw.shape[0] != 3 or bool(np.all(qw == qw[0])))
+
+
+def origin_extent(p, counts):
+    """Largest distance of a point from its group's mean; the points [n, 3]
+    come in consecutive groups of ``counts`` (the last may be shorter)."""
+    n = p.shape[0]
+    start = np.arange(0, n, counts)
+    cnt = np.minimum(start + counts, n) - start
+    mean = np.add.reduceat(p, start, axis=0) / cnt[:, None]
+    d = p - np.repeat(mean, cnt, axis=0)
+    return float(np.sqrt(np.max(np.einsum('ij,ij->i', d, d))))
+
+
+def source_chunks(obs_blocks, n_tiles, resident):
+    """Source chunks of a launch of obs_blocks x chunks workgroups, of which
+    the chip holds ``resident`` at once, four waves each.  Sixteen rounds of
+    workgroups, whose loads and sums then overlap others' arithmetic (H FP32,
+    32,256 triangles: 7.97 ms in one round, 7.41 in four, 7.18 in sixteen),
+    but at least two tiles for every wave (RH FP32, 4,982 triangles: 137 us
+    with two, 139 with one, 154 with six); where that leaves part of the chip
+    idle, one tile (U FP32, 2,048 triangles: 33 us).  From the sizes and the
+    compiled kernel alone: the chunks set the summation order."""
+    c = min(-(-16 * resident // obs_blocks), n_tiles // 8)
+    if c * obs_blocks < resident:
+        c = min(-(-resident // obs_blocks), n_tiles // 4)
+    return max(1, c)
+
+
+_RESIDENT = {}
+
+
+def resident_blocks(kid, nq, prec_id):
+    """N-body workgroups the chip (256 CUs) holds at once."""
+    key = (kid, nq, prec_id)
+    if key not in _RESIDENT:
+        b = ctypes.c_int(0)
+        N.call('tct_tri_resident', kid, nq, prec_id, ctypes.byref(b))
+        _RESIDENT[key] = 256 * max(1, b.value)
+    return _RESIDENT[key]
+
+
+class TriFarfield:
+    """Device layout + launches of one operator.  ``plan``: the host arrays
+    of ``sparse_farfield_op.farfield_plan``."""
+
+    def __init__(self, K_name, params, plan, device):
+        K = KERNELS[K_name]
+        self.K = K
+        self.device = device
+        nq = plan['nq']
+        qw = np.asarray(plan['q'][1], dtype=np.float64)
+        o_pts, s_pts = plan['o_pts'], plan['s_pts']
+        self.n_obs, self.n_src = o_pts.shape[0] // nq, s_pts.shape[0] // nq
+        if self.n_obs == 0 or self.n_src == 0:
+            raise N.TctError('empty point set')
+        self.nq = nq
+        n_pad = -(-self.n_obs // LANES) * LANES
+        n_tiles = -(-self.n_src // TILE)
+        self.n_obs_pad, self.n_tiles = n_pad, n_tiles
+        self.n_out = N.lib().tct_tri_outputs(K.kid, nq)
+        words = N.lib().tct_tri_words(K.kid, nq)
+        same = s_pts is o_pts
+        up = lambda a: N.upload(a, None, device)
+        f64 = dict(dtype=torch.float64, device=device)
+        f32 = dict(dtype=torch.float32, device=device)
+        obs_of = np.empty(self.n_obs, dtype=np.int32)   # packed position -> triangle
+        obs_of[plan['pt_of_tri']] = np.arange(self.n_obs, dtype=np.int32)
+        jac = lambda wj: np.ascontiguousarray(wj[nq - 1::nq]) / qw[nq - 1]
+        t = {'obs32': torch.empty((3 * nq + 3) * n_pad, **f32),
+             'obs64': torch.empty((3 * nq + 3) * n_pad, **f64),
+             'obs_org': torch.empty(3 * n_pad, **f64),
+             'rec32': torch.empty(n_tiles * TILE * words, **f32),
+             'rec64': torch.empty(n_tiles * TILE * words, **f64),
+             'src_org': torch.empty(3 * n_tiles, **f64),
+             'obs_tri': up(obs_of), 'src_tri': up(plan['tri_of_pt'][::nq]),
+             'obs_jac': up(jac(plan['o_wj']))}
+        t['src_jac'] = t['obs_jac'] if same else up(jac(plan['s_wj']))
+        if K.surf_curl_obs:
+            t['obs_curl'] = up(plan['curl_obs'])
+        if K.surf_curl_src:
+            shared = K.surf_curl_obs and plan['curl_src'] is plan['curl_obs']
+            t['src_curl'] = t['obs_curl'] if shared else up(plan['curl_src'])
+        self._t = t
+        # rounding bound of one point stored against two different origins
+        self.group_extent = origin_extent(o_pts, nq) + origin_extent(s_pts, nq * TILE)
+        p = N.TriPlan(kernel=K.kid, nq=nq, n_obs=self.n_obs, n_obs_pad=n_pad, n_src=self.n_src,
+                      n_tiles=n_tiles, eps2=(8.0 * 2.0 ** -24 * self.group_extent) ** 2,
+                      group_extent=self.group_extent)
+        p.params[:] = [float(x) for x in params][:2]
+        p.qw[:nq] = qw.tolist()
+        p.phi[:3 * nq] = np.asarray(plan['phi'], dtype=np.float64).reshape(-1).tolist()
+        p.chunks[:] = [source_chunks(n_pad // LANES, n_tiles, resident_blocks(K.kid, nq, i))
+                       for i in (N.F32, N.F64)]
+        for k, v in t.items():
+            setattr(p, k, N.ptr(v))
+        self.plan = p
+        self._partial = {}
+        o, on = up(o_pts), up(plan['o_ns'][::nq])
+        s, sn = (o, on) if same else (up(s_pts), up(plan['s_ns'][::nq]))
+        N.call('tct_tri_pack', ctypes.addressof(p), N.ptr(o), N.ptr(on), N.ptr(s), N.ptr(sn),
+               N.stream_ptr())
+
+    @staticmethod
+    def prec_id(prec):
+        if prec not in ('f32', 'f64'):
+            raise ValueError('precision must be f32 or f64')
+        return N.F32 if prec == 'f32' else N.F64
+
+    def partial(self, prec):
+        """The partial sums of ``prec`` (allocated at the first use)."""
+        pid = self.prec_id(prec)
+        buf = self._partial.get(pid)
+        if buf is None:
+            buf = torch.empty(self.plan.chunks[pid] * self.n_out * self.n_obs_pad,
+                              dtype=torch.float64, device=self.device)
+            self._partial[pid] = buf
+            self.plan.partial[pid] = N.ptr(buf)
+        return buf
+
+    def gather(self, v_dev, prec):
+        N.call('tct_tri_gather', ctypes.addressof(self.plan), self.prec_id(prec), N.ptr(v_dev),
+               N.stream_ptr())
+
+    def run(self, prec):
+        """Launch the N-body; returns the partial sums."""
+        return run_batched([self], prec)[0]
+
+    def scatter(self, prec, out_dev):
+        self.partial(prec)
+        N.call('tct_tri_scatter', ctypes.addressof(self.plan), self.prec_id(prec),
+               N.ptr(out_dev), N.stream_ptr())
+
+    def matvec(self, v_dev, out_dev, prec):
+        pid = self.prec_id(prec)
+        if pid not in self._partial:
+            self.partial(prec)
+        N.call('tct_tri_matvec', ctypes.addressof(self.plan), pid, N.ptr(v_dev), N.ptr(out_dev),
+               N.stream_ptr())
+        return out_dev
+
+    @property
+    def pair_evals(self):
+        return self.n_obs * self.n_src * self.nq ** 2
+
+
+def run_batched(tris, prec='f32'):
+    """One launch for the N-bodies of several ``TriFarfield`` (same kernel,
+    rule and constants); every one's partial sums get what its own ``run``
+    would write.  Returns the partial-sum buffers."""
+    outs = [t.partial(prec) for t in tris]
+    if tris:
+        ptrs = (ctypes.c_void_p * len(tris))(*[ctypes.addressof(t.plan) for t in tris])
+        N.call('tct_tri_nbody', len(tris), ctypes.addressof(ptrs), TriFarfield.prec_id(prec),
+               N.stream_ptr())
+    return outs
