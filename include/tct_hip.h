@@ -353,6 +353,17 @@ int tct_pairs_integrate(int kernel, int64_t nq, const double *qx, const double *
                         const double *params_host, int lanes_per_pair, double *out,
                         void *stream);
 
+/* tct_pairs_integrate for a product rule: every point of the obs rule
+ * (qo [n_o][2], weights wo) with every one of the src rule (qs [n_s][2], ws),
+ * the points of gauss4d_tri (tectosaur/util/quadrature.py:47-60) in another
+ * order of summation.  check0 as there (1 and 2 both skip r2 == 0 and the
+ * points with equal parameters). */
+int tct_pairs_product(int kernel, int n_o, const double *qo, const double *wo, int n_s,
+                      const double *qs, const double *ws, const double *pts,
+                      const int32_t *tris, int64_t n_pairs, const int32_t *pairs,
+                      int pair_width, int check0, const double *params_host, double *out,
+                      void *stream);
+
 /* out[i] = a[i] - b[i] over n doubles (nearfield correction, tectosaur/
  * nearfield/nearfield_op.py:135-141). */
 int tct_sub_f64(int64_t n, const double *a, const double *b, double *out, void *stream);

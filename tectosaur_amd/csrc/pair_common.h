@@ -14,6 +14,10 @@ struct Tri {
     double curl[3][3];           // surface curl of the basis functions
 };
 
+// Vectors at their elements' alignment.
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+typedef int i3u __attribute__((ext_vector_type(3), aligned(4)));
+
 __device__ __forceinline__ int pmod3(int i) { return ((i % 3) + 3) % 3; }
 
 // tri_info of tectosaur/integral_primitives.cl:56-93 (+ surf_curl_basis
@@ -22,14 +26,20 @@ __device__ __forceinline__ int pmod3(int i) { return ((i % 3) + 3) % 3; }
 __device__ __forceinline__ void load_tri(Tri &t, const double *__restrict__ pts,
                                          const int32_t *__restrict__ tris, int idx, int clicks,
                                          int flip) {
+    // every lane gathers from lines of its own, one line a cycle: the three
+    // indices come in one load and a point in two
+    const i3u id = *(const i3u *)(tris + 3 * (size_t)idx);
     double v[3][3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         int fc = c;
         if (flip) fc = (c == 0) ? 1 : (c == 1 ? 0 : 2);
-        const int p = tris[3 * idx + pmod3(fc + clicks)];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) v[c][d] = pts[3 * p + d];
+        const int r = pmod3(fc + clicks);
+        const int p = r == 0 ? id.x : (r == 1 ? id.y : id.z);
+        const d2u xy = *(const d2u *)(pts + 3 * (size_t)p);
+        v[c][0] = xy.x;
+        v[c][1] = xy.y;
+        v[c][2] = pts[3 * (size_t)p + 2];
     }
     double s20[3], s21[3], un[3];
 #pragma unroll
@@ -59,6 +69,23 @@ __device__ __forceinline__ void load_tri(Tri &t, const double *__restrict__ pts,
         t.curl[0][s] = (-e2 + e1) * inv;
         t.curl[1][s] = e2 * inv;
         t.curl[2][s] = -e1 * inv;
+    }
+}
+
+// The Jacobian and surface curls of a triangle (rotated, flipped vertex
+// order) from its edges e1 = v1 - v0, e2 = v2 - v0; the vertices and the
+// normal stay unset.
+__device__ __forceinline__ void tri_from_edges(Tri &t, const double (&e1)[3],
+                                               const double (&e2)[3]) {
+    const double n0 = e1[1] * e2[2] - e1[2] * e2[1], n1 = e1[2] * e2[0] - e1[0] * e2[2],
+                 n2 = e1[0] * e2[1] - e1[1] * e2[0];
+    t.jac = sqrt(n0 * n0 + n1 * n1 + n2 * n2);
+    const double inv = 1.0 / t.jac;
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+        t.curl[0][s] = (e1[s] - e2[s]) * inv;
+        t.curl[1][s] = e2[s] * inv;
+        t.curl[2][s] = -e1[s] * inv;
     }
 }
 
@@ -143,5 +170,236 @@ __device__ __forceinline__ constexpr int sym6(int p, int t) {
 
 // Levi-Civita symbol of (i, j, k) in {0,1,2}^3.
 __device__ __forceinline__ int levi(int i, int j, int k) { return (i - j) * (j - k) * (k - i) / 2; }
+
+// The r = 0 test of a pair class (CK): CK_NONE for pairs that never touch;
+// CK_FULL skips r2 == 0 and the points whose obs and src parameters are
+// equal on pairs that are one triangle in one frame; CK_R2 skips r2 == 0
+// only, for rules with no point of equal obs and src parameters.
+constexpr int CK_NONE = 0, CK_FULL = 1, CK_R2 = 2;
+
+// Normals a kernel body reads: obs (m) and src (n).
+struct PairNormals {
+    double m[3], n[3];
+};
+
+// ---------------------------------------------------------------------------
+// From a pair's sums to its 81 outputs.  Memory wants whole lines: rows of
+// 648 bytes written lane by lane, or in runs of 72 or 216 bytes, reached
+// 2.2 to 2.5 TB/s, whole rows one after another 5.3 (710,704 rows).  So a wave
+// puts what its pairs' outputs are made of in LDS, a few pairs at a time, and
+// its lanes then form the outputs in the order of memory, each from a few
+// LDS words at offsets that a table gives for the 81 entries.
+//
+// The formulas (integral_primitives.cl:174-213, kernels.cl:29-98), with the
+// factor J = J_obs J_src in the packed sums, obs basis b, src basis e,
+// components d (obs) and f (src), curls o (obs) and s (src):
+//   U       sum[b][e][d f]
+//   T, A, H sum[b][d][e][f]
+//   RH      P[d f] (o_b . s_e) + A_bd s_ef + B_bf s_ed with P = -2 c0 (S2 +
+//           S0 I), A = c0 CsRH1 S0 o, B = c0 CsRH2 S0 o
+//   RT      C[b][d, f+2] s_e,f+1 - C[b][d, f+1] s_e,f+2 + (d = f) A3[b][e],
+//           C[b] = A2[b] + A1[b] I (the Levi-Civita sums written out)
+//   RA      the same with the sides exchanged and -A3.
+struct PairTable {
+    uint2 off[81];   // six byte-sized offsets per entry
+};
+
+// Doubles of one pair in LDS.
+template <int KID>
+constexpr int pack_size() {
+    return KID == TCT_U ? 54 : (KID <= TCT_H ? 81 : (KID == TCT_RH ? 42 : 37));
+}
+// Pairs in LDS at a time (GL lanes a pair).
+template <int KID, int GL>
+constexpr int pack_pairs() {
+    const int pw = 64 / GL, most = KID <= TCT_H ? 8 : 16;
+    return pw < most ? pw : most;
+}
+
+// Filled by the first 81 threads of a workgroup (a barrier before its use).
+template <int KID>
+__device__ __forceinline__ void fill_pair_table(PairTable &t) {
+    for (int i = (int)threadIdx.x; i < 81; i += (int)blockDim.x) {
+        const int b = i / 27, d = i / 9 % 3, e = i / 3 % 3, f = i % 3;
+        int o[6] = {0, 0, 0, 0, 0, 0};
+        if constexpr (KID == TCT_U) {
+            o[0] = (3 * b + e) * 6 + sym6(d, f);
+        } else if constexpr (KID <= TCT_H) {
+            o[0] = i;
+        } else if constexpr (KID == TCT_RH) {
+            // P 0-5, o.s 6-14, A 15-23, B 24-32, s 33-41
+            o[0] = sym6(d, f);
+            o[1] = 6 + 3 * b + e;
+            o[2] = 15 + 3 * b + d;
+            o[3] = 33 + 3 * e + f;
+            o[4] = 24 + 3 * b + f;
+            o[5] = 33 + 3 * e + d;
+        } else {
+            // C 0-17, A3 18-26, curls 27-35, zero 36
+            const int cb = KID == TCT_RT ? b : e, cd = KID == TCT_RT ? d : f;   // side of C
+            const int xb = KID == TCT_RT ? e : b, xd = KID == TCT_RT ? f : d;   // side of the curl
+            o[0] = 6 * cb + sym6(cd, (xd + 2) % 3);
+            o[1] = 27 + 3 * xb + (xd + 1) % 3;
+            o[2] = 6 * cb + sym6(cd, (xd + 1) % 3);
+            o[3] = 27 + 3 * xb + (xd + 2) % 3;
+            o[4] = d == f ? 18 + 3 * b + e : 36;
+        }
+        t.off[i] = make_uint2(o[0] | o[1] << 8 | o[2] << 16 | o[3] << 24, o[4] | o[5] << 8);
+    }
+}
+
+template <int KID>
+__device__ __forceinline__ double pair_entry(const double *p, uint2 o) {
+    if constexpr (KID <= TCT_H) {
+        return p[o.x];
+    } else {
+        const double a = p[o.x & 255], b = p[o.x >> 8 & 255], c = p[o.x >> 16 & 255],
+                     d = p[o.x >> 24], e = p[o.y & 255];
+        if constexpr (KID == TCT_RH)
+            return fma(e, p[o.y >> 8 & 255], fma(c, d, a * b));
+        else
+            return fma(a, b, e) - c * d;
+    }
+}
+
+// What the outputs of one pair are made of, from its sums `acc` (rotated
+// frame: bases in the integrator's order) into p (bases in the caller's order:
+// the de-rotation of assemble.cl:77-101, out[b1] = res[od[b1]] with od[i] =
+// (i - clicks) mod 3, entries 0 and 1 of the source map swapped when the
+// source was flipped).
+template <int KID>
+__device__ __forceinline__ void pack_pair(const double *acc, const Tri &ot, const Tri &st,
+                                          const ElasticConsts &c, int oc, int sc, int flip,
+                                          double *p) {
+    int oi[3], si[3];   // caller's position of each basis
+    {
+        int sd[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) sd[i] = pmod3(i - sc);
+        if (flip) {
+            const int tmp = sd[0];
+            sd[0] = sd[1];
+            sd[1] = tmp;
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            oi[i] = pmod3(i + oc);
+            si[i] = (sd[0] == i) ? 0 : ((sd[1] == i) ? 1 : 2);
+        }
+    }
+    const double J = ot.jac * st.jac;
+    if constexpr (KID == TCT_U) {
+#pragma unroll
+        for (int b = 0; b < 3; ++b)
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+#pragma unroll
+                    for (int f = d; f < 3; ++f)
+                        p[(3 * oi[b] + si[e]) * 6 + sym6(d, f)] =
+                            J * acc[b * 27 + d * 9 + e * 3 + f];
+    } else if constexpr (KID <= TCT_H) {
+#pragma unroll
+        for (int b = 0; b < 3; ++b)
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+#pragma unroll
+                    for (int f = 0; f < 3; ++f)
+                        p[oi[b] * 27 + d * 9 + si[e] * 3 + f] =
+                            J * acc[b * 27 + d * 9 + e * 3 + f];
+    } else if constexpr (KID == TCT_RH) {
+        const double c0 = J * c.CsRH0, s0 = c0 * acc[0];
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+            for (int f = d; f < 3; ++f) {
+                const double s2 = c0 * acc[1 + sym6(d, f)];
+                p[sym6(d, f)] = -2.0 * (d == f ? s2 + s0 : s2);
+            }
+#pragma unroll
+        for (int b = 0; b < 3; ++b) {
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                p[6 + 3 * oi[b] + si[e]] = ot.curl[b][0] * st.curl[e][0] +
+                                           ot.curl[b][1] * st.curl[e][1] +
+                                           ot.curl[b][2] * st.curl[e][2];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                p[15 + 3 * oi[b] + d] = s0 * c.CsRH1 * ot.curl[b][d];
+                p[24 + 3 * oi[b] + d] = s0 * c.CsRH2 * ot.curl[b][d];
+                p[33 + 3 * si[b] + d] = st.curl[b][d];
+            }
+        }
+    } else {
+        const int *ci = KID == TCT_RT ? oi : si;   // side of the weights
+        const int *xi = KID == TCT_RT ? si : oi;   // side of the curls
+        const Tri &x = KID == TCT_RT ? st : ot;
+#pragma unroll
+        for (int b = 0; b < 3; ++b) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+#pragma unroll
+                for (int f = d; f < 3; ++f) {
+                    const double a2 = acc[3 + 6 * b + sym6(d, f)];
+                    p[6 * ci[b] + sym6(d, f)] = J * (d == f ? a2 + acc[b] : a2);
+                }
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                p[18 + 3 * oi[b] + si[e]] = (KID == TCT_RT ? J : -J) * acc[21 + 3 * b + e];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) p[27 + 3 * xi[b] + d] = x.curl[b][d];
+        }
+        p[36] = 0.0;
+    }
+}
+
+// LDS of one wave.
+template <int KID, int GL>
+struct PairStage {
+    double v[pack_pairs<KID, GL>() * pack_size<KID>()];
+    int row[pack_pairs<KID, GL>()];   // output row (-1: none)
+};
+
+// The outputs of the 64 / GL pairs of one wave.  Every lane of the wave
+// calls it; the GL lanes of pair pl, of which `writer` has the sums.
+// pack(p) puts the pair's sums in LDS (pack_pair).  SUB: subtracted from what
+// is there instead of written.
+template <int KID, int GL, bool SUB, typename F>
+__device__ __forceinline__ void write_pairs(F &&pack, const PairTable &tab,
+                                            PairStage<KID, GL> &sg, int pl, bool writer, int row,
+                                            double *__restrict__ out) {
+    constexpr int PW = 64 / GL, SP = pack_pairs<KID, GL>(), ND = pack_size<KID>();
+    constexpr int NE = SP * 81;
+    const int lane = (int)threadIdx.x & 63;
+#pragma unroll 1
+    for (int h = 0; h < PW / SP; ++h) {
+        // a wave's LDS operations complete in order: no barrier needed
+        // between its writes and reads but the compiler's
+        __builtin_amdgcn_wave_barrier();
+        if (writer && pl / SP == h) {
+            pack(&sg.v[(pl % SP) * ND]);
+            sg.row[pl % SP] = row;
+        }
+        __builtin_amdgcn_wave_barrier();
+        int p = 0, i = lane;   // entry i of pair p: element p * 81 + i
+#pragma unroll 2
+        for (int e = lane; e < NE; e += 64) {
+            const int r = sg.row[p];
+            const double x = pair_entry<KID>(&sg.v[p * ND], tab.off[i]);
+            if (r >= 0) {
+                double *o = out + (size_t)r * 81 + i;
+                *o = SUB ? *o - x : x;
+            }
+            i += 64;
+            if (i >= 81) {
+                i -= 81;
+                ++p;
+            }
+        }
+    }
+}
 
 }  // namespace tct

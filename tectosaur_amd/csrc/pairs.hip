@@ -46,17 +46,6 @@ __device__ __forceinline__ void pair_geom(const Tri &ot, const Tri &st, PairGeom
     }
 }
 
-// The r = 0 test of a pair class (CK): CK_NONE for pairs that never touch;
-// CK_FULL skips r2 == 0 and the points whose obs and src parameters are
-// equal on pairs that are one triangle in one frame; CK_R2 skips r2 == 0
-// only, for rules with no point of equal obs and src parameters.
-constexpr int CK_NONE = 0, CK_FULL = 1, CK_R2 = 2;
-
-// Normals a kernel body reads: obs (m) and src (n).
-struct PairNormals {
-    double m[3], n[3];
-};
-
 // One rule point of one pair.  The r = 0 test skips the points at r = 0
 // (the "Z" kernels, assemble.cl:24-47, and the adjacent kernels, :49-103,
 // which test r2 == 0 on the basis-weighted positions).  The edge form
@@ -145,46 +134,6 @@ __device__ __forceinline__ void accumulate_point(const PairNormals &nm, const Pa
 }
 
 
-// Output value (rotated-frame indices bo, dob, bs, ds) from the reduced
-// accumulators, before the J_obs J_src factor.
-template <int KID>
-__device__ __forceinline__ double final_value(const double *acc, const Tri &ot, const Tri &st,
-                                              const ElasticConsts &c, int bo, int dob, int bs,
-                                              int ds) {
-    if constexpr (KID <= TCT_H) {
-        return acc[bo * 27 + dob * 9 + bs * 3 + ds];
-    } else if constexpr (KID == TCT_RH) {
-        const double *co = ot.curl[bo];
-        const double *cs = st.curl[bs];
-        const double cc = co[0] * cs[0] + co[1] * cs[1] + co[2] * cs[2];
-        const double S0 = acc[0];
-        const double S2 = acc[1 + sym6(dob, ds)];
-        return c.CsRH0 * (-2.0 * S2 * cc +
-                          S0 * (c.CsRH1 * co[dob] * cs[ds] + c.CsRH2 * co[ds] * cs[dob] -
-                                (dob == ds ? 2.0 * cc : 0.0)));
-    } else if constexpr (KID == TCT_RT) {
-        // sum_Ij curl_s[bs][Ij] (e[Ij][do][ds] A1[bo] + sum_t e[Ij][t][ds] A2[bo][do,t])
-        //   + delta(do, ds) A3[bo][bs]
-        double v = (dob == ds) ? acc[21 + 3 * bo + bs] : 0.0;
-        for (int Ij = 0; Ij < 3; ++Ij) {
-            double g = levi(Ij, dob, ds) * acc[bo];
-            for (int t = 0; t < 3; ++t) g += levi(Ij, t, ds) * acc[3 + 6 * bo + sym6(dob, t)];
-            v += st.curl[bs][Ij] * g;
-        }
-        return v;
-    } else {
-        // RA: sum_Ij curl_o[bo][Ij] (e[Ij][ds][do] B1[bs] + sum_t e[Ij][t][do] B2[bs][ds,t])
-        //   - delta(do, ds) B3[bo][bs]
-        double v = (dob == ds) ? -acc[21 + 3 * bo + bs] : 0.0;
-        for (int Ij = 0; Ij < 3; ++Ij) {
-            double g = levi(Ij, ds, dob) * acc[bs];
-            for (int t = 0; t < 3; ++t) g += levi(Ij, t, dob) * acc[3 + 6 * bs + sym6(ds, t)];
-            v += ot.curl[bo][Ij] * g;
-        }
-        return v;
-    }
-}
-
 // Rule point iq: (obs xi, obs eta, src xi, src eta, weight).
 __device__ __forceinline__ void load_point(double (&q)[5], const double *__restrict__ qx,
                                            const double *__restrict__ qw, int iq) {
@@ -205,51 +154,6 @@ __device__ __forceinline__ void load_point_at(double (&q)[5], const double *pq, 
 // point's arithmetic, which starts from b, after it.
 __device__ __forceinline__ void fence_point(double last, double (&b)[3], double &dep) {
     asm volatile("" : "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(dep) : "s"(last) : "memory");
-}
-
-// The 81 outputs of one pair from its reduced accumulators: the triangle
-// records are formed again, from indices the compiler cannot match with the
-// first loads (it would otherwise keep those records live through the rule
-// loop), and the de-rotation of assemble.cl:77-101 is applied: out[b1] =
-// res[od[b1]] with od[i] = (i - clicks) mod 3, entries 0 and 1 of the source
-// map swapped when the source was flipped -- written as the inverse map on
-// the output address, so every register index stays static.
-template <int KID>
-__device__ __forceinline__ void write_pair_output(const double *acc,
-                                                  const double *__restrict__ pts,
-                                                  const int32_t *__restrict__ tris,
-                                                  const int32_t *pp, int oc, int sc, int flip,
-                                                  const ElasticConsts &c, double *o) {
-    int oi = pp[0], si = pp[1];
-    asm volatile("" : "+v"(oi), "+v"(si));
-    Tri ot, st;
-    load_tri(ot, pts, tris, oi, oc, 0);
-    load_tri(st, pts, tris, si, sc, flip);
-    int sd[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) sd[i] = pmod3(i - sc);
-    if (flip) {
-        const int tmp = sd[0];
-        sd[0] = sd[1];
-        sd[1] = tmp;
-    }
-    int oinv[3], sinv[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        oinv[i] = pmod3(i + oc);
-        sinv[i] = (sd[0] == i) ? 0 : ((sd[1] == i) ? 1 : 2);
-    }
-    const double J = ot.jac * st.jac;
-#pragma unroll
-    for (int i1 = 0; i1 < 3; ++i1)
-#pragma unroll
-        for (int d1 = 0; d1 < 3; ++d1)
-#pragma unroll
-            for (int i2 = 0; i2 < 3; ++i2)
-#pragma unroll
-                for (int d2 = 0; d2 < 3; ++d2)
-                    o[oinv[i1] * 27 + d1 * 9 + sinv[i2] * 3 + d2] =
-                        J * final_value<KID>(acc, ot, st, c, i1, d1, i2, d2);
 }
 
 // One lane walks rule points [q0, q1) of its pair; every lane of the wave
@@ -291,6 +195,10 @@ __global__ __launch_bounds__(256) void pairs_kernel(int nq, const double *__rest
                                                     int pair_width, ElasticConsts c,
                                                     double *__restrict__ out) {
     constexpr int NA = n_acc<KID>();
+    __shared__ PairTable table;
+    __shared__ PairStage<KID, GL> stage[4];
+    fill_pair_table<KID>(table);
+    __syncthreads();
     const int gid = blockIdx.x * blockDim.x + threadIdx.x;
     const int pair = gid / GL;
     const int sub = gid % GL;
@@ -304,9 +212,9 @@ __global__ __launch_bounds__(256) void pairs_kernel(int nq, const double *__rest
         sc = pp[3];
         flip = pp[4] != 0;
     }
-    // The rule loop needs only the pair geometry and the normals; the whole
-    // triangle records (curls, Jacobians) are formed again after it, so
-    // they hold no registers during the loop.
+    // The rule loop needs only the pair geometry and the normals; the
+    // curls and Jacobians are formed again after it, so they hold no
+    // registers during the loop.
     PairGeom g;
     PairNormals nm;
     {
@@ -365,8 +273,21 @@ __global__ __launch_bounds__(256) void pairs_kernel(int nq, const double *__rest
             acc[k] = v;
         }
     }
-    if (!live || sub != 0) return;
-    write_pair_output<KID>(acc, pts, tris, pp, oc, sc, flip, c, out + (size_t)pair * 81);
+    // the curls and Jacobians again, from the edges the loop has kept
+    Tri ot, st;
+    {
+        double oe[2][3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            oe[0][d] = -g.oe[0][d];
+            oe[1][d] = -g.oe[1][d];
+        }
+        tri_from_edges(ot, oe[0], oe[1]);
+        tri_from_edges(st, g.se[0], g.se[1]);
+    }
+    write_pairs<KID, GL, false>(
+        [&](double *p) { pack_pair<KID>(acc, ot, st, c, oc, sc, flip, p); }, table,
+        stage[threadIdx.x / 64], (int)(threadIdx.x % 64) / GL, sub == 0, live ? pair : -1, out);
 }
 
 // RH3 pairs, one lane per (pair, rule chunk): grid (pair blocks, C slots).
@@ -451,25 +372,36 @@ __global__ __launch_bounds__(256) void pairs_rh_finish_kernel(
     const int32_t *__restrict__ pairs, int pair_width, int nch, ElasticConsts c,
     double *__restrict__ out) {
     constexpr int NA = n_acc<TCT_RH>();
+    __shared__ PairTable table;
+    __shared__ PairStage<TCT_RH, 1> stage[4];
+    fill_pair_table<TCT_RH>(table);
+    __syncthreads();
     const int pair = blockIdx.x * blockDim.x + threadIdx.x;
-    if (pair >= n_pairs) return;
-    const int32_t *pp = pairs + (size_t)pair * pair_width;
+    const bool live = pair < n_pairs;
+    const int pr = live ? pair : n_pairs - 1;
+    const int32_t *pp = pairs + (size_t)pr * pair_width;
     int oc = 0, sc = 0, flip = 0;
     if (pair_width == 5) {
         oc = pp[2];
         sc = pp[3];
         flip = pp[4] != 0;
     }
-    double *o = out + (size_t)pair * 81;
-    // every chunk's accumulators are read (in chunk order) before the row
-    // is overwritten with the outputs
+    const double *o = out + (size_t)pr * 81;
+    // a wave's rows are all read (each in chunk order) before the first of
+    // them is overwritten: the outputs pass through the wave's LDS
     double acc[NA];
 #pragma unroll
     for (int k = 0; k < NA; ++k) acc[k] = 0.0;
-    for (int ch = 0; ch < nch; ++ch)
+    if (live)
+        for (int ch = 0; ch < nch; ++ch)
 #pragma unroll
-        for (int k = 0; k < NA; ++k) acc[k] += o[NA * ch + k];
-    write_pair_output<TCT_RH>(acc, pts, tris, pp, oc, sc, flip, c, o);
+            for (int k = 0; k < NA; ++k) acc[k] += o[NA * ch + k];
+    Tri ot, st;
+    load_tri(ot, pts, tris, pp[0], oc, 0);
+    load_tri(st, pts, tris, pp[1], sc, flip);
+    write_pairs<TCT_RH, 1, false>(
+        [&](double *p) { pack_pair<TCT_RH>(acc, ot, st, c, oc, sc, flip, p); }, table,
+        stage[threadIdx.x / 64], (int)(threadIdx.x % 64), true, live ? pair : -1, out);
 }
 
 __global__ void sub_f64_kernel(int64_t n, const double *__restrict__ a,

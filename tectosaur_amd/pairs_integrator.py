@@ -17,7 +17,7 @@ import torch
 
 from . import _native as N
 from . import triangle_rules
-from .quadrature import gauss4d_tri
+from .quadrature import gauss2d_tri, gauss4d_tri
 
 # pairs per launch: bounds the output buffer of one call (81 doubles/pair)
 CALL_SIZE = 1 << 20
@@ -32,11 +32,14 @@ class DeviceRule(tuple):
     ``has_equal_params`` says whether some point has equal observation and
     source parameters: on a pair that is one triangle in one frame those
     points are at r = 0, and the kernel's r = 0 test must look for them; a
-    rule without such points needs only the r2 == 0 test."""
+    rule without such points needs only the r2 == 0 test.  ``side``: the
+    triangle rule (q [n, 2], w [n], on the device) whose product with itself
+    the rule is, or None."""
 
-    def __new__(cls, qx, qw, has_equal_params):
+    def __new__(cls, qx, qw, has_equal_params, side=None):
         t = super().__new__(cls, (qx, qw))
         t.has_equal_params = bool(has_equal_params)
+        t.side = side
         return t
 
 
@@ -45,6 +48,16 @@ def rule_has_equal_params(qx):
     src xhat, src yhat) has equal observation and source parameters."""
     qx = np.asarray(qx, dtype=np.float64)
     return bool(qx.size) and bool(np.any((qx[:, 0] == qx[:, 2]) & (qx[:, 1] == qx[:, 3])))
+
+
+def product_pays(kernel, n):
+    """Whether a rule that is a product of an n-point triangle rule with
+    itself runs as one: always for the surface-curl kernels, whose sums are
+    few (3 x 3 points, RH3 135 -> 106 us for 710,704 pairs); for U, T, A and H,
+    with 81 sums a pair and a wave less per SIMD, from 19 points (U3, 710,704
+    pairs: 4 x 4 points 142 -> 167 us, 19 x 19 873 -> 626; 13 x 13, 29,128
+    pairs: 56 -> 90; T3, 19 x 19: 1212 -> 1106)."""
+    return kernel in ('elasticRT3', 'elasticRA3', 'elasticRH3') or n >= 19
 
 
 def r0_test_mode(q, check0):
@@ -69,15 +82,19 @@ class PairsIntegrator:
         self.gpu_pts = N.upload(np.asarray(pts, dtype=np.float64), None, self.device)
         self.gpu_tris = N.upload(np.asarray(tris, dtype=np.int32), None, self.device)
         self._rules = {}
-        self.near_q = self._rule(('near4d', nq_near), lambda: gauss4d_tri(nq_near, nq_near))
-        self.far_q = self._rule(('far4d', nq_far), lambda: gauss4d_tri(nq_far, nq_far))
+        self.near_q = self._product_rule('near4d', nq_near)
+        self.far_q = self._product_rule('far4d', nq_far)
 
-    def quad_to_gpu(self, q):
+    def quad_to_gpu(self, q, side=None):
+        up = lambda a: N.upload(a, torch.float64, self.device)
         qx = np.asarray(q[0], dtype=np.float64)
-        return DeviceRule(N.upload(qx, torch.float64, self.device),
-                          N.upload(q[1], torch.float64, self.device), rule_has_equal_params(qx))
+        return DeviceRule(up(qx), up(q[1]), rule_has_equal_params(qx),
+                          None if side is None else (up(side[0]), up(side[1])))
 
-    def _rule(self, key, make):
+    def _product_rule(self, name, nq):
+        return self._rule((name, nq), lambda: gauss4d_tri(nq, nq), lambda: gauss2d_tri(nq))
+
+    def _rule(self, key, make, side=None):
         if key not in self._rules:
             # rules are pure functions of their orders and read-only on the
             # device: one copy per device shared by every integrator
@@ -87,7 +104,7 @@ class PairsIntegrator:
                 with _RULES_LOCK:
                     q = _RULES.get(dkey)
                     if q is None:
-                        q = _RULES[dkey] = self.quad_to_gpu(make())
+                        q = _RULES[dkey] = self.quad_to_gpu(make(), side and side())
             self._rules[key] = q
         return self._rules[key]
 
@@ -98,8 +115,20 @@ class PairsIntegrator:
         if out is None:
             out = torch.empty((n, 81), dtype=torch.float64, device=self.device)
         st = N.stream_ptr()
+        # a rule that is a product runs as one, unless the caller chooses how
+        # many lanes share a pair's 4-D rule
+        side = getattr(q, 'side', None) if lanes_per_pair == 0 else None
+        if side is not None and not product_pays(self.kernel, side[1].shape[0]):
+            side = None
         for s in range(0, n, CALL_SIZE):
             e = min(n, s + CALL_SIZE)
+            if side is not None:
+                sq, sw = side
+                N.call('tct_pairs_product', self.kid, sw.shape[0], N.ptr(sq), N.ptr(sw),
+                       sw.shape[0], N.ptr(sq), N.ptr(sw), N.ptr(self.gpu_pts),
+                       N.ptr(self.gpu_tris), e - s, N.ptr(pairs_dev[s:e]), width,
+                       r0_test_mode(q, check0), self.params.ctypes.data, N.ptr(out[s:e]), st)
+                continue
             N.call('tct_pairs_integrate', self.kid, q[0].shape[0], N.ptr(q[0]), N.ptr(q[1]),
                    N.ptr(self.gpu_pts), N.ptr(self.gpu_tris), e - s, N.ptr(pairs_dev[s:e]),
                    width, r0_test_mode(q, check0), self.params.ctypes.data, lanes_per_pair,
