@@ -353,16 +353,50 @@ int tct_pairs_integrate(int kernel, int64_t nq, const double *qx, const double *
                         const double *params_host, int lanes_per_pair, double *out,
                         void *stream);
 
-/* tct_pairs_integrate for a product rule: every point of the obs rule
- * (qo [n_o][2], weights wo) with every one of the src rule (qs [n_s][2], ws),
- * the points of gauss4d_tri (tectosaur/util/quadrature.py:47-60) in another
- * order of summation.  check0 as there (1 and 2 both skip r2 == 0 and the
- * points with equal parameters). */
+/* tct_pairs_integrate with pair i's outputs in row rows[i] of out (rows NULL:
+ * row i). */
+int tct_pairs_integrate_rows(int kernel, int64_t nq, const double *qx, const double *qw,
+                             const double *pts, const int32_t *tris, int64_t n_pairs,
+                             const int32_t *pairs, int pair_width, int check0,
+                             const double *params_host, int lanes_per_pair,
+                             const int32_t *rows, double *out, void *stream);
+
+/* The same for a product rule: every point of the obs rule (qo [n_o][2],
+ * weights wo) with every one of the src rule (qs [n_s][2], ws), the points of
+ * gauss4d_tri (tectosaur/util/quadrature.py:47-60) in another order of
+ * summation.  n_minus > 0: less the same pairs under the product of the rule
+ * (q_minus, w_minus) with itself, in one pass.  check0 as there (1 and 2 both
+ * skip r2 == 0 and the points with equal parameters).  subtract: out[row] -=
+ * the integrals instead of out[row] = them. */
 int tct_pairs_product(int kernel, int n_o, const double *qo, const double *wo, int n_s,
-                      const double *qs, const double *ws, const double *pts,
-                      const int32_t *tris, int64_t n_pairs, const int32_t *pairs,
-                      int pair_width, int check0, const double *params_host, double *out,
-                      void *stream);
+                      const double *qs, const double *ws, int n_minus, const double *q_minus,
+                      const double *w_minus, const double *pts, const int32_t *tris,
+                      int64_t n_pairs, const int32_t *pairs, int pair_width, int check0,
+                      const double *params_host, const int32_t *rows, int subtract,
+                      double *out, void *stream);
+
+/* Host: a pair list (int64, width 2 or 5, rows contiguous) into int32 with the
+ * ranges checked: triangles in [0, n_tris), clicks in [0, 3), flip 0 or 1;
+ * with dofs (int64 [n][2], rows dofs_stride values apart) those into dofs32,
+ * in [0, n_rows) and [0, n_cols).  Returns TCT_EARG when a value is out of
+ * range; *sorted tells whether the dofs (the pairs without dofs) come in
+ * ascending order of (row, column), equal ones allowed. */
+int tct_pairs_pack(int64_t n, int width, const int64_t *pairs, int64_t n_tris,
+                   const int64_t *dofs, int64_t dofs_stride, int64_t n_rows, int64_t n_cols,
+                   int32_t *pairs32, int32_t *dofs32, int *sorted);
+/* Host: whether the dofs (int64 [n][2], rows dofs_stride apart) are the first
+ * two columns of the pairs. */
+int tct_pairs_same(int64_t n, int width, const int64_t *pairs, const int64_t *dofs,
+                   int64_t dofs_stride, int *same);
+
+/* The block rows of n_lists (at most 4) lists of blocks, each sorted by (row,
+ * column), merged: list k has n[k] blocks at dofs[k] (dev, (row, column) at a
+ * stride of strides[k] int32).  rank[k][i]: position of its block i in the
+ * merged order (earlier lists first where equal); indices: the merged
+ * columns; indptr [n_rows + 1]: the row starts. */
+int tct_bsr_merge(int n_lists, const int64_t *n, const int32_t *const *dofs, const int *strides,
+                  int64_t n_rows, int32_t *const *rank, int32_t *indices, int32_t *indptr,
+                  void *stream);
 
 /* out[i] = a[i] - b[i] over n doubles (nearfield correction, tectosaur/
  * nearfield/nearfield_op.py:135-141). */

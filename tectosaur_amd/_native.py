@@ -95,8 +95,13 @@ SIGNATURES = {
     'tct_far_scatter_tris': [_i64, _int, _vp, _vp, _vp, _i64, _int, _vp, _vp, _vp],
     'tct_pairs_integrate': [_int, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _int, _int, _vp, _int,
                             _vp, _vp],
-    'tct_pairs_product': [_int, _int, _vp, _vp, _int, _vp, _vp, _vp, _vp, _i64, _vp, _int, _int,
-                          _vp, _vp, _vp],
+    'tct_pairs_integrate_rows': [_int, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _int, _int, _vp, _int,
+                                 _vp, _vp, _vp],
+    'tct_pairs_product': [_int, _int, _vp, _vp, _int, _vp, _vp, _int, _vp, _vp, _vp, _vp, _i64,
+                          _vp, _int, _int, _vp, _vp, _int, _vp, _vp],
+    'tct_pairs_pack': [_i64, _int, _vp, _i64, _vp, _i64, _i64, _i64, _vp, _vp, _vp],
+    'tct_pairs_same': [_i64, _int, _vp, _vp, _i64, _vp],
+    'tct_bsr_merge': [_int, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp],
     'tct_sub_f64': [_i64, _vp, _vp, _vp, _vp],
     'tct_bsr9_spmv': [_i64, _vp, _vp, _vp, _vp, _vp, _int, _vp],
     'tct_interior_pairs': [_int, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _int, _int, _vp,

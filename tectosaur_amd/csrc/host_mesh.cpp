@@ -215,3 +215,55 @@ extern "C" int tct_split_adjacent_close(int64_t n_pairs, const int64_t *pairs,
     counts[2] = ne;
     return TCT_OK;
 }
+
+// One pass over a pair list: int64 -> int32, range checks and whether it is
+// sorted.  The separate numpy passes (two reductions, a conversion and two
+// strided column copies) took 2.9 ms of a 4.4 ms set-up of 700,000 pairs.
+extern "C" int tct_pairs_pack(int64_t n, int width, const int64_t *pairs, int64_t n_tris,
+                              const int64_t *dofs, int64_t dofs_stride, int64_t n_rows,
+                              int64_t n_cols, int32_t *pairs32, int32_t *dofs32, int *sorted) {
+    if (n < 0 || (width != 2 && width != 5) || !sorted || n_tris >= (1LL << 31) ||
+        n_rows >= (1LL << 31) || n_cols >= (1LL << 31) ||
+        (n > 0 && (!pairs || !pairs32 || (dofs && !dofs32))))
+        return tct::set_error(TCT_EARG, "pairs_pack: bad arguments");
+    int bad = 0, unsorted = 0;
+#pragma omp parallel for schedule(static) reduction(| : bad, unsorted) if (n > 32768)
+    for (int64_t i = 0; i < n; ++i) {
+        const int64_t *p = pairs + i * width;
+        int32_t *o = pairs32 + i * width;
+        bad |= p[0] < 0 || p[0] >= n_tris || p[1] < 0 || p[1] >= n_tris;
+        if (width == 5) {
+            bad |= p[2] < 0 || p[2] > 2 || p[3] < 0 || p[3] > 2 || p[4] < 0 || p[4] > 1;
+            for (int k = 2; k < 5; ++k) o[k] = (int32_t)p[k];
+        }
+        o[0] = (int32_t)p[0];
+        o[1] = (int32_t)p[1];
+        const int64_t *d = dofs ? dofs + i * dofs_stride : p;
+        if (dofs) {
+            bad |= d[0] < 0 || d[0] >= n_rows || d[1] < 0 || d[1] >= n_cols;
+            dofs32[2 * i] = (int32_t)d[0];
+            dofs32[2 * i + 1] = (int32_t)d[1];
+        }
+        if (i > 0) {
+            const int64_t *e = dofs ? d - dofs_stride : p - width;
+            unsorted |= e[0] > d[0] || (e[0] == d[0] && e[1] > d[1]);
+        }
+    }
+    *sorted = !unsorted;
+    if (bad) return tct::set_error(TCT_EARG, "pairs_pack: value out of range");
+    return TCT_OK;
+}
+
+extern "C" int tct_pairs_same(int64_t n, int width, const int64_t *pairs, const int64_t *dofs,
+                              int64_t dofs_stride, int *same) {
+    if (n < 0 || (width != 2 && width != 5) || !same || (n > 0 && (!pairs || !dofs)))
+        return tct::set_error(TCT_EARG, "pairs_same: bad arguments");
+    int differ = 0;
+#pragma omp parallel for schedule(static) reduction(| : differ) if (n > 32768)
+    for (int64_t i = 0; i < n; ++i) {
+        const int64_t *p = pairs + i * width, *d = dofs + i * dofs_stride;
+        differ |= p[0] != d[0] || p[1] != d[1];
+    }
+    *same = !differ;
+    return TCT_OK;
+}

@@ -356,6 +356,11 @@ __device__ __forceinline__ void pack_pair(const double *acc, const Tri &ot, cons
     }
 }
 
+// The output row of a pair: rows[pair], or the pair itself.
+__device__ __forceinline__ int out_row(const int32_t *__restrict__ rows, int pair) {
+    return rows ? rows[pair] : pair;
+}
+
 // LDS of one wave.
 template <int KID, int GL>
 struct PairStage {

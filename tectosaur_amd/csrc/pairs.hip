@@ -193,6 +193,7 @@ __global__ __launch_bounds__(256) void pairs_kernel(int nq, const double *__rest
                                                     const int32_t *__restrict__ tris, int n_pairs,
                                                     const int32_t *__restrict__ pairs,
                                                     int pair_width, ElasticConsts c,
+                                                    const int32_t *__restrict__ rows,
                                                     double *__restrict__ out) {
     constexpr int NA = n_acc<KID>();
     __shared__ PairTable table;
@@ -287,7 +288,8 @@ __global__ __launch_bounds__(256) void pairs_kernel(int nq, const double *__rest
     }
     write_pairs<KID, GL, false>(
         [&](double *p) { pack_pair<KID>(acc, ot, st, c, oc, sc, flip, p); }, table,
-        stage[threadIdx.x / 64], (int)(threadIdx.x % 64) / GL, sub == 0, live ? pair : -1, out);
+        stage[threadIdx.x / 64], (int)(threadIdx.x % 64) / GL, sub == 0,
+        live ? out_row(rows, pair) : -1, out);
 }
 
 // RH3 pairs, one lane per (pair, rule chunk): grid (pair blocks, C slots).
@@ -311,7 +313,8 @@ template <int CK, int S>
 __global__ __launch_bounds__(rh_chunk_block(S)) void pairs_rh_chunk_kernel(
     int nq, const double *__restrict__ qx, const double *__restrict__ qw,
     const double *__restrict__ pts, const int32_t *__restrict__ tris, int n_pairs,
-    const int32_t *__restrict__ pairs, int pair_width, ElasticConsts c, double *__restrict__ out) {
+    const int32_t *__restrict__ pairs, int pair_width, ElasticConsts c,
+    const int32_t *__restrict__ rows, double *__restrict__ out) {
     constexpr int NA = n_acc<TCT_RH>();
     constexpr int PB = rh_chunk_block(S) / S;   // pairs per workgroup, a multiple of 64
     static_assert(PB % 64 == 0, "a wave must not straddle two chunks");
@@ -362,7 +365,7 @@ __global__ __launch_bounds__(rh_chunk_block(S)) void pairs_rh_chunk_kernel(
             for (int k = 0; k < NA; ++k) acc[k] += part[s][k][lane];
     }
     if (!live) return;
-    double *o = out + (size_t)pair * 81 + NA * ch;
+    double *o = out + (size_t)out_row(rows, pair) * 81 + NA * ch;
 #pragma unroll
     for (int k = 0; k < NA; ++k) o[k] = acc[k];
 }
@@ -370,7 +373,7 @@ __global__ __launch_bounds__(rh_chunk_block(S)) void pairs_rh_chunk_kernel(
 __global__ __launch_bounds__(256) void pairs_rh_finish_kernel(
     int n_pairs, const double *__restrict__ pts, const int32_t *__restrict__ tris,
     const int32_t *__restrict__ pairs, int pair_width, int nch, ElasticConsts c,
-    double *__restrict__ out) {
+    const int32_t *__restrict__ rows, double *__restrict__ out) {
     constexpr int NA = n_acc<TCT_RH>();
     __shared__ PairTable table;
     __shared__ PairStage<TCT_RH, 1> stage[4];
@@ -386,7 +389,8 @@ __global__ __launch_bounds__(256) void pairs_rh_finish_kernel(
         sc = pp[3];
         flip = pp[4] != 0;
     }
-    const double *o = out + (size_t)pr * 81;
+    const int row = out_row(rows, pr);
+    const double *o = out + (size_t)row * 81;
     // a wave's rows are all read (each in chunk order) before the first of
     // them is overwritten: the outputs pass through the wave's LDS
     double acc[NA];
@@ -401,7 +405,7 @@ __global__ __launch_bounds__(256) void pairs_rh_finish_kernel(
     load_tri(st, pts, tris, pp[1], sc, flip);
     write_pairs<TCT_RH, 1, false>(
         [&](double *p) { pack_pair<TCT_RH>(acc, ot, st, c, oc, sc, flip, p); }, table,
-        stage[threadIdx.x / 64], (int)(threadIdx.x % 64), true, live ? pair : -1, out);
+        stage[threadIdx.x / 64], (int)(threadIdx.x % 64), true, live ? row : -1, out);
 }
 
 __global__ void sub_f64_kernel(int64_t n, const double *__restrict__ a,
@@ -414,30 +418,30 @@ template <int KID, int GL>
 static void launch_pairs(hipStream_t st, int nq, const double *qx, const double *qw,
                          const double *pts, const int32_t *tris, int n_pairs,
                          const int32_t *pairs, int pair_width, int check0,
-                         const ElasticConsts &c, double *out) {
+                         const ElasticConsts &c, const int32_t *rows, double *out) {
     const int64_t threads = (int64_t)n_pairs * GL;
     const unsigned nb = (unsigned)ceil_div(threads, 256);
     if (check0 == CK_FULL)
         hipLaunchKernelGGL((pairs_kernel<KID, GL, CK_FULL>), dim3(nb), dim3(256), 0, st, nq, qx,
-                           qw, pts, tris, n_pairs, pairs, pair_width, c, out);
+                           qw, pts, tris, n_pairs, pairs, pair_width, c, rows, out);
     else if (check0 == CK_R2)
         hipLaunchKernelGGL((pairs_kernel<KID, GL, CK_R2>), dim3(nb), dim3(256), 0, st, nq, qx,
-                           qw, pts, tris, n_pairs, pairs, pair_width, c, out);
+                           qw, pts, tris, n_pairs, pairs, pair_width, c, rows, out);
     else
         hipLaunchKernelGGL((pairs_kernel<KID, GL, CK_NONE>), dim3(nb), dim3(256), 0, st, nq, qx,
-                           qw, pts, tris, n_pairs, pairs, pair_width, c, out);
+                           qw, pts, tris, n_pairs, pairs, pair_width, c, rows, out);
 }
 
 template <int KID>
 static void launch_pairs_g(int gl, hipStream_t st, int nq, const double *qx, const double *qw,
                            const double *pts, const int32_t *tris, int n_pairs,
                            const int32_t *pairs, int pair_width, int check0,
-                           const ElasticConsts &c, double *out) {
+                           const ElasticConsts &c, const int32_t *rows, double *out) {
     switch (gl) {
-    case 1: launch_pairs<KID, 1>(st, nq, qx, qw, pts, tris, n_pairs, pairs, pair_width, check0, c, out); break;
-    case 4: launch_pairs<KID, 4>(st, nq, qx, qw, pts, tris, n_pairs, pairs, pair_width, check0, c, out); break;
-    case 16: launch_pairs<KID, 16>(st, nq, qx, qw, pts, tris, n_pairs, pairs, pair_width, check0, c, out); break;
-    default: launch_pairs<KID, 64>(st, nq, qx, qw, pts, tris, n_pairs, pairs, pair_width, check0, c, out); break;
+    case 1: launch_pairs<KID, 1>(st, nq, qx, qw, pts, tris, n_pairs, pairs, pair_width, check0, c, rows, out); break;
+    case 4: launch_pairs<KID, 4>(st, nq, qx, qw, pts, tris, n_pairs, pairs, pair_width, check0, c, rows, out); break;
+    case 16: launch_pairs<KID, 16>(st, nq, qx, qw, pts, tris, n_pairs, pairs, pair_width, check0, c, rows, out); break;
+    default: launch_pairs<KID, 64>(st, nq, qx, qw, pts, tris, n_pairs, pairs, pair_width, check0, c, rows, out); break;
     }
 }
 
@@ -450,6 +454,16 @@ extern "C" int tct_pairs_integrate(int kernel, int64_t nq, const double *qx, con
                                    const int32_t *pairs, int pair_width, int check0,
                                    const double *params_host, int lanes_per_pair, double *out,
                                    void *stream) {
+    return tct_pairs_integrate_rows(kernel, nq, qx, qw, pts, tris, n_pairs, pairs, pair_width,
+                                    check0, params_host, lanes_per_pair, nullptr, out, stream);
+}
+
+extern "C" int tct_pairs_integrate_rows(int kernel, int64_t nq, const double *qx,
+                                        const double *qw, const double *pts,
+                                        const int32_t *tris, int64_t n_pairs,
+                                        const int32_t *pairs, int pair_width, int check0,
+                                        const double *params_host, int lanes_per_pair,
+                                        const int32_t *rows, double *out, void *stream) {
     TCT_CHECK_ARG(kernel >= TCT_U && kernel <= TCT_RH, "pairs: kernel id %d", kernel);
     TCT_CHECK_ARG(nq > 0 && nq < (1LL << 31), "pairs: nq %lld", (long long)nq);
     TCT_CHECK_ARG(n_pairs >= 0 && n_pairs < (1LL << 26), "pairs: n_pairs %lld (max 2^26 per call)",
@@ -530,14 +544,14 @@ extern "C" int tct_pairs_integrate(int kernel, int64_t nq, const double *qx, con
     if (S == RH_WAVE_SPLIT_MAX)                                                                \
         hipLaunchKernelGGL((pairs_rh_chunk_kernel<CK, RH_WAVE_SPLIT_MAX>), grid,               \
                            dim3(rh_chunk_block(RH_WAVE_SPLIT_MAX)), 0, st, q, qx, qw, pts,     \
-                           tris, np, pairs, pair_width, c, out);                               \
+                           tris, np, pairs, pair_width, c, rows, out);                         \
     else if (S == RH_WAVE_SPLIT)                                                               \
         hipLaunchKernelGGL((pairs_rh_chunk_kernel<CK, RH_WAVE_SPLIT>), grid,                   \
                            dim3(rh_chunk_block(RH_WAVE_SPLIT)), 0, st, q, qx, qw, pts, tris,   \
-                           np, pairs, pair_width, c, out);                                     \
+                           np, pairs, pair_width, c, rows, out);                               \
     else                                                                                       \
         hipLaunchKernelGGL((pairs_rh_chunk_kernel<CK, 1>), grid, dim3(rh_chunk_block(1)), 0,   \
-                           st, q, qx, qw, pts, tris, np, pairs, pair_width, c, out)
+                           st, q, qx, qw, pts, tris, np, pairs, pair_width, c, rows, out)
         if (check0 == CK_FULL)
             TCT_RH_CHUNKS(CK_FULL);
         else if (check0 == CK_R2)
@@ -546,18 +560,18 @@ extern "C" int tct_pairs_integrate(int kernel, int64_t nq, const double *qx, con
             TCT_RH_CHUNKS(CK_NONE);
 #undef TCT_RH_CHUNKS
         hipLaunchKernelGGL(pairs_rh_finish_kernel, dim3((unsigned)ceil_div(n_pairs, (int64_t)256)),
-                           dim3(256), 0, st, np, pts, tris, pairs, pair_width, slots, c, out);
+                           dim3(256), 0, st, np, pts, tris, pairs, pair_width, slots, c, rows, out);
         TCT_CHECK_LAUNCH("pairs_integrate");
         return TCT_OK;
     }
     switch (kernel) {
-    case TCT_U: launch_pairs_g<TCT_U>(gl, st, q, qx, qw, pts, tris, np, pairs, pair_width, check0, c, out); break;
-    case TCT_T: launch_pairs_g<TCT_T>(gl, st, q, qx, qw, pts, tris, np, pairs, pair_width, check0, c, out); break;
-    case TCT_A: launch_pairs_g<TCT_A>(gl, st, q, qx, qw, pts, tris, np, pairs, pair_width, check0, c, out); break;
-    case TCT_H: launch_pairs_g<TCT_H>(gl, st, q, qx, qw, pts, tris, np, pairs, pair_width, check0, c, out); break;
-    case TCT_RT: launch_pairs_g<TCT_RT>(gl, st, q, qx, qw, pts, tris, np, pairs, pair_width, check0, c, out); break;
-    case TCT_RA: launch_pairs_g<TCT_RA>(gl, st, q, qx, qw, pts, tris, np, pairs, pair_width, check0, c, out); break;
-    default: launch_pairs_g<TCT_RH>(gl, st, q, qx, qw, pts, tris, np, pairs, pair_width, check0, c, out); break;
+    case TCT_U: launch_pairs_g<TCT_U>(gl, st, q, qx, qw, pts, tris, np, pairs, pair_width, check0, c, rows, out); break;
+    case TCT_T: launch_pairs_g<TCT_T>(gl, st, q, qx, qw, pts, tris, np, pairs, pair_width, check0, c, rows, out); break;
+    case TCT_A: launch_pairs_g<TCT_A>(gl, st, q, qx, qw, pts, tris, np, pairs, pair_width, check0, c, rows, out); break;
+    case TCT_H: launch_pairs_g<TCT_H>(gl, st, q, qx, qw, pts, tris, np, pairs, pair_width, check0, c, rows, out); break;
+    case TCT_RT: launch_pairs_g<TCT_RT>(gl, st, q, qx, qw, pts, tris, np, pairs, pair_width, check0, c, rows, out); break;
+    case TCT_RA: launch_pairs_g<TCT_RA>(gl, st, q, qx, qw, pts, tris, np, pairs, pair_width, check0, c, rows, out); break;
+    default: launch_pairs_g<TCT_RH>(gl, st, q, qx, qw, pts, tris, np, pairs, pair_width, check0, c, rows, out); break;
     }
     TCT_CHECK_LAUNCH("pairs_integrate");
     return TCT_OK;

@@ -160,8 +160,9 @@ __device__ __forceinline__ void fold_point(const double *a, double wf, double fx
 
 template <int KID, int P, int GL, int CK, bool SUB>
 __global__ __launch_bounds__(256) void pairs_product_kernel(
-    SideRule ro, SideRule rs, const double *__restrict__ pts, const int32_t *__restrict__ tris,
-    int n_pairs, const int32_t *__restrict__ pairs, int pair_width, ElasticConsts c,
+    SideRule ro, SideRule rs, SideRule minus, const double *__restrict__ pts,
+    const int32_t *__restrict__ tris, int n_pairs, const int32_t *__restrict__ pairs,
+    int pair_width, ElasticConsts c, const int32_t *__restrict__ rows,
     double *__restrict__ out) {
     constexpr int NI = n_inner<KID>(), NA = n_outer<KID>();
     constexpr bool FS = fix_src<KID>();
@@ -201,55 +202,62 @@ __global__ __launch_bounds__(256) void pairs_product_kernel(
         }
     }
     const bool same = pp[0] == pp[1] && oc == sc && !flip;
-    const SideRule rf = FS ? rs : ro, rm = FS ? ro : rs;
-    const rule_ptr mq = (rule_ptr)rm.q, mw = (rule_ptr)rm.w;
     const double *mn = FS ? mo : ns;   // the moving side's normal
 
     double acc[NA];
 #pragma unroll
     for (int k = 0; k < NA; ++k) acc[k] = 0.0;
-    const int groups = (rf.n + P - 1) / P;
-    for (int g0 = 0; g0 < groups; g0 += GL) {
-        // a lane without a group, and points past the end of the rule, repeat
-        // the last point with weight zero
-        double F[P][3], fq[P][2], wf[P], a[P][NI];
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            const int i = (g0 + sub) * P + p;
-            const int ic = i < rf.n ? i : rf.n - 1;
-            fq[p][0] = rf.q[2 * ic];
-            fq[p][1] = rf.q[2 * ic + 1];
-            wf[p] = i < rf.n ? rf.w[ic] : 0.0;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) F[p][d] = fma(fq[p][1], fe[1][d], fq[p][0] * fe[0][d]);
-#pragma unroll
-            for (int k = 0; k < NI; ++k) a[p][k] = 0.0;
-        }
-        double qx = mq[0], qy = mq[1], qw = mw[0];
+    // the rule, then the one to subtract (on both sides, with the fixed
+    // points' weights negative): the outputs are linear in the sums
 #pragma unroll 1
-        for (int j = 0; j < rm.n; ++j) {
-            // wait for this point's scalar loads here, then issue the next
-            // one's: they come back while this point computes
-            asm volatile("" : "+v"(m0[0]), "+v"(m0[1]), "+v"(m0[2]), "+v"(KID == TCT_RH ? acc[0] : a[P - 1][NI - 1])
-                         : "s"(qw) : "memory");
-            const double x = qx, y = qy, w = qw;
-            const int jn = j + 1 < rm.n ? j + 1 : j;
-            qx = mq[2 * jn];
-            qy = mq[2 * jn + 1];
-            qw = mw[jn];
-            double M[3];
+    for (int pass = 0; pass < (minus.n > 0 ? 2 : 1); ++pass) {
+        const SideRule rf = pass ? minus : (FS ? rs : ro), rm = pass ? minus : (FS ? ro : rs);
+        const rule_ptr mq = (rule_ptr)rm.q, mw = (rule_ptr)rm.w;
+        const int groups = (rf.n + P - 1) / P;
+        for (int g0 = 0; g0 < groups; g0 += GL) {
+            // a lane without a group, and points past the end of the rule, repeat
+            // the last point with weight zero
+            double F[P][3], fq[P][2], wf[P], a[P][NI];
 #pragma unroll
-            for (int d = 0; d < 3; ++d) M[d] = fma(y, me[1][d], fma(x, me[0][d], m0[d]));
-            walk_point<KID, P, CK>(M, x, y, w, F, fq, wf, same, mo, ns, c, acc, a);
-        }
-        if constexpr (KID != TCT_RH)
+            for (int p = 0; p < P; ++p) {
+                const int i = (g0 + sub) * P + p;
+                const int ic = i < rf.n ? i : rf.n - 1;
+                fq[p][0] = rf.q[2 * ic];
+                fq[p][1] = rf.q[2 * ic + 1];
+                wf[p] = i < rf.n ? (pass ? -rf.w[ic] : rf.w[ic]) : 0.0;
 #pragma unroll
-        for (int p = 0; p < P; ++p) {
-            double dn = 0.0;
-            if constexpr (KID == TCT_RT || KID == TCT_RA)
+                for (int d = 0; d < 3; ++d) F[p][d] = fma(fq[p][1], fe[1][d], fq[p][0] * fe[0][d]);
 #pragma unroll
-                for (int d = 0; d < 3; ++d) dn = fma(mn[d], m0[d] - F[p][d], dn);
-            fold_point<KID>(a[p], wf[p], fq[p][0], fq[p][1], dn, c, acc);
+                for (int k = 0; k < NI; ++k) a[p][k] = 0.0;
+            }
+            double qx = mq[0], qy = mq[1], qw = mw[0];
+#pragma unroll 1
+            for (int j = 0; j < rm.n; ++j) {
+                // wait for this point's scalar loads here, then issue the next
+                // one's: they come back while this point computes
+                double &dep = KID == TCT_RH ? acc[0] : a[P - 1][NI - 1];
+                asm volatile("" : "+v"(m0[0]), "+v"(m0[1]), "+v"(m0[2]), "+v"(dep)
+                             : "s"(qw) : "memory");
+                const double x = qx, y = qy, w = qw;
+                const int jn = j + 1 < rm.n ? j + 1 : j;
+                qx = mq[2 * jn];
+                qy = mq[2 * jn + 1];
+                qw = mw[jn];
+                double M[3];
+#pragma unroll
+                for (int d = 0; d < 3; ++d) M[d] = fma(y, me[1][d], fma(x, me[0][d], m0[d]));
+                walk_point<KID, P, CK>(M, x, y, w, F, fq, wf, same, mo, ns, c, acc, a);
+            }
+            if constexpr (KID != TCT_RH) {
+#pragma unroll
+                for (int p = 0; p < P; ++p) {
+                    double dn = 0.0;
+                    if constexpr (KID == TCT_RT || KID == TCT_RA)
+#pragma unroll
+                        for (int d = 0; d < 3; ++d) dn = fma(mn[d], m0[d] - F[p][d], dn);
+                    fold_point<KID>(a[p], wf[p], fq[p][0], fq[p][1], dn, c, acc);
+                }
+            }
         }
     }
     if constexpr (GL > 1) {
@@ -286,8 +294,8 @@ __global__ __launch_bounds__(256) void pairs_product_kernel(
                 pack_pair<KID>(acc, ot, st, c, oc, sc, flip, p);
             }
         },
-        table, stage[threadIdx.x / 64], (int)(threadIdx.x % 64) / GL, sub == 0, live ? pair : -1,
-        out);
+        table, stage[threadIdx.x / 64], (int)(threadIdx.x % 64) / GL, sub == 0,
+        live ? out_row(rows, pair) : -1, out);
 }
 
 // Fixed points per lane (P) and lanes per pair (GL) for a rule of nf fixed
@@ -326,20 +334,41 @@ inline Split product_split(int kernel, int nf, int nm, int64_t n_pairs) {
     return best;
 }
 
+struct ProductArgs {
+    SideRule ro, rs, minus;
+    const double *pts;
+    const int32_t *tris;
+    int n_pairs;
+    const int32_t *pairs;
+    int pair_width, check0;
+    ElasticConsts c;
+    const int32_t *rows;
+    bool subtract;
+    double *out;
+};
+
+template <int KID, int P, int GL, int CK, bool SUB>
+static void product_launch(const ProductArgs &a, hipStream_t st) {
+    const unsigned nb = (unsigned)ceil_div((int64_t)a.n_pairs * GL, (int64_t)256);
+    hipLaunchKernelGGL((pairs_product_kernel<KID, P, GL, CK, SUB>), dim3(nb), dim3(256), 0, st,
+                       a.ro, a.rs, a.minus, a.pts, a.tris, a.n_pairs, a.pairs, a.pair_width, a.c,
+                       a.rows, a.out);
+}
+
 template <int KID, int P, int GL>
-static void product_go(int check0, hipStream_t st, const SideRule &ro, const SideRule &rs,
-                       const double *pts, const int32_t *tris, int n_pairs, const int32_t *pairs,
-                       int pair_width, const ElasticConsts &c, double *out) {
-    const unsigned nb = (unsigned)ceil_div((int64_t)n_pairs * GL, (int64_t)256);
-#define TCT_PP(CK)                                                                             \
-    hipLaunchKernelGGL((pairs_product_kernel<KID, P, GL, CK, false>), dim3(nb), dim3(256), 0, st, ro, \
-                       rs, pts, tris, n_pairs, pairs, pair_width, c, out)
+static void product_go(const ProductArgs &a, hipStream_t st) {
     // where no point has equal parameters the full test is the r2 == 0 test
-    if (check0 == CK_NONE)
-        TCT_PP(CK_NONE);
-    else
-        TCT_PP(CK_FULL);
-#undef TCT_PP
+    if (a.check0 == CK_NONE) {
+        if (a.subtract)
+            product_launch<KID, P, GL, CK_NONE, true>(a, st);
+        else
+            product_launch<KID, P, GL, CK_NONE, false>(a, st);
+    } else {
+        if (a.subtract)
+            product_launch<KID, P, GL, CK_FULL, true>(a, st);
+        else
+            product_launch<KID, P, GL, CK_FULL, false>(a, st);
+    }
 }
 
 }  // namespace tct
@@ -347,10 +376,11 @@ static void product_go(int check0, hipStream_t st, const SideRule &ro, const Sid
 using namespace tct;
 
 extern "C" int tct_pairs_product(int kernel, int n_o, const double *qo, const double *wo, int n_s,
-                                 const double *qs, const double *ws, const double *pts,
+                                 const double *qs, const double *ws, int n_minus,
+                                 const double *q_minus, const double *w_minus, const double *pts,
                                  const int32_t *tris, int64_t n_pairs, const int32_t *pairs,
                                  int pair_width, int check0, const double *params_host,
-                                 double *out, void *stream) {
+                                 const int32_t *rows, int subtract, double *out, void *stream) {
     TCT_CHECK_ARG(kernel >= TCT_U && kernel <= TCT_RH, "pairs_product: kernel id %d", kernel);
     TCT_CHECK_ARG(n_o > 0 && n_s > 0 && n_o < (1 << 20) && n_s < (1 << 20),
                   "pairs_product: rules of %d x %d points", n_o, n_s);
@@ -359,19 +389,20 @@ extern "C" int tct_pairs_product(int kernel, int n_o, const double *qo, const do
     TCT_CHECK_ARG(pair_width == 2 || pair_width == 5, "pairs_product: pair_width %d", pair_width);
     TCT_CHECK_ARG(check0 == CK_NONE || check0 == CK_FULL || check0 == CK_R2,
                   "pairs_product: check0 %d", check0);
+    TCT_CHECK_ARG(n_minus >= 0 && n_minus < (1 << 20) && (n_minus == 0 || (q_minus && w_minus)),
+                  "pairs_product: rule of %d points to subtract", n_minus);
     TCT_CHECK_ARG(qo && wo && qs && ws && pts && tris && params_host && out &&
                       (pairs || n_pairs == 0),
                   "pairs_product: null pointer");
     if (n_pairs == 0) return TCT_OK;
-    const SideRule ro{n_o, qo, wo}, rs{n_s, qs, ws};
     const int nf = kernel == TCT_RA ? n_s : n_o;
     const Split sp = product_split(kernel, nf, kernel == TCT_RA ? n_o : n_s, n_pairs);
     const int P = sp.P, gl = sp.GL;
-    const ElasticConsts c = elastic_consts(params_host);
     hipStream_t st = as_stream(stream);
-    const int np = (int)n_pairs;
-#define TCT_GO(K, P, GL)                                                                         \
-    product_go<K, P, GL>(check0, st, ro, rs, pts, tris, np, pairs, pair_width, c, out)
+    const ProductArgs args{{n_o, qo, wo}, {n_s, qs, ws}, {n_minus, q_minus, w_minus},
+                           pts, tris, (int)n_pairs, pairs, pair_width, check0,
+                           elastic_consts(params_host), rows, subtract != 0, out};
+#define TCT_GO(K, P, GL) product_go<K, P, GL>(args, st)
 #define TCT_GL(K, P)                                                                             \
     switch (gl) {                                                                                \
     case 1: TCT_GO(K, P, 1); break;                                                              \

@@ -97,9 +97,90 @@ __global__ __launch_bounds__(256) void csr_kernel(int n_rows, const int32_t *__r
     y[r] = accumulate ? y[r] + s : s;
 }
 
+// Lists of blocks, each sorted by (row, column), merged into block rows by
+// rank: a block's position is its own index plus, for every other list, the
+// number of blocks before it there (equal ones of an earlier list first), a
+// binary search each.  One launch in place of a sort of all keys, a histogram
+// and a scan with a host wait.
+constexpr int MERGE_MAX = 4;
+struct MergeLists {
+    int n_lists, total, n_rows;
+    int n[MERGE_MAX], start[MERGE_MAX], stride[MERGE_MAX];
+    const int32_t *dofs[MERGE_MAX];
+    int32_t *rank[MERGE_MAX];
+};
+
+// Blocks of list k before (row, col): before or at it with `at`.
+__device__ __forceinline__ int blocks_before(const MergeLists &m, int k, int row, int col, bool at) {
+    int lo = 0, hi = m.n[k];
+    while (lo < hi) {
+        const int mid = (lo + hi) / 2;
+        const int32_t *d = m.dofs[k] + (size_t)mid * m.stride[k];
+        const int r = d[0], c = d[1];
+        const bool before = r < row || (r == row && (c < col || (at && c == col)));
+        lo = before ? mid + 1 : lo;
+        hi = before ? hi : mid;
+    }
+    return lo;
+}
+
+__global__ __launch_bounds__(256) void bsr_merge_kernel(MergeLists m,
+                                                        int32_t *__restrict__ indices,
+                                                        int32_t *__restrict__ indptr) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < m.total) {
+        int k = 0;
+        while (k + 1 < m.n_lists && t >= m.start[k + 1]) ++k;
+        const int i = t - m.start[k];
+        const int32_t *d = m.dofs[k] + (size_t)i * m.stride[k];
+        const int row = d[0], col = d[1];
+        int r = i;
+        for (int j = 0; j < m.n_lists; ++j)
+            if (j != k) r += blocks_before(m, j, row, col, j < k);
+        m.rank[k][i] = r;
+        indices[r] = col;
+    }
+    if (t <= m.n_rows) {
+        int s = 0;
+        for (int j = 0; j < m.n_lists; ++j) s += blocks_before(m, j, t, 0, false);
+        indptr[t] = s;
+    }
+}
+
 }  // namespace tct
 
 using namespace tct;
+
+extern "C" int tct_bsr_merge(int n_lists, const int64_t *n, const int32_t *const *dofs,
+                             const int *strides, int64_t n_rows, int32_t *const *rank,
+                             int32_t *indices, int32_t *indptr, void *stream) {
+    TCT_CHECK_ARG(n_lists >= 0 && n_lists <= MERGE_MAX, "bsr_merge: %d lists", n_lists);
+    TCT_CHECK_ARG(n_rows >= 0 && n_rows < (1LL << 31) - 1, "bsr_merge: n_rows %lld",
+                  (long long)n_rows);
+    TCT_CHECK_ARG(indptr && (n_lists == 0 || (n && dofs && strides && rank && indices)),
+                  "bsr_merge: null pointer");
+    MergeLists m{};
+    m.n_lists = n_lists;
+    m.n_rows = (int)n_rows;
+    int64_t total = 0;
+    for (int k = 0; k < n_lists; ++k) {
+        TCT_CHECK_ARG(n[k] >= 0 && strides[k] >= 2 && (n[k] == 0 || (dofs[k] && rank[k])),
+                      "bsr_merge: list %d", k);
+        m.n[k] = (int)n[k];
+        m.start[k] = (int)total;
+        m.stride[k] = strides[k];
+        m.dofs[k] = dofs[k];
+        m.rank[k] = rank[k];
+        total += n[k];
+        TCT_CHECK_ARG(total < (1LL << 31), "bsr_merge: too many blocks");
+    }
+    m.total = (int)total;
+    const int64_t threads = total > n_rows + 1 ? total : n_rows + 1;
+    hipLaunchKernelGGL(bsr_merge_kernel, dim3((unsigned)ceil_div(threads, (int64_t)256)),
+                       dim3(256), 0, as_stream(stream), m, indices, indptr);
+    TCT_CHECK_LAUNCH("bsr_merge");
+    return TCT_OK;
+}
 
 extern "C" int tct_bsr9_spmv(int64_t n_block_rows, const int32_t *indptr,
                              const int32_t *indices, const double *data, const double *x,

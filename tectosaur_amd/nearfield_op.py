@@ -15,13 +15,15 @@ Assembly (one-time, per mesh), following nearfield_op.py:95-141:
     keeps four BCOO matrices and applies them on the host).
 All integration runs on the device in FP64 (pairs.hip).
 """
+import ctypes
+
 import numpy as np
 import torch
 
 from . import _native as N
 from . import find_near_adj
-from .pairs_integrator import PairsIntegrator
-from .sparse import bcoo_to_bsr_dev
+from .pairs_integrator import PairsIntegrator, check_pairs
+from .sparse import BSRMatrix, bcoo_to_bsr_dev
 
 
 def edge_adj_orient(tv0, tv1):
@@ -53,11 +55,15 @@ def _is_identity(subset):
 
 def to_tri_space(dof_indices, obs_subset, src_subset):
     di = np.asarray(dof_indices, dtype=np.int64)
+    # identity subsets (the whole mesh) map positions to themselves: the
+    # array itself where both are
+    o_id, s_id = _is_identity(obs_subset), _is_identity(src_subset)
+    if o_id and s_id:
+        return di
     out = di.copy()
-    # identity subsets (the whole mesh) map positions to themselves
-    if not _is_identity(obs_subset):
+    if not o_id:
         out[:, 0] = obs_subset[di[:, 0]]
-    if not _is_identity(src_subset):
+    if not s_id:
         out[:, 1] = src_subset[di[:, 1]]
     return out
 
@@ -126,7 +132,7 @@ class RegularizedNearfieldIntegralOp:
         self.device = N.require_device()
         dev = self.device
         pairs_int = PairsIntegrator(K_near_name, params, float_type, nq_far, nq_near, pts, tris)
-        corr_int = PairsIntegrator(K_far_name, params, float_type, nq_far, nq_near, pts, tris)
+        corr_int = pairs_int.with_kernel(K_far_name)
         if plan is None:
             plan = nearfield_plan(pts, tris, obs_subset, src_subset, near_threshold)
 
@@ -148,14 +154,16 @@ class RegularizedNearfieldIntegralOp:
                    ('ea',) + plan['ea'] + (True, False),
                    ('va',) + plan['va'] + (True, False),
                    ('near',) + plan['near'] + (False, False))
-        rows, cols, corrected, uncorrected = [], [], [], []
-        self.counts = {}
+        self.counts = {name: int(prs.shape[0]) for name, prs, _, _, _ in classes}
         self.classes = {}
+        self.n_pairs = sum(self.counts.values())
+        if not keep_classes and self._assemble_rows(classes, rules, far_q, pairs_int, corr_int,
+                                                    tris.shape[0], keep_uncorrected):
+            return
+        rows, cols, corrected, uncorrected = [], [], [], []
         for name, prs, dofs, check0, corr_check0 in classes:
-            self.counts[name] = int(prs.shape[0])
             if prs.shape[0] == 0:
                 continue
-            from .pairs_integrator import check_pairs
             check_pairs(prs, tris.shape[0])
             p_dev = N.upload(prs.astype(np.int32), None, dev)
             acc = pairs_int.pairs_quad_dev(rules[name], p_dev, check0)
@@ -182,7 +190,94 @@ class RegularizedNearfieldIntegralOp:
             e = torch.zeros(0, dtype=torch.int64, device=dev)
             self.mat = bcoo_to_bsr_dev(e, e, z, self.shape)
             self.mat_no_correction = self.mat
-        self.n_pairs = sum(self.counts.values())
+
+    def _assemble_rows(self, classes, rules, far_q, pairs_int, corr_int, n_tris,
+                       keep_uncorrected):
+        """The matrix with every block integrated straight into its place.
+
+        Each class comes sorted by (obs, src) from the finder, so a block's
+        place is its rank in the merge of at most four sorted lists
+        (tct_bsr_merge), and the integrators write there: no list of accurate
+        blocks, list of corrections, difference, concatenation and reordering,
+        each a pass over 648 bytes a pair.  Where both kernels are the same and
+        the accurate rule is a product rule the correction is part of the
+        same pass; otherwise it is subtracted in place.  Returns False,
+        having done nothing, for lists that are not sorted (or dofs outside
+        the matrix), which the general way below takes."""
+        dev = self.device
+        nr, nc = self.shape[0] // 9, self.shape[1] // 9
+        # (name, pairs, dofs or None where they are the pairs', tests)
+        work = []
+        for name, prs, dofs, check0, corr_check0 in classes:
+            if prs.shape[0] == 0:
+                continue
+            prs = np.ascontiguousarray(prs, dtype=np.int64)
+            dofs = np.asarray(dofs, dtype=np.int64)
+            if dofs.shape != (prs.shape[0], 2) or prs.shape[1] not in (2, 5):
+                return False
+            if dofs.strides[1] != 8 or dofs.strides[0] % 8 or dofs.strides[0] < 16:
+                dofs = np.ascontiguousarray(dofs)
+            same = ctypes.c_int(dofs is prs)
+            if not same.value:
+                N.call('tct_pairs_same', prs.shape[0], prs.shape[1], N.ptr(prs), N.ptr(dofs),
+                       dofs.strides[0] // 8, ctypes.byref(same))
+            work.append((name, prs, None if same.value else dofs, check0, corr_check0))
+        if not work:
+            return False
+        # pairs, and dofs where they are others, as int32 in one pinned
+        # buffer: one conversion pass, one copy
+        n = [c[1].shape[0] for c in work]
+        width = [c[1].shape[1] for c in work]
+        own = [c[2] is not None for c in work]
+        size = [k * (w + 2 * o) for k, w, o in zip(n, width, own)]
+        off = np.concatenate([[0], np.cumsum(size)]).astype(np.int64)
+        host = torch.empty(int(off[-1]), dtype=torch.int32, pin_memory=True)
+        flag = ctypes.c_int(0)
+        for (_, prs, dofs, _, _), o, k, w in zip(work, off, n, width):
+            at = host.data_ptr() + 4 * int(o)
+            d = dofs is not None
+            rc = N.lib().tct_pairs_pack(
+                k, w, N.ptr(prs), n_tris, N.ptr(dofs), dofs.strides[0] // 8 if d else 0, nr, nc,
+                at, at + 4 * k * w if d else None, ctypes.byref(flag))
+            if rc != 0 or not flag.value:
+                check_pairs(prs, n_tris)      # raises for a bad pair
+                return False
+        buf = host.to(dev, non_blocking=True)
+        total = sum(n)
+        rank = torch.empty(total, dtype=torch.int32, device=dev)
+        indices = torch.empty(total, dtype=torch.int32, device=dev)
+        indptr = torch.empty(nr + 1, dtype=torch.int32, device=dev)
+        start = np.concatenate([[0], np.cumsum(n)[:-1]]).astype(np.int64)
+        ptrs = lambda base, offs: (ctypes.c_void_p * len(n))(*[base + 4 * int(i) for i in offs])
+        dof_off = [o + (k * w if d else 0) for o, k, w, d in zip(off, n, width, own)]
+        N.call('tct_bsr_merge', len(n), (ctypes.c_int64 * len(n))(*n),
+               ptrs(N.ptr(buf), dof_off),
+               (ctypes.c_int * len(n))(*[2 if d else w for w, d in zip(width, own)]), nr,
+               ptrs(N.ptr(rank), start), N.ptr(indices), N.ptr(indptr), N.stream_ptr())
+        data = torch.empty((total, 81), dtype=torch.float64, device=dev)
+        same = corr_int is pairs_int
+        plain = None
+        lists = []
+        for (name, _, _, check0, corr_check0), o, k, w, s in zip(work, off, n, width, start):
+            p_dev = buf[int(o):int(o) + k * w].view(k, w)
+            r_dev = rank[int(s):int(s) + k]
+            q = rules[name]
+            fused = (same and not keep_uncorrected and w == 2 and check0 == corr_check0 and
+                     pairs_int.product_side(q) is not None)
+            pairs_int.pairs_quad_rows(q, p_dev, check0, r_dev, data,
+                                      minus=far_q if fused else None)
+            if not fused:
+                lists.append((p_dev, r_dev, corr_check0))
+        if keep_uncorrected:
+            plain = data.clone()
+        for p_dev, r_dev, corr_check0 in lists:
+            # the correction takes the triangles in their own frames
+            corr_int.pairs_quad_rows(far_q, p_dev[:, :2].contiguous(), corr_check0, r_dev, data,
+                                     subtract=True)
+        self.mat = BSRMatrix(indptr, indices, data, self.shape)
+        self.mat_no_correction = (BSRMatrix(indptr, indices, plain, self.shape)
+                                  if keep_uncorrected else None)
+        return True
 
     def dot_dev(self, x, out=None, accumulate=False, prec='f64'):
         """prec other than 'f64' uses the FP32 copy of the blocks when one

@@ -10,6 +10,7 @@ summation); results are returned as float64.
 The ``*_dev`` variants take and return device tensors, for assembling the
 nearfield matrix without host round trips.
 """
+import copy
 import threading
 
 import numpy as np
@@ -108,6 +109,49 @@ class PairsIntegrator:
             self._rules[key] = q
         return self._rules[key]
 
+    def with_kernel(self, kernel):
+        """An integrator of another kernel on the same mesh and rules."""
+        if kernel == self.kernel:
+            return self
+        o = copy.copy(self)
+        o.kernel = kernel
+        o.kid = N.KERNEL_IDS[kernel]
+        return o
+
+    def product_side(self, q):
+        """The triangle rule of a product rule that this kernel runs as one,
+        or None."""
+        side = getattr(q, 'side', None)
+        return side if side is not None and product_pays(self.kernel, side[1].shape[0]) else None
+
+    def pairs_quad_rows(self, q, pairs_dev, check0, rows, out, minus=None, subtract=False):
+        """Pair i's block into row rows[i] (int32 device tensor) of ``out``
+        [., 81].  minus: a product rule whose integrals of the same pairs are
+        subtracted (q must be one too: ``product_side``).  subtract: the
+        integrals are subtracted from the rows instead of written."""
+        n = pairs_dev.shape[0]
+        width = pairs_dev.shape[1]
+        side = getattr(q, 'side', None)
+        product = self.product_side(q) is not None or subtract
+        if (minus is not None or subtract) and (side is None or not product):
+            raise N.TctError('only product rules subtract')
+        mq, mw = (None, None) if minus is None else minus.side
+        st = N.stream_ptr()
+        for s in range(0, n, CALL_SIZE):
+            e = min(n, s + CALL_SIZE)
+            if product:
+                sq, sw = side
+                N.call('tct_pairs_product', self.kid, sw.shape[0], N.ptr(sq), N.ptr(sw),
+                       sw.shape[0], N.ptr(sq), N.ptr(sw), 0 if mw is None else mw.shape[0],
+                       N.ptr(mq), N.ptr(mw), N.ptr(self.gpu_pts), N.ptr(self.gpu_tris), e - s,
+                       N.ptr(pairs_dev[s:e]), width, r0_test_mode(q, check0),
+                       self.params.ctypes.data, N.ptr(rows[s:e]), int(subtract), N.ptr(out), st)
+            else:
+                N.call('tct_pairs_integrate_rows', self.kid, q[0].shape[0], N.ptr(q[0]),
+                       N.ptr(q[1]), N.ptr(self.gpu_pts), N.ptr(self.gpu_tris), e - s,
+                       N.ptr(pairs_dev[s:e]), width, r0_test_mode(q, check0),
+                       self.params.ctypes.data, 0, N.ptr(rows[s:e]), N.ptr(out), st)
+
     def pairs_quad_dev(self, q, pairs_dev, check0, out=None, lanes_per_pair=0):
         """pairs_dev: int32 device tensor [n, 2] or [n, 5]; returns [n, 81]."""
         n = pairs_dev.shape[0]
@@ -117,17 +161,16 @@ class PairsIntegrator:
         st = N.stream_ptr()
         # a rule that is a product runs as one, unless the caller chooses how
         # many lanes share a pair's 4-D rule
-        side = getattr(q, 'side', None) if lanes_per_pair == 0 else None
-        if side is not None and not product_pays(self.kernel, side[1].shape[0]):
-            side = None
+        side = self.product_side(q) if lanes_per_pair == 0 else None
         for s in range(0, n, CALL_SIZE):
             e = min(n, s + CALL_SIZE)
             if side is not None:
                 sq, sw = side
                 N.call('tct_pairs_product', self.kid, sw.shape[0], N.ptr(sq), N.ptr(sw),
-                       sw.shape[0], N.ptr(sq), N.ptr(sw), N.ptr(self.gpu_pts),
+                       sw.shape[0], N.ptr(sq), N.ptr(sw), 0, None, None, N.ptr(self.gpu_pts),
                        N.ptr(self.gpu_tris), e - s, N.ptr(pairs_dev[s:e]), width,
-                       r0_test_mode(q, check0), self.params.ctypes.data, N.ptr(out[s:e]), st)
+                       r0_test_mode(q, check0), self.params.ctypes.data, None, 0,
+                       N.ptr(out[s:e]), st)
                 continue
             N.call('tct_pairs_integrate', self.kid, q[0].shape[0], N.ptr(q[0]), N.ptr(q[1]),
                    N.ptr(self.gpu_pts), N.ptr(self.gpu_tris), e - s, N.ptr(pairs_dev[s:e]),

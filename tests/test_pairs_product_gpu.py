@@ -55,8 +55,8 @@ def test_product_rule_vs_oracle(oracle, K, n, order):
     out = torch.full((n + 1, 81), 7.0, dtype=torch.float64, device='cuda')
     m = side[1].shape[0]
     N.call('tct_pairs_product', pi.kid, m, N.ptr(side[0]), N.ptr(side[1]), m, N.ptr(side[0]),
-           N.ptr(side[1]), N.ptr(pi.gpu_pts), N.ptr(pi.gpu_tris), n, N.ptr(p), 2, 0,
-           pi.params.ctypes.data, N.ptr(out), N.stream_ptr())
+           N.ptr(side[1]), 0, None, None, N.ptr(pi.gpu_pts), N.ptr(pi.gpu_tris), n, N.ptr(p), 2, 0,
+           pi.params.ctypes.data, None, 0, N.ptr(out), N.stream_ptr())
     out = out.cpu().numpy()
     assert _close(out[:n], want) <= 1e-10
     assert np.all(out[n] == 7.0)      # nothing past the last pair
@@ -90,3 +90,47 @@ def test_product_rule_many_pairs(K):
     got = pi.pairs_quad_dev(pi.near_q, p, False).cpu().numpy()
     want = pi.pairs_quad_dev(pi.near_q, p, False, lanes_per_pair=1).cpu().numpy()
     assert _close(got, want) <= 1e-10
+
+
+@pytest.mark.parametrize('kernels', [('elasticRH3', 'elasticRH3'), ('elasticRH3', 'elasticH3'),
+                                     ('elasticRT3', 'elasticRT3'), ('elasticU3', 'elasticU3')])
+@pytest.mark.parametrize('which', ['whole', 'subset', 'keep', 'unsorted'])
+def test_blocks_integrated_into_place_equal_the_lists(kernels, which):
+    # the matrix assembled in place against the one from lists of accurate
+    # blocks and corrections (keep_classes), for the whole mesh, subsets whose
+    # dofs are not the triangles, the uncorrected matrix beside it, and a plan
+    # that is not sorted (general way)
+    from tectosaur_amd.nearfield_op import RegularizedNearfieldIntegralOp, nearfield_plan
+    pts, tris = _mesh()
+    n = tris.shape[0]
+    obs, src = (np.arange(40, 170), np.arange(10, 200)) if which == 'subset' else \
+        (np.arange(n), np.arange(n))
+    plan = nearfield_plan(pts, tris, obs, src, 2.0)
+    if which == 'unsorted':
+        k = np.random.default_rng(0).permutation(plan['near'][0].shape[0])
+        plan['near'] = tuple(a[k] for a in plan['near'])
+    args = (pts, tris, obs, src, 3, 3, 3, 1, 3, 2.0) + kernels + (PARAMS, np.float64)
+    keep = which == 'keep'
+    a = RegularizedNearfieldIntegralOp(*args, plan=plan, keep_uncorrected=keep)
+    b = RegularizedNearfieldIntegralOp(*args, plan=plan, keep_uncorrected=keep, keep_classes=True)
+    assert a.counts == b.counts and a.n_pairs == b.n_pairs
+    for x, y in ((a.mat, b.mat), (a.mat_no_correction, b.mat_no_correction))[:1 + keep]:
+        assert torch.equal(x.indptr, y.indptr) and torch.equal(x.indices, y.indices)
+        scale = y.data.abs().amax(1, keepdim=True)
+        assert float(((x.data - y.data).abs() / scale).max()) <= 1e-10
+    assert keep or a.mat_no_correction is None
+
+
+def test_bad_plans_are_refused():
+    from tectosaur_amd.nearfield_op import RegularizedNearfieldIntegralOp, nearfield_plan
+    pts, tris = _mesh()
+    idx = np.arange(tris.shape[0])
+    for col, val, err in ((0, -1, IndexError), (1, tris.shape[0], IndexError),
+                          (2, 3, ValueError), (4, 2, ValueError)):
+        plan = nearfield_plan(pts, tris, idx, idx, 2.0)
+        prs = plan['ea'][0].copy()
+        prs[7, col] = val
+        plan['ea'] = (prs, plan['ea'][1])
+        with pytest.raises(err):
+            RegularizedNearfieldIntegralOp(pts, tris, idx, idx, 3, 3, 3, 1, 3, 2.0, 'elasticRH3',
+                                           'elasticRH3', PARAMS, np.float64, plan=plan)
