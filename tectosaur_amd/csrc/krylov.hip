@@ -224,6 +224,109 @@ __global__ __launch_bounds__(KB) void reduce_update_dot_kernel(
     }
 }
 
+// A step's pass over V with its columns in registers: a workgroup of eight
+// waves takes 64 points at a time, lane = point, and wave wv holds columns wv,
+// wv + 8, ... of them (NC a lane); then every lane adds V_i w to the running
+// sum of each of its columns, which meet in a butterfly after the last tile.
+//   MODE 0: the sums V w.
+//   MODE 1: w' = w - V^T c first (the waves' partial sums through LDS), then
+//           the sums V w'.
+//   MODE 2: w' = w - V^T c, then the sum of w'^2 (partial_out's one column).
+// c: c_in, or, without, the column sums of partial_in [m][nb_in] formed by
+// every workgroup, one wave a column in a fixed order, and written to hout
+// (plus add) by the first.
+// What bounds it: HBM at large n, where reduce_update_dot_kernel reads its
+// block's slice of V twice, beyond any cache; a whole step then reads V three
+// times (n = 978,432, m = 200: 4.7 GB in 903 us, 5.2 TB/s; walking, 6.3 GB in
+// 1,265).  Latency at small n, where a walking block takes its columns eight at
+// a time and few blocks have work (n = 8,370, m = 30: nine blocks, 49 us a step;
+// here 131 blocks with all their loads in flight, 22 us).  Registers hold up to
+// 400 columns (222 VGPRs, one workgroup a CU; m = 400 at the large n: 2,430 us
+// -> 1,740).
+constexpr int OW = 8;              // waves of a workgroup
+constexpr int ONCE_MAX_M = OW * 50;
+
+template <int NC, int MODE>
+__global__ __launch_bounds__(64 * OW) void once_kernel(
+    int m, int64_t n, int64_t ld, const double *__restrict__ V,
+    const double *__restrict__ partial_in, int nb_in, const double *__restrict__ c_in,
+    const double *__restrict__ add, double *__restrict__ hout, double *__restrict__ w,
+    double *__restrict__ partial_out) {
+    __shared__ double c[OW * NC];
+    __shared__ double part[2][OW][64];
+    const int lane = (int)threadIdx.x % 64;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
+    const int nb = gridDim.x;
+    const int64_t tiles = (n + 63) / 64;
+    const int64_t t0 = tiles * blockIdx.x / nb, t1 = tiles * (blockIdx.x + 1) / nb;
+    if constexpr (MODE > 0) {
+        if (c_in) {
+            for (int i = threadIdx.x; i < OW * NC; i += 64 * OW) c[i] = i < m ? c_in[i] : 0.0;
+        } else {
+#pragma unroll 4
+            for (int k = 0; k < NC; ++k) {
+                const int i = k * OW + wave;
+                double s = 0.0;
+                if (i < m)
+                    for (int b = lane; b < nb_in; b += 64) s += partial_in[(size_t)i * nb_in + b];
+#pragma unroll
+                for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+                if (lane == 0) {
+                    c[i] = s;
+                    if (i < m && blockIdx.x == 0) hout[i] = add ? s + add[i] : s;
+                }
+            }
+        }
+        __syncthreads();
+    }
+    double acc[MODE == 2 ? 1 : NC];
+#pragma unroll
+    for (int k = 0; k < (MODE == 2 ? 1 : NC); ++k) acc[k] = 0.0;
+    int par = 0;   // one barrier per tile: the partial sums are double-buffered
+    for (int64_t tile = t0; tile < t1; ++tile, par ^= 1) {
+        const int64_t t = tile * 64 + lane;
+        const bool ok = t < n;
+        const int64_t tc = ok ? t : n - 1;
+        double v[NC];
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            // columns past the last (their c is 0, their sums are not
+            // stored) read the last again
+            const int i = k * OW + wave < m ? k * OW + wave : m - 1;
+            v[k] = V[(size_t)i * ld + tc];
+        }
+        const double wt = w[tc];
+        double u = wt;
+        if constexpr (MODE > 0) {
+            double s = 0.0;
+#pragma unroll
+            for (int k = 0; k < NC; ++k) s = fma(v[k], c[k * OW + wave], s);
+            part[par][wave][lane] = s;
+            __syncthreads();
+            double r = 0.0;
+#pragma unroll
+            for (int j = 0; j < OW; ++j) r += part[par][j][lane];
+            u = wt - r;
+            if (wave == 0 && ok) w[t] = u;   // every wave has read w[t] before the barrier
+        }
+        u = ok ? u : 0.0;
+        if constexpr (MODE == 2) {
+            acc[0] = fma(u, u, acc[0]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < NC; ++k) acc[k] = fma(v[k], u, acc[k]);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < (MODE == 2 ? 1 : NC); ++k) {
+        double r = acc[k];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) r += __shfl_xor(r, off, 64);
+        const int i = k * OW + wave;
+        if (lane == 0 && i < (MODE == 2 ? 1 : m)) partial_out[(size_t)i * nb + blockIdx.x] = r;
+    }
+}
+
 // |w| from the norm partials (every block, same order), written to *hnorm
 // by block 0, and vnext (vnext2) = w / |w| when given.
 __global__ __launch_bounds__(KB) void norm_normalize_kernel(int64_t n,
@@ -232,17 +335,21 @@ __global__ __launch_bounds__(KB) void norm_normalize_kernel(int64_t n,
                                                             int nb, double *__restrict__ hnorm,
                                                             double *__restrict__ vnext,
                                                             double *__restrict__ vnext2) {
-    __shared__ double nrm;
-    if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int b = 0; b < nb; ++b) s += partial[b];
-        s = sqrt(s);
-        nrm = s;
-        if (blockIdx.x == 0) *hnorm = s;
-    }
+    // thread x adds partials x, x + KB, ... (one thread adding all 956 of
+    // n = 978,432 took 50 us), then the usual butterfly and the waves in order
+    __shared__ double sum[KB / 64];
+    double s = 0.0;
+    for (int b = threadIdx.x; b < nb; b += KB) s += partial[b];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (threadIdx.x % 64 == 0) sum[threadIdx.x / 64] = s;
     __syncthreads();
+    double d = 0.0;
+#pragma unroll
+    for (int wv = 0; wv < KB / 64; ++wv) d += sum[wv];
+    d = sqrt(d);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *hnorm = d;
     if (!vnext) return;
-    const double d = nrm;
     for (int64_t t = (int64_t)blockIdx.x * KB + threadIdx.x; t < n;
          t += (int64_t)gridDim.x * KB) {
         const double v = w[t] / d;
@@ -277,37 +384,94 @@ inline int n_blocks(int64_t n) {
 // block of the update (nb^2 m re-reads).
 constexpr int NB_SEPARATE_REDUCE = 128;
 
+// Workgroups of once_kernel: two on each of 256 CUs where V is large (never
+// more than the first sums have: the partial arrays are sized for those), one
+// a tile up to one on each CU where it is small (every one sums their partials).
+inline int once_blocks(int64_t n, bool sep) {
+    const int64_t tiles = (n + 63) / 64, most = sep ? (n_blocks(n) < 512 ? n_blocks(n) : 512) : 256;
+    return (int)(tiles < most ? tiles : most);
+}
+// Doubles of scratch for that form, and for the one that walks the columns.
+inline int64_t scratch_once(int m, int64_t n) {
+    const bool sep = n_blocks(n) >= NB_SEPARATE_REDUCE;
+    const int64_t nb = sep ? n_blocks(n) : once_blocks(n, false);
+    return 2 * nb * m + 2 * m;
+}
+inline int64_t scratch_walk(int m, int64_t n) { return 2 * (int64_t)n_blocks(n) * m + 2 * m; }
+
+template <int MODE>
+static void once_launch(int m, int64_t n, int64_t ld, const double *V, const double *partial_in,
+                        int nb_in, const double *c_in, const double *add, double *hout, double *w,
+                        double *partial_out, int nb, hipStream_t st) {
+#define TCT_ONCE(NC)                                                                           \
+    hipLaunchKernelGGL((once_kernel<NC, MODE>), dim3(nb), dim3(64 * OW), 0, st, m, n, ld, V,   \
+                       partial_in, nb_in, c_in, add, hout, w, partial_out)
+    const int nc = (m + OW - 1) / OW;
+    if (nc <= 2)
+        TCT_ONCE(2);
+    else if (nc <= 4)
+        TCT_ONCE(4);
+    else if (nc <= 8)
+        TCT_ONCE(8);
+    else if (nc <= 16)
+        TCT_ONCE(16);
+    else if (nc <= 26)
+        TCT_ONCE(26);
+    else if (nc <= 38)
+        TCT_ONCE(38);
+    else
+        TCT_ONCE(50);
+#undef TCT_ONCE
+}
+
 // The four (or six) launches of one CGS2 step; scratch = p1 [m][nb],
 // p2 [m][nb], h1 [m], c [m].
+//   m <= 400: the columns in registers (once_kernel).  With many blocks
+//   (n >= 131k) the first sums and the norm pass, which read V once anyway,
+//   keep the walking kernels and the column sums their own launch.
+//   m > 400, or a scratch for the walking form only: the columns walked eight
+//   at a time (multi_dot_kernel, reduce_update_dot_kernel).
 inline void cgs2_launch(int m, int64_t n, int64_t ld, const double *V, double *w, double *h,
-                        double *scratch, double *vnext, double *vnext2, hipStream_t st) {
-    const int nb = n_blocks(n);
+                        double *scratch, int64_t scratch_doubles, double *vnext, double *vnext2,
+                        hipStream_t st) {
+    const int nbw = n_blocks(n);
+    const bool sep = nbw >= NB_SEPARATE_REDUCE;
+    const bool once = m <= ONCE_MAX_M && scratch_doubles >= scratch_once(m, n);
+    const int nbs = once ? once_blocks(n, sep) : nbw;   // of the second sums
+    const int nb = once && !sep ? nbs : nbw;            // of the first sums and the norm
     double *p1 = scratch;                     // [m][nb], later the norm partials
     double *p2 = scratch + (size_t)nb * m;    // [m][nb]
     double *h1 = scratch + 2 * (size_t)nb * m;
     double *cs = h1 + m;                      // column sums (separate reduce)
-    const bool sep = nb >= NB_SEPARATE_REDUCE;
     const unsigned gr = (unsigned)ceil_div((int64_t)m, (int64_t)(KB / 64));
     // normalisation launch: enough blocks to cover the points, at most 1024
     const int64_t gpl = ceil_div(n, (int64_t)KB);
     const unsigned gp = (unsigned)(gpl < 1024 ? gpl : 1024);
     const size_t lds = sizeof(double) * (size_t)m;
+    const double *none = nullptr, *cin = sep ? cs : nullptr;
     // p1 = partial sums of V w
-    hipLaunchKernelGGL(multi_dot_kernel, dim3(nb), dim3(KB), 0, st, m, n, ld, V, w, 0, p1);
+    if (once && !sep)
+        once_launch<0>(m, n, ld, V, none, 0, none, none, nullptr, w, p1, nb, st);
+    else
+        hipLaunchKernelGGL(multi_dot_kernel, dim3(nb), dim3(KB), 0, st, m, n, ld, V, w, 0, p1);
     // h1 = sum p1; w -= V^T h1; p2 = partial sums of V w
     if (sep)
         hipLaunchKernelGGL(reduce_cols_kernel, dim3(gr), dim3(KB), 0, st, m, nb,
-                           (const double *)p1, (const double *)nullptr, cs, h1);
-    hipLaunchKernelGGL(reduce_update_dot_kernel, dim3(nb), dim3(KB), lds, st, m, n, ld, V,
-                       (const double *)p1, (const double *)(sep ? cs : nullptr),
-                       (const double *)nullptr, h1, w, 0, p2);
+                           (const double *)p1, none, cs, h1);
+    if (once)
+        once_launch<1>(m, n, ld, V, p1, nb, cin, none, h1, w, p2, nbs, st);
+    else
+        hipLaunchKernelGGL(reduce_update_dot_kernel, dim3(nb), dim3(KB), lds, st, m, n, ld, V,
+                           (const double *)p1, cin, none, h1, w, 0, p2);
     // h2 = sum p2, h = h1 + h2; w -= V^T h2; p1 = partial sums of w^2
     if (sep)
-        hipLaunchKernelGGL(reduce_cols_kernel, dim3(gr), dim3(KB), 0, st, m, nb,
+        hipLaunchKernelGGL(reduce_cols_kernel, dim3(gr), dim3(KB), 0, st, m, nbs,
                            (const double *)p2, (const double *)h1, cs, h);
-    hipLaunchKernelGGL(reduce_update_dot_kernel, dim3(nb), dim3(KB), lds, st, m, n, ld, V,
-                       (const double *)p2, (const double *)(sep ? cs : nullptr),
-                       (const double *)h1, h, w, 1, p1);
+    if (once && !sep)
+        once_launch<2>(m, n, ld, V, p2, nbs, none, h1, h, w, p1, nb, st);
+    else
+        hipLaunchKernelGGL(reduce_update_dot_kernel, dim3(nb), dim3(KB), lds, st, m, n, ld, V,
+                           (const double *)p2, cin, (const double *)h1, h, w, 1, p1);
     // h[m] = |w|, and the next basis vector
     hipLaunchKernelGGL(norm_normalize_kernel, dim3(vnext ? gp : 1), dim3(KB), 0, st, n, w, p1, nb,
                        h + m, vnext, vnext2);
@@ -320,8 +484,10 @@ using namespace tct;
 extern "C" int tct_krylov_scratch(int m, int64_t n, int64_t *n_doubles) {
     TCT_CHECK_ARG(m >= 1 && n >= 1 && n_doubles, "krylov_scratch: bad arguments");
     // two partial arrays of m columns per block (one read while the other
-    // is written), plus h1 [m] and the column sums [m]
-    *n_doubles = 2 * (int64_t)n_blocks(n) * m + 2 * m;
+    // is written), plus h1 [m] and the column sums [m], of the larger form.
+    // A basis that grows past 400 columns changes form on the way.
+    const int64_t a = scratch_walk(m, n), b = scratch_once(m < ONCE_MAX_M ? m : ONCE_MAX_M, n);
+    *n_doubles = a > b ? a : b;
     return TCT_OK;
 }
 
@@ -331,11 +497,10 @@ extern "C" int tct_cgs2(int m, int64_t n, int64_t ld, const double *V, double *w
     TCT_CHECK_ARG(m >= 1 && n >= 1 && ld >= n && m < (1 << 20), "cgs2: m %d n %lld ld %lld", m,
                   (long long)n, (long long)ld);
     TCT_CHECK_ARG(V && w && h && scratch, "cgs2: null pointer");
-    const int nb = n_blocks(n);
-    TCT_CHECK_ARG(scratch_doubles >= 2 * (int64_t)nb * m + 2 * m, "cgs2: scratch too small");
+    TCT_CHECK_ARG(scratch_doubles >= scratch_walk(m, n), "cgs2: scratch too small");
     TCT_CHECK_ARG(sizeof(double) * (size_t)m <= 60 * 1024, "cgs2: basis size %d too large for LDS",
                   m);
-    cgs2_launch(m, n, ld, V, w, h, scratch, vnext, vnext2, as_stream(stream));
+    cgs2_launch(m, n, ld, V, w, h, scratch, scratch_doubles, vnext, vnext2, as_stream(stream));
     TCT_CHECK_LAUNCH("cgs2");
     return TCT_OK;
 }
@@ -387,8 +552,7 @@ extern "C" int tct_cgs2_noalloc(int m, int64_t n, int64_t ld, const double *V, d
     TCT_CHECK_ARG(V && w && h, "cgs2_noalloc: null pointer");
     TCT_CHECK_ARG(sizeof(double) * (size_t)m <= 60 * 1024,
                   "cgs2_noalloc: basis size %d too large for LDS", m);
-    const int nb = n_blocks(n);
-    const int64_t need = 2 * (int64_t)nb * m + 2 * m;
+    const int64_t need = scratch_walk(m, n);
     TCT_CHECK_ARG(need <= CGS2_NOALLOC_MAX_DOUBLES,
                   "cgs2_noalloc: m %d, n %lld need %lld doubles of scratch, more than the "
                   "static %lld",
@@ -396,7 +560,8 @@ extern "C" int tct_cgs2_noalloc(int m, int64_t n, int64_t ld, const double *V, d
     double *s = nullptr;
     const int rc = scratch_address(&s);
     if (rc != TCT_OK) return rc;
-    cgs2_launch(m, n, ld, V, w, h, s, vnext, vnext2, as_stream(stream));
+    cgs2_launch(m, n, ld, V, w, h, s, CGS2_NOALLOC_MAX_DOUBLES, vnext, vnext2,
+                as_stream(stream));
     TCT_CHECK_LAUNCH("cgs2_noalloc");
     return TCT_OK;
 }
