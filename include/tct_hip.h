@@ -192,9 +192,10 @@ int tct_far_p2p_batched(int kernel, const double *params_host, int block, int ob
 
 /* ---------------- Triangle-to-triangle farfield ---------------------------
  * farfield_tris_to_tris{K} (tectosaur/matrix_free.cl:19-107) for rules of 3
- * (equal weights) or 4 points, all seven kernels: one lane holds the points
- * of one observation triangle and walks whole source triangles, so what is
- * constant over a flat triangle is formed once (far_tri.h).  A plan holds one
+ * (equal weights) or 4 points (the last three weights equal), all seven
+ * kernels: one lane holds the points of one observation triangle and walks
+ * whole source triangles, so what is constant over a flat triangle is formed
+ * once (far_tri.h).  A plan holds one
  * operator's layout; every pointer is dev memory of the caller.
  *   n_obs, n_obs_pad: observation triangles, padded to a multiple of 64;
  *   n_src, n_tiles:   source triangles, tiles of TCT_TRI_TILE of them;

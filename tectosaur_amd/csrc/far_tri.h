@@ -20,7 +20,7 @@
 //     contraction with the source curl (RH); RT's 1/r term likewise;
 //   * U keeps its two terms in separate sums, scaled once per tile.
 // VALU instructions per point pair with a three-point rule, point form ->
-// this: H 54 -> 39, RH 40 -> 23, T 31 -> 27, A 30 -> 26, RT 27 -> 24,
+// this: H 54 -> 39, RH 40 -> 23, T 31 -> 25, A 30 -> 24, RT 27 -> 23,
 // RA 26 -> 23, U 20 -> 19.
 #pragma once
 #include "far_pair.h"
@@ -29,9 +29,11 @@ namespace tct {
 
 constexpr int TT = TCT_TRI_TILE;   // source triangles per tile (one origin)
 
-// Rules of NQ = 3 points have equal weights.
+// Weights relative to the last one: the rules of three points have equal
+// ones, those of four points (the centre and a ring of three) one that
+// differs, the first.
 template <int NQ>
-constexpr bool equal_w() { return NQ == 3; }
+constexpr bool unit_w(int q) { return NQ == 3 || q > 0; }
 
 // Record of one source triangle: a block of SW words per point, so that a
 // point is read with whole 16-byte vectors, and the words of the triangle in
@@ -71,12 +73,11 @@ constexpr bool tri_obs_normal() { return KID == TCT_A || KID == TCT_H || KID == 
 template <int KID>
 constexpr bool tri_src_normal() { return KID == TCT_T || KID == TCT_H || KID == TCT_RT; }
 
-// Kernel constants, and the rule weights relative to the last one: rw[q] for
-// one rule, ww[p NQ + q] for products.
-template <typename T, int NQ>
+// Kernel constants, and of a four-point rule the first weight relative to the
+// others (rw), its square (rw2) and c0 times it (rwc).
+template <typename T>
 struct TriConst {
-    T c0, c1, c2, c3, c4, eps2;
-    T rw[NQ], ww[NQ * NQ];
+    T c0, c1, c2, c3, c4, eps2, rw, rw2, rwc;
 };
 
 // Words [w, w + SW) of a record (w a multiple of the vector length).
@@ -109,21 +110,47 @@ __device__ __forceinline__ void tri_head(const T *r, TriHead<KID, T> &h) {
         for (int d = 0; d < 3; ++d) h.e[d] = r[tri_e_word(d)];
 }
 
+// Fences keep the scheduler from moving instructions across: NQ: one after
+// each source point; 1: one between the observation points of a source point;
+// 0: none.  They hold few points in registers at a time, and with the order of
+// the terms in tri_pair they decide which instructions can meet in the FP32
+// unit's two-at-once issue (which register numbers may forbid), so only
+// measurement tells.  15,842 triangles, FP32, us, terms in any order and one
+// fence per source point -> the order below and this:
+//   3 points  U 1045 -> 912, T 1337 -> 1213, A 1443 -> 1183, H 1824 -> 1649,
+//             RT 1234 -> 1091, RA 1292 -> 1070, RH 1208 -> 1214
+//   4 points  U 1970 -> 1658, T 2503 -> 2146, A 2602 -> 2025, H 3364 -> 3028,
+//             RT 2383 -> 1927, RA 2345 -> 1879, RH 2201 -> 2017
+// (point form, 3 and 4 points: U 1164 2011, T 1465 2556, A 1377 2458,
+// H 2353 4111, RT 1413 2459, RA 1253 2217, RH 1916 3275).  FP64 issues no pairs
+// and is within 2% either way.
+template <int KID, int NQ, typename T>
+constexpr int tri_fence() {
+    if (sizeof(T) == 8) return NQ;
+    return KID == TCT_U || KID == TCT_A || KID == TCT_RA ? 1 : 0;
+}
+
+// a += f v
+template <typename T>
+__device__ __forceinline__ void add3(T *a, T f, const T *v) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) a[d] = fma_t(f, v[d], a[d]);
+}
+
 // One observation triangle (points x, normal m) against one source triangle
 // (record r, in LDS, its head already in h): acc += its terms, and h becomes
-// the head of the record `next`.  The source points come one after another,
-// fenced from each other, so few of them are in registers at a time; each
-// one's words are read while the point before it computes.  Every fused
+// the head of the record `next`.  The source points come one after another;
+// each one's words are read while the point before it computes.  Every fused
 // multiply-add is written out, as in pair_eval, so every copy of the body
 // performs the same operations.
 template <int KID, int NQ, typename T, bool MASK>
 __device__ __forceinline__ void tri_pair(const T (&x)[NQ][3], const T (&m)[3], const T *r,
-                                         const T *next, const TriConst<T, NQ> &k,
+                                         const T *next, const TriConst<T> &k,
                                          TriHead<KID, T> &h, T *acc) {
 #pragma clang fp contract(off)
-    constexpr bool EQ = equal_w<NQ>();
     constexpr int SW = tri_sw<KID>();
-    T an[NQ], nt[NQ], s0 = T(0), s2[6], G[9];
+    constexpr int F = tri_fence<KID, NQ, T>();
+    T an[NQ], ca[NQ], nt[NQ], s0 = T(0), s2[6], G[9];
     const T n[3] = {h.n[0], h.n[1], h.n[2]}, e[3] = {h.e[0], h.e[1], h.e[2]};
     T mn0 = T(0), mn1 = T(0);
     if constexpr (KID == TCT_H) {
@@ -146,7 +173,9 @@ __device__ __forceinline__ void tri_pair(const T (&x)[NQ][3], const T (&m)[3], c
         }
         const T *s = q + 3;
         // the same for every observation point: m . D, m . s and products
-        T bm = T(0), sm = T(0), sm4 = T(0), e1b = T(0), b4 = T(0), si = T(0);
+        T bm = T(0), cb = T(0), sm = T(0), sm4 = T(0), e1b = T(0), b4 = T(0), si = T(0);
+        T ce = T(0), ej[3] = {T(0), T(0), T(0)};
+        const bool uj = unit_w<NQ>(j);
         if constexpr (tri_obs_normal<KID>())
             bm = dot3(m[0], m[1], m[2], q[0] - x[0][0], q[1] - x[0][1], q[2] - x[0][2]);
         if constexpr (KID == TCT_H || KID == TCT_A)
@@ -157,17 +186,32 @@ __device__ __forceinline__ void tri_pair(const T (&x)[NQ][3], const T (&m)[3], c
             e1b = q[7] * bm;
             b4 = k.c4 * bm;
         }
+        if constexpr (KID == TCT_A) {
+            sm = k.c0 * sm;
+            cb = k.c0 * bm;
+        }
+        if constexpr (KID == TCT_T) ce = k.c0 * q[6];
+        if constexpr (KID == TCT_RT)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) ej[d] = (uj ? k.c0 : k.rwc) * e[d];
 #pragma unroll
         for (int p = 0; p < NQ; ++p) {
             const T D[3] = {q[0] - x[p][0], q[1] - x[p][1], q[2] - x[p][2]};
+            if constexpr (F == 1)
+                if (p > 0) __builtin_amdgcn_sched_barrier(0);
             const T r2 = dot3(D[0], D[1], D[2], D[0], D[1], D[2]);
             const T invr = MASK ? rsq_masked(r2, k.eps2) : rsq_plain(r2);
             const T w = invr * invr;
             // n . D, the same for every source point
             if constexpr (tri_src_normal<KID>())
-                if (j == 0) an[p] = dot3(n[0], n[1], n[2], D[0], D[1], D[2]);
+                if (j == 0) {
+                    an[p] = dot3(n[0], n[1], n[2], D[0], D[1], D[2]);
+                    // in units of the constant its products carry
+                    if constexpr (KID == TCT_T) ca[p] = -k.c0 * an[p];
+                }
             if constexpr (KID == TCT_RH) {
-                const T iw = EQ ? invr : invr * k.ww[p * NQ + j];
+                const bool up = unit_w<NQ>(p);
+                const T iw = up && uj ? invr : invr * (up || uj ? k.rw : k.rw2);
                 const T i3 = iw * w;
                 const T e0 = i3 * D[0], e1 = i3 * D[1], e2 = i3 * D[2];
                 if (p == 0 && j == 0) {
@@ -191,81 +235,51 @@ __device__ __forceinline__ void tri_pair(const T (&x)[NQ][3], const T (&m)[3], c
             }
             const T i3 = invr * w;
             if constexpr (KID == TCT_U) {
-                const T b = i3 * dot3(D[0], D[1], D[2], s[0], s[1], s[2]);
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    acc[6 * p + d] = fma_t(invr, s[d], acc[6 * p + d]);
-                    acc[6 * p + 3 + d] = fma_t(b, D[d], acc[6 * p + 3 + d]);
-                }
+                add3(acc + 6 * p, invr, s);
+                add3(acc + 6 * p + 3, i3 * dot3(D[0], D[1], D[2], s[0], s[1], s[2]), D);
             } else if constexpr (KID == TCT_T) {
                 const T ds = dot3(D[0], D[1], D[2], s[0], s[1], s[2]);
-                const T al = k.c0 * i3;
-                const T be = -al * an[p];
-                const T g = ((i3 * w) * an[p]) * ds;
-                const T de = fma_t(al, q[6], -g);
-                nt[p] = j == 0 ? al * ds : fma_t(al, ds, nt[p]);
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    acc[3 * p + d] = fma_t(be, s[d], acc[3 * p + d]);
-                    acc[3 * p + d] = fma_t(de, D[d], acc[3 * p + d]);
-                }
+                nt[p] = j == 0 ? i3 * ds : fma_t(i3, ds, nt[p]);
+                const T be = i3 * ca[p];
+                if (NQ == 4) add3(acc + 3 * p, be, s);
+                add3(acc + 3 * p, i3 * fma_t(-(w * an[p]), ds, ce), D);
+                if (NQ == 3) add3(acc + 3 * p, be, s);
             } else if constexpr (KID == TCT_A) {
+                add3(acc + 4 * p, i3 * cb, s);
                 const T ds = dot3(D[0], D[1], D[2], s[0], s[1], s[2]);
-                const T al = k.c0 * i3;
-                const T be = al * bm;
-                const T de = fma_t(al, sm, ((i3 * w) * bm) * ds);
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    acc[4 * p + d] = fma_t(be, s[d], acc[4 * p + d]);
-                    acc[4 * p + d] = fma_t(de, D[d], acc[4 * p + d]);
-                }
                 acc[4 * p + 3] = fma_t(i3, ds, acc[4 * p + 3]);
+                add3(acc + 4 * p, i3 * fma_t(w * bm, ds, sm), D);
             } else if constexpr (KID == TCT_H) {
                 const T c = dot3(s[0], s[1], s[2], D[0], D[1], D[2]);
-                const T wa = w * an[p];
                 const T wbc = (w * bm) * c;
-                acc[5 * p + 3] = fma_t(i3, q[6], acc[5 * p + 3]);
-                acc[5 * p + 4] = fma_t(i3, wa * c, acc[5 * p + 4]);
                 const T ni = fma_t(k.c1, wbc, sm);
                 nt[p] = j == 0 ? i3 * ni : fma_t(i3, ni, nt[p]);
+                const T wa = w * an[p];
+                acc[5 * p + 3] = fma_t(i3, q[6], acc[5 * p + 3]);
+                acc[5 * p + 4] = fma_t(i3, wa * c, acc[5 * p + 4]);
                 const T inner = fma_t(T(-15), wbc, sm4);
-                const T DT = (i3 * w) * fma_t(an[p], inner, fma_t(c, mn1, e1b));
-                const T ST = i3 * fma_t(wa, b4, mn0);
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    acc[5 * p + d] = fma_t(D[d], DT, acc[5 * p + d]);
-                    acc[5 * p + d] = fma_t(s[d], ST, acc[5 * p + d]);
-                }
+                add3(acc + 5 * p, (i3 * w) * fma_t(an[p], inner, fma_t(c, mn1, e1b)), D);
+                add3(acc + 5 * p, i3 * fma_t(wa, b4, mn0), s);
             } else if constexpr (KID == TCT_RT) {
-                const T iw = EQ ? invr : invr * k.rw[j];
-                const T iw3 = EQ ? i3 : iw * w;
-                const T cd = (k.c0 * iw3) * dot3(D[0], D[1], D[2], e[0], e[1], e[2]);
-                const T cs = i3 * an[p];
+                const T iw = uj ? invr : invr * k.rw;
                 nt[p] = j == 0 ? iw : nt[p] + iw;
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    acc[3 * p + d] = fma_t(cd, D[d], acc[3 * p + d]);
-                    acc[3 * p + d] = fma_t(cs, s[d], acc[3 * p + d]);
-                }
+                add3(acc + 3 * p, i3 * an[p], s);
+                add3(acc + 3 * p, i3 * dot3(D[0], D[1], D[2], ej[0], ej[1], ej[2]), D);
             } else {
                 // RA: acc = [sum w_p s/r (3), sum w_p (D.s) D/r^3 (3),
                 // per point sum (m.D) s/r^3 (3 NQ)]
-                const T iw = EQ ? invr : invr * k.rw[p];
-                const T iw3 = EQ ? i3 : iw * w;
-                const T cd = iw3 * dot3(D[0], D[1], D[2], s[0], s[1], s[2]);
-                const T cs = i3 * bm;
+                const bool up = unit_w<NQ>(p);
+                const T iw = up ? invr : invr * k.rw;
                 si = p == 0 ? iw : si + iw;
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    acc[3 + d] = fma_t(cd, D[d], acc[3 + d]);
-                    acc[6 + 3 * p + d] = fma_t(cs, s[d], acc[6 + 3 * p + d]);
-                }
+                add3(acc + 6 + 3 * p, i3 * bm, s);
+                add3(acc + 3,
+                     (up ? i3 : i3 * k.rw) * dot3(D[0], D[1], D[2], s[0], s[1], s[2]), D);
             }
         }
         if constexpr (KID == TCT_RA)
 #pragma unroll
             for (int d = 0; d < 3; ++d) acc[d] = fma_t(si, s[d], acc[d]);
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (F == NQ) __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (KID == TCT_RH) {
         // acc[0..9) += s0 G; acc[9..18) += S2 G
@@ -283,17 +297,18 @@ __device__ __forceinline__ void tri_pair(const T (&x)[NQ][3], const T (&m)[3], c
         // the sums along n (T, H) or of 1/r (RT)
         constexpr int A = KID == TCT_H ? 5 : 3;
 #pragma unroll
-        for (int p = 0; p < NQ; ++p)
+        for (int p = 0; p < NQ; ++p) {
+            const T f = KID == TCT_T ? -k.c0 * nt[p] : nt[p];
 #pragma unroll
             for (int d = 0; d < 3; ++d)
-                acc[A * p + d] = fma_t(KID == TCT_T ? -nt[p] : nt[p],
-                                       KID == TCT_RT ? e[d] : n[d], acc[A * p + d]);
+                acc[A * p + d] = fma_t(f, KID == TCT_RT ? e[d] : n[d], acc[A * p + d]);
+        }
     }
 }
 
 // The outputs of a tile's accumulators.
 template <int KID, int NQ, typename T>
-__device__ __forceinline__ void tri_fold(const T (&m)[3], const TriConst<T, NQ> &k, const T *acc,
+__device__ __forceinline__ void tri_fold(const T (&m)[3], const TriConst<T> &k, const T *acc,
                                          T (&o)[tri_out<KID, NQ>()]) {
 #pragma clang fp contract(off)
     if constexpr (KID == TCT_RH) {
@@ -376,7 +391,7 @@ constexpr size_t tri_lds_bytes() {
 // last tile, which holds padding, keeps it).
 template <int KID, int NQ, typename T>
 __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> segs,
-                                                               TriConst<T, NQ> kc) {
+                                                               TriConst<T> kc) {
     constexpr bool F32 = sizeof(T) == 4;
     constexpr int RW = tri_words<KID, NQ>();
     constexpr int NO = tri_out<KID, NQ>();
@@ -411,7 +426,7 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> 
 #pragma unroll
     for (int d = 0; d < 3; ++d)
         m[d] = tri_obs_normal<KID>() ? g.obs[(size_t)(3 * NQ + d) * n_obs_pad + i] : T(0);
-    TriConst<T, NQ> k = kc;
+    TriConst<T> k = kc;
     k.eps2 = F32 ? (T)g.eps2 : T(0);
     if constexpr (F32) {
         // an instruction that reads an SGPR is never dual-issued
@@ -532,16 +547,17 @@ template <int KID, int NQ, typename T>
 inline void far_tri_go(const double *params, const double *qw, const TriSegTable<T> &t,
                        unsigned blocks, hipStream_t st) {
     const KConst<T> kc = kernel_consts<T>(KID, params, 0.0);
-    TriConst<T, NQ> k{kc.c0, kc.c1, kc.c2, kc.c3, kc.c4, T(0), {}, {}};
+    TriConst<T> k{kc.c0, kc.c1, kc.c2, kc.c3, kc.c4, T(0), T(1), T(1), kc.c0};
     if (KID == TCT_RA) {
         const ElasticConsts c = elastic_consts(params);
         k.c0 = (T)c.CsRT1;
         k.c1 = (T)c.CsRT0;
     }
-    for (int p = 0; p < NQ; ++p) {
-        k.rw[p] = (T)(qw[p] / qw[NQ - 1]);
-        for (int j = 0; j < NQ; ++j)
-            k.ww[p * NQ + j] = (T)(qw[p] / qw[NQ - 1] * (qw[j] / qw[NQ - 1]));
+    if (NQ == 4) {
+        const double rw = qw[0] / qw[NQ - 1];
+        k.rw = (T)rw;
+        k.rw2 = (T)(rw * rw);
+        k.rwc = (T)(kc.c0 * rw);
     }
     const unsigned lds = (unsigned)tri_lds_bytes<KID, NQ, T>();
     hipLaunchKernelGGL((far_tri_kernel<KID, NQ, T>), dim3(blocks), dim3(64 * TRI_WAVES), lds, st,

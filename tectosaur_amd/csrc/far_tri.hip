@@ -228,6 +228,8 @@ static int check_plan(const tct_tri_plan *p, const char *what) {
         return set_error(TCT_EUNSUPPORTED, "%s: rule of %d points (3 or 4)", what, p->nq);
     TCT_CHECK_ARG(p->nq != 3 || (p->qw[0] == p->qw[1] && p->qw[1] == p->qw[2]),
                   "%s: a 3-point rule must have equal weights", what);
+    TCT_CHECK_ARG(p->nq != 4 || (p->qw[1] == p->qw[2] && p->qw[2] == p->qw[3]),
+                  "%s: a 4-point rule must have three equal last weights", what);
     TCT_CHECK_ARG(p->qw[p->nq - 1] != 0.0, "%s: the last weight is zero", what);
     TCT_CHECK_ARG(p->n_obs > 0 && p->n_obs_pad >= p->n_obs && p->n_obs_pad % 64 == 0 &&
                       p->n_obs_pad < (1LL << 28),

@@ -19,13 +19,13 @@ TILE = N.TRI_TILE
 LANES = 64
 # points of the rules with a triangle form: a lane keeps every point of its
 # triangle, its accumulators and a source triangle's record in registers,
-# and with seven points they no longer fit
+# and with seven points they no longer fit; the last three weights are equal
 RULE_POINTS = (3, 4)
 
 
 def supports(qw):
     """Whether a triangle rule with weights ``qw`` has a triangle form."""
-    return qw.shape[0] in RULE_POINTS and (qw.shape[0] != 3 or bool(np.all(qw == qw[0])))
+    return qw.shape[0] in RULE_POINTS and bool(np.all(qw[-3:] == qw[-1]))
 
 
 def origin_extent(p, counts):
@@ -46,11 +46,13 @@ def source_chunks(obs_blocks, n_tiles, resident):
     32,256 triangles: 7.97 ms in one round, 7.41 in four, 7.18 in sixteen),
     but at least two tiles for every wave (RH FP32, 4,982 triangles: 137 us
     with two, 139 with one, 154 with six); where that leaves part of the chip
-    idle, one tile (U FP32, 2,048 triangles: 33 us).  From the sizes and the
-    compiled kernel alone: the chunks set the summation order."""
+    idle, one tile (U FP32, 2,048 triangles: 33 us) and never a second one for
+    some (A FP32, 264 triangles, 17 tiles: 29 us in five chunks, 44 in four).
+    From the sizes and the compiled kernel alone: the chunks set the
+    summation order."""
     c = min(-(-16 * resident // obs_blocks), n_tiles // 8)
     if c * obs_blocks < resident:
-        c = min(-(-resident // obs_blocks), n_tiles // 4)
+        c = min(-(-resident // obs_blocks), -(-n_tiles // 4))
     return max(1, c)
 
 
