@@ -257,6 +257,49 @@ int tct_tri_scatter(const tct_tri_plan *plan, int prec, double *out, void *strea
 int tct_tri_matvec(const tct_tri_plan *plan, int prec, const double *v, double *out,
                    void *stream);
 
+/* ---------------- Triangle-to-point farfield, FP32 ------------------------
+ * farfield_tris_to_pts{K} (tectosaur/interior.py:139-185) for U, T, A and H
+ * and rules of 3, 4 or 7 points: one lane holds an observation point and walks
+ * whole source triangles (far_tri_pts.hip).
+ *   n_pts, n_obs_pad: observation points, padded to a multiple of 64;
+ *   n_src, n_tiles, qw, phi, chunks, flags: as tct_tri_plan;
+ *   eps2, group_extent: as tct_far_p2p, with one origin per source tile only;
+ *   obs_n, obs [3][n_obs_pad], src_org [n_tiles][3],
+ *   rec [n_tiles TCT_TRI_TILE][tct_tri_pts_words(kernel, nq)]: written by
+ *                     tct_tri_pts_pack;
+ *   obs_pt:           caller's point of each packed position;
+ *   src_tri, src_jac: DOF-space triangle and Jacobian of each packed one;
+ *   partial:          [chunks][3][n_obs_pad]. */
+typedef struct {
+    int32_t kernel, nq;
+    double params[2];
+    double qw[7];
+    double phi[21];
+    int64_t n_pts, n_obs_pad, n_src, n_tiles;
+    double eps2, group_extent;
+    int32_t chunks, flags;
+    float *obs_n;
+    double *obs;
+    float *rec;
+    double *src_org;
+    const int32_t *obs_pt, *src_tri;
+    const double *src_jac;
+    double *partial;
+} tct_tri_pts_plan;
+
+/* Words of a source triangle's record (0: no such form), and the N-body's
+ * workgroups that a CU holds at once. */
+int tct_tri_pts_words(int kernel, int nq);
+int tct_tri_pts_resident(int kernel, int nq, int *blocks);
+/* Geometry into the plan's layout: observation points and normals [n_pts][3],
+ * source quadrature points [n_src][nq][3] and unit normals [n_src][3], in
+ * packed order. */
+int tct_tri_pts_pack(const tct_tri_pts_plan *plan, const double *obs_pts, const double *obs_ns,
+                     const double *src_pts, const double *src_ns, void *stream);
+/* out [n_pts][3] (caller's point order) = K v, v 9 doubles a source triangle:
+ * strengths, N-body and chunk sums. */
+int tct_tri_pts_matvec(const tct_tri_pts_plan *plan, const double *v, double *out, void *stream);
+
 /* Sum of the chunk partials: out [n][3] f64 (point order of the packing). */
 int tct_far_reduce_pts(int64_t n, int64_t n_obs_pad, int chunks, const double *partial,
                        double *out, void *stream);

@@ -58,6 +58,19 @@ class TriPlan(ctypes.Structure):
           'obs_jac', 'src_jac', 'obs_curl', 'src_curl')] + [('partial', ctypes.c_void_p * 2)]
 
 
+class TriPtsPlan(ctypes.Structure):
+    """tct_tri_pts_plan: the layout of one triangle-to-point operator."""
+    _fields_ = [('kernel', ctypes.c_int32), ('nq', ctypes.c_int32),
+                ('params', ctypes.c_double * 2), ('qw', ctypes.c_double * 7),
+                ('phi', ctypes.c_double * 21), ('n_pts', ctypes.c_int64),
+                ('n_obs_pad', ctypes.c_int64), ('n_src', ctypes.c_int64),
+                ('n_tiles', ctypes.c_int64), ('eps2', ctypes.c_double),
+                ('group_extent', ctypes.c_double), ('chunks', ctypes.c_int32),
+                ('flags', ctypes.c_int32)] + \
+        [(k, ctypes.c_void_p) for k in ('obs_n', 'obs', 'rec', 'src_org', 'obs_pt', 'src_tri',
+                                        'src_jac', 'partial')]
+
+
 _vp = ctypes.c_void_p
 _i64 = ctypes.c_int64
 _int = ctypes.c_int
@@ -86,6 +99,10 @@ SIGNATURES = {
     'tct_tri_nbody': [_int, _vp, _int, _vp],
     'tct_tri_scatter': [_vp, _int, _vp, _vp],
     'tct_tri_matvec': [_vp, _int, _vp, _vp, _vp],
+    'tct_tri_pts_words': [_int, _int],
+    'tct_tri_pts_resident': [_int, _int, _vp],
+    'tct_tri_pts_pack': [_vp, _vp, _vp, _vp, _vp, _vp],
+    'tct_tri_pts_matvec': [_vp, _vp, _vp, _vp],
     'tct_far_reduce_pts': [_i64, _i64, _int, _vp, _vp, _vp],
     'tct_tree_p2m': [_int, _int, _int, _i64, _i64, _vp, _vp, _vp, _vp, _vp],
     'tct_tree_m2m': [_int, _int, _int, _int, _int, _int, _int, _vp, _vp, _vp],

@@ -15,7 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, 'csrc')
 LIB = os.path.join(HERE, 'libtct_hip.so')
 HIP_SOURCES = ['abi.hip', 'far_p2p.hip', 'far_tri.hip', 'far_tri_f32.hip',
-               'far_tri_f64.hip', 'far_tree.hip', 'far_tree_eval_u.hip',
+               'far_tri_f64.hip', 'far_tri_pts.hip', 'far_tree.hip', 'far_tree_eval_u.hip',
                'far_tree_eval_rt.hip', 'far_tree_eval_ra.hip', 'far_tree_eval_rh.hip', 'pairs.hip',
                'pairs_product.hip',
                'interior.hip', 'near_find.hip', 'krylov.hip', 'sparse.hip', 'calib.hip']

@@ -28,7 +28,7 @@ import numpy as np
 import scipy.sparse
 import torch
 
-from . import _native as N
+from . import _native as N, tri_farfield
 from .farfield import FarfieldEngine, morton_order, prec_of, group_extent
 from .find_near_adj import find_near_pairs, get_tri_centroids_rs
 from .kernels import kernels as KERNELS
@@ -169,31 +169,67 @@ class TriToPtDirectFarfieldOp:
         o_pts = obs_pts[self.po]
         self.device = device if device is not None else N.require_device()
         dev = self.device
-        self.engine = FarfieldEngine(K_name, params, o_pts, obs_ns[self.po], s_pts, s_ns,
-                                     precisions=precisions or (self.prec,), device=dev,
-                                     extents=(group_extent(o_pts), group_extent(s_pts)))
-        i32 = dict(dtype=torch.int32, device=dev)
-        f64 = dict(dtype=torch.float64, device=dev)
-        self.tri_of_pt = torch.as_tensor(np.repeat(s_order, self.nq).astype(np.int32), **i32)
-        self.qphi = torch.as_tensor(np.ascontiguousarray(phi), **f64)
-        self.wj_src = torch.as_tensor(s_wj, **f64)
+        self._engine = None
+        self._points = (params, precisions or (self.prec,), o_pts, obs_ns[self.po], s_pts, s_ns,
+                        s_order, s_wj, phi)
         self.curl_src = None
         if K.surf_curl_src:
             e1 = v[:, 1] - v[:, 0]
             e2 = v[:, 2] - v[:, 0]
             J = np.linalg.norm(np.cross(v[:, 2] - v[:, 0], v[:, 2] - v[:, 1]), axis=1)[:, None]
             c = np.stack([(-e2 + e1) / J, e2 / J, -e1 / J], axis=1).reshape((-1, 9))
-            self.curl_src = torch.as_tensor(np.ascontiguousarray(c), **f64)
-        # point k of the packed observation set is caller point po[k]
-        self.po_dev = torch.as_tensor(self.po, dtype=torch.int64, device=dev)
-        self._packed = torch.empty((self.n_obs, 3), **f64)
+            self.curl_src = torch.as_tensor(np.ascontiguousarray(c), dtype=torch.float64,
+                                            device=dev)
+        # FP32 runs over whole source triangles where that form pays; FP64
+        # and the rest over points
+        self.tri = None
+        if 'f32' in self._points[1] and self._tri_pays(K_name):
+            self.tri = tri_farfield.TriToPtFarfield(K_name, params, o_pts, obs_ns[self.po],
+                                                    self.po, s_pts, s_ns, s_order, jac, self.q,
+                                                    phi, dev)
+        else:
+            self.engine
+
+    def _tri_pays(self, K_name):
+        return tri_farfield.pts_supported(K_name, self.nq)
+
+    @property
+    def engine(self):
+        """The point layout and N-body (built when first used)."""
+        if self._engine is None:
+            params, precisions, o_pts, o_ns, s_pts, s_ns, s_order, s_wj, phi = self._points
+            dev = self.device
+            self._engine = FarfieldEngine(self.K.name, params, o_pts, o_ns, s_pts, s_ns,
+                                          precisions=precisions, device=dev,
+                                          extents=(group_extent(o_pts), group_extent(s_pts)))
+            i32 = dict(dtype=torch.int32, device=dev)
+            f64 = dict(dtype=torch.float64, device=dev)
+            self.tri_of_pt = torch.as_tensor(np.repeat(s_order, self.nq).astype(np.int32), **i32)
+            self.qphi = torch.as_tensor(np.ascontiguousarray(phi), **f64)
+            self.wj_src = torch.as_tensor(s_wj, **f64)
+            # point k of the packed observation set is caller point po[k]
+            self.po_dev = torch.as_tensor(self.po, dtype=torch.int64, device=dev)
+            self._packed = torch.empty((self.n_obs, 3), **f64)
+        return self._engine
 
     @property
     def pair_evals(self):
-        return self.engine.pair_evals
+        return self.n_obs * self.n_src * self.nq
 
     def dot_dev(self, v_dev, out=None, prec=None):
         prec = prec or self.prec
+        if out is None:
+            out = torch.empty(self.n_obs * 3, dtype=torch.float64, device=self.device)
+        rows = out.view(-1, 3)
+        if self.tri is not None and prec == 'f32':
+            if rows.is_contiguous() and rows.dtype == torch.float64 and \
+                    rows.is_cuda and rows.shape[0] >= self.n_obs:
+                self.tri.matvec(v_dev, rows)
+            else:
+                r = self.tri.matvec(v_dev, torch.empty((self.n_obs, 3), dtype=torch.float64,
+                                                       device=self.device))
+                rows.index_copy_(0, torch.arange(self.n_obs, device=self.device), r)
+            return out
         e = self.engine
         if self.curl_src is not None:
             e.gather_curl(v_dev, self.tri_of_pt, self.qphi, self.wj_src, self.curl_src, self.nq,
@@ -202,9 +238,7 @@ class TriToPtDirectFarfieldOp:
             e.gather_tris(v_dev, self.tri_of_pt, self.qphi, self.wj_src, self.nq, prec)
         e.run(prec)
         e.reduce_pts(prec, self._packed)
-        if out is None:
-            out = torch.empty(self.n_obs * 3, dtype=torch.float64, device=self.device)
-        out.view(-1, 3).index_copy_(0, self.po_dev, self._packed)
+        rows.index_copy_(0, self.po_dev, self._packed)
         return out
 
     def dot(self, v):

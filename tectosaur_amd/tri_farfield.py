@@ -183,3 +183,69 @@ def run_batched(tris, prec='f32'):
         N.call('tct_tri_nbody', len(tris), ctypes.addressof(ptrs), TriFarfield.prec_id(prec),
                N.stream_ptr())
     return outs
+
+
+class TriToPtFarfield:
+    """Device layout + launches of one FP32 triangle-to-point operator.
+    ``o_pts``, ``o_ns`` [n, 3] in packing order, ``pt`` the caller's point of
+    each; ``s_pts``, ``s_ns`` [n_src * nq, 3] the sources' rule points, whole
+    triangles together, ``tri`` and ``jac`` [n_src]; ``q`` the rule, ``phi``
+    its basis values [nq, 3]."""
+
+    def __init__(self, K_name, params, o_pts, o_ns, pt, s_pts, s_ns, tri, jac, q, phi, device):
+        kid = KERNELS[K_name].kid
+        nq = q[1].shape[0]
+        if o_pts.shape[0] == 0 or tri.shape[0] == 0:
+            raise N.TctError('empty point set')
+        n_pad = -(-o_pts.shape[0] // LANES) * LANES
+        n_tiles = -(-tri.shape[0] // TILE)
+        self.device = device
+        up = lambda a: N.upload(a, None, device)
+        f64 = dict(dtype=torch.float64, device=device)
+        f32 = dict(dtype=torch.float32, device=device)
+        words = N.lib().tct_tri_pts_words(kid, nq)
+        self.chunks = source_chunks(n_pad // LANES, n_tiles, resident_pts(kid, nq))
+        t = {'obs_n': torch.empty(3 * n_pad, **f32), 'obs': torch.empty(3 * n_pad, **f64),
+             'rec': torch.empty(n_tiles * TILE * words, **f32),
+             'src_org': torch.empty(3 * n_tiles, **f64),
+             'obs_pt': up(np.ascontiguousarray(pt, dtype=np.int32)),
+             'src_tri': up(np.ascontiguousarray(tri, dtype=np.int32)),
+             'src_jac': up(np.ascontiguousarray(jac, dtype=np.float64)),
+             'partial': torch.empty(self.chunks * 3 * n_pad, **f64)}
+        self._t = t
+        # rounding bound of a source point against its tile's origin
+        self.group_extent = origin_extent(s_pts, nq * TILE)
+        p = N.TriPtsPlan(kernel=kid, nq=nq, n_pts=o_pts.shape[0], n_obs_pad=n_pad,
+                         n_src=tri.shape[0], n_tiles=n_tiles, chunks=self.chunks,
+                         eps2=(8.0 * 2.0 ** -24 * self.group_extent) ** 2,
+                         group_extent=self.group_extent)
+        p.params[:] = [float(x) for x in params][:2]
+        p.qw[:nq] = np.asarray(q[1], dtype=np.float64).tolist()
+        p.phi[:3 * nq] = np.asarray(phi, dtype=np.float64).reshape(-1).tolist()
+        for k, v in t.items():
+            setattr(p, k, N.ptr(v))
+        self.plan = p
+        dev = [up(np.ascontiguousarray(a)) for a in (o_pts, o_ns, s_pts, s_ns[::nq])]
+        N.call('tct_tri_pts_pack', ctypes.addressof(p), *[N.ptr(a) for a in dev],
+               N.stream_ptr())
+
+    def matvec(self, v_dev, out_dev):
+        N.call('tct_tri_pts_matvec', ctypes.addressof(self.plan), N.ptr(v_dev), N.ptr(out_dev),
+               N.stream_ptr())
+        return out_dev
+
+
+def resident_pts(kid, nq):
+    """As ``resident_blocks``, of the triangle-to-point N-body."""
+    key = ('pts', kid, nq)
+    if key not in _RESIDENT:
+        b = ctypes.c_int(0)
+        N.call('tct_tri_pts_resident', kid, nq, ctypes.byref(b))
+        _RESIDENT[key] = 256 * max(1, b.value)
+    return _RESIDENT[key]
+
+
+def pts_supported(K_name, nq):
+    """Whether a kernel and a rule of ``nq`` points have the triangle-to-point
+    form."""
+    return N.lib().tct_tri_pts_words(KERNELS[K_name].kid, nq) > 0
