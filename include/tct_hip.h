@@ -259,12 +259,12 @@ int tct_tri_matvec(const tct_tri_plan *plan, int prec, const double *v, double *
 
 /* ---------------- Triangle-to-point farfield, FP32 ------------------------
  * farfield_tris_to_pts{K} (tectosaur/interior.py:139-185) for U, T, A and H
- * and rules of 3, 4 or 7 points: one lane holds an observation point and walks
- * whole source triangles (far_tri_pts.hip).
+ * and rules of 3, 4 or (not H) 7 points: one lane holds an observation point
+ * and walks whole source triangles (far_tri_pts.hip).
  *   n_pts, n_obs_pad: observation points, padded to a multiple of 64;
  *   n_src, n_tiles, qw, phi, chunks, flags: as tct_tri_plan;
- *   eps2, group_extent: as tct_far_p2p, with one origin per source tile only;
- *   obs_n, obs [3][n_obs_pad], src_org [n_tiles][3],
+ *   eps2, group_extent: as tct_far_p2p, one origin per 64 points and tile;
+ *   obs [6][n_obs_pad], obs_org [n_obs_pad / 64][3], src_org [n_tiles][3],
  *   rec [n_tiles TCT_TRI_TILE][tct_tri_pts_words(kernel, nq)]: written by
  *                     tct_tri_pts_pack;
  *   obs_pt:           caller's point of each packed position;
@@ -278,8 +278,8 @@ typedef struct {
     int64_t n_pts, n_obs_pad, n_src, n_tiles;
     double eps2, group_extent;
     int32_t chunks, flags;
-    float *obs_n;
-    double *obs;
+    float *obs;
+    double *obs_org;
     float *rec;
     double *src_org;
     const int32_t *obs_pt, *src_tri;

@@ -67,7 +67,7 @@ class TriPtsPlan(ctypes.Structure):
                 ('n_tiles', ctypes.c_int64), ('eps2', ctypes.c_double),
                 ('group_extent', ctypes.c_double), ('chunks', ctypes.c_int32),
                 ('flags', ctypes.c_int32)] + \
-        [(k, ctypes.c_void_p) for k in ('obs_n', 'obs', 'rec', 'src_org', 'obs_pt', 'src_tri',
+        [(k, ctypes.c_void_p) for k in ('obs', 'obs_org', 'rec', 'src_org', 'obs_pt', 'src_tri',
                                         'src_jac', 'partial')]
 
 

@@ -12,8 +12,8 @@
 // triangle and terms along n are summed as scalars over it.
 // 62,500 points x 2,048 triangles, us, point form (far_p2p.hip, its sums and
 // the permutation of its outputs) -> this:
-//   4 points  U 316 -> 249, T 403 -> 315, A 371 -> 343, H 577 -> 482
-//   7 points  U 496 -> 399, T 627 -> 502, A 604 -> 552, H 966 -> 766
+//   4 points  U 312 -> 255, T 388 -> 322, A 371 -> 332, H 580 -> 457
+//   7 points  U 492 -> 411, T 622 -> 503, A 586 -> 547
 // Two, three and four points a lane (fewer LDS reads a pair) were slower: U
 // 421, 428 and 438, T 518, 557 and 557 with seven rule points.
 #include "far_tri.h"
@@ -124,13 +124,18 @@ constexpr size_t pts_lds_bytes() {
 // A workgroup of four waves holds 64 observation points (one a lane, the same
 // in every wave) and one chunk of the source tiles, as in far_tri_kernel: wave
 // w takes tiles w, w + 4, ... through its own LDS tile, FP32 sums within a
-// tile, FP64 across them, the four waves' sums added in wave order.  The
-// points are FP64 and rounded in each tile's frame.
-// obs_n [3][n_pad], obs [3][n_pad], partial [chunks][3][n_pad].
+// tile, FP64 across them, the four waves' sums added in wave order.  The 64
+// points have one FP64 origin and are moved to a tile's frame as in
+// far_p2p_f32_kernel; with four rule points a tile holds 64 source points, the
+// same as there, and every D is the same bit for bit.  (A point next to the
+// surface has large far-rule terms that the near blocks take off again: what
+// is left of them is D's rounding.)
+// obs [6][n_pad]: local points, normals; obs_org [n_pad / 64][3];
+// partial [chunks][3][n_pad].
 template <int KID, int NS>
 __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
-    int n_pad, int n_tiles, int chunks, const float *__restrict__ obs_n,
-    const double *__restrict__ obs, const float *__restrict__ rec,
+    int n_pad, int n_tiles, int chunks, const float *__restrict__ obs,
+    const double *__restrict__ obs_org, const float *__restrict__ rec,
     const double *__restrict__ src_org, double sep2, TriConst<float> kc,
     double *__restrict__ partial) {
     typedef float vec __attribute__((ext_vector_type(4)));
@@ -146,12 +151,13 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
     const int i = ob * 64 + lane;
     TriConst<float> k = kc;
     asm volatile("" : "+v"(k.c0), "+v"(k.c1), "+v"(k.c2), "+v"(k.c4), "+v"(k.eps2));
-    float m[3];
-    double xo[3];
+    float m[3], xl[3];
+    double oo[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        m[d] = tri_obs_normal<KID>() ? obs_n[(size_t)d * n_pad + i] : 0.0f;
-        xo[d] = obs[(size_t)d * n_pad + i];
+        m[d] = tri_obs_normal<KID>() ? obs[(size_t)(3 + d) * n_pad + i] : 0.0f;
+        xl[d] = obs[(size_t)d * n_pad + i];
+        oo[d] = obs_org[3 * ob + d];
     }
     double *out = lds_raw + (size_t)wave * NO * 64 + lane;
 #pragma unroll
@@ -189,14 +195,13 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
         float x[3], acc[pts_acc<KID>()];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            dd[d] = xo[d] - src_org[3 * t + d];
-            x[d] = (float)dd[d];
+            dd[d] = src_org[3 * t + d] - oo[d];
+            x[d] = xl[d] - (float)dd[d];
         }
-        const bool close =
+        const bool mask =   // the same in every lane
             t == n_tiles - 1 || dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2] <= sep2;
 #pragma unroll
         for (int a = 0; a < pts_acc<KID>(); ++a) acc[a] = 0.0f;
-        const bool mask = __any(close);
         TriHead<KID, float> h;
         tri_head<KID, NS, float>(tw, h);
         if (mask) {
@@ -225,15 +230,24 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
     }
 }
 
-__global__ void pts_pack_obs_kernel(int64_t n, int64_t n_pad, const double *__restrict__ pts,
-                                    const double *__restrict__ ns, float *__restrict__ obs_n,
-                                    double *__restrict__ obs) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_pad) return;
-    const int64_t c = i < n ? i : n - 1;   // padding repeats the last point
+// One wave per 64 points: their origin (the mean) and local points.
+__global__ __launch_bounds__(64) void pts_pack_obs_kernel(
+    int64_t n, int64_t n_pad, const double *__restrict__ pts, const double *__restrict__ ns,
+    float *__restrict__ obs, double *__restrict__ org) {
+    const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x;
+    const bool valid = i < n;
+    double cnt = valid ? 1.0 : 0.0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
     for (int d = 0; d < 3; ++d) {
-        obs[d * n_pad + i] = pts[3 * c + d];
-        obs_n[d * n_pad + i] = (float)ns[3 * c + d];
+        const double p = valid ? pts[3 * i + d] : 0.0;
+        double o = p;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) o += __shfl_xor(o, off, 64);
+        o /= cnt;
+        if (threadIdx.x == 0) org[3 * blockIdx.x + d] = o;
+        obs[d * n_pad + i] = valid ? (float)(p - o) : 0.0f;
+        obs[(3 + d) * n_pad + i] = valid ? (float)ns[3 * i + d] : 0.0f;
     }
 }
 
@@ -343,7 +357,7 @@ static void pts_go(const tct_tri_pts_plan &p, hipStream_t st) {
     const unsigned lds = (unsigned)pts_lds_bytes<KID, NS>();
     hipLaunchKernelGGL((tri_pts_kernel<KID, NS>), dim3((unsigned)(p.n_obs_pad / 64 * p.chunks)),
                        dim3(64 * TRI_WAVES), lds, st, (int)p.n_obs_pad, (int)p.n_tiles, p.chunks,
-                       (const float *)p.obs_n, (const double *)p.obs, (const float *)p.rec,
+                       (const float *)p.obs, (const double *)p.obs_org, (const float *)p.rec,
                        (const double *)p.src_org, sep2, k, p.partial);
 }
 
@@ -362,8 +376,8 @@ static void pts_gather_go(const tct_tri_pts_plan &p, const double *v, hipStream_
 template <int KID, int NS>
 static void pts_pack_go(const tct_tri_pts_plan &p, const double *op, const double *on,
                         const double *sp, const double *sn, hipStream_t st) {
-    hipLaunchKernelGGL(pts_pack_obs_kernel, dim3((unsigned)ceil_div(p.n_obs_pad, (int64_t)256)),
-                       dim3(256), 0, st, p.n_pts, p.n_obs_pad, op, on, p.obs_n, p.obs);
+    hipLaunchKernelGGL(pts_pack_obs_kernel, dim3((unsigned)(p.n_obs_pad / 64)), dim3(64), 0, st,
+                       p.n_pts, p.n_obs_pad, op, on, p.obs, p.obs_org);
     hipLaunchKernelGGL((pts_pack_src_kernel<KID, NS>),
                        dim3((unsigned)ceil_div(3 * p.n_tiles, (int64_t)64)), dim3(64), 0, st,
                        p.n_src, p.n_tiles, sp, sn, p.rec, p.src_org);
@@ -376,12 +390,22 @@ static hipError_t pts_occ(int *blocks) {
         blocks, (const void *)tri_pts_kernel<KID, NS>, 64 * TRI_WAVES, lds);
 }
 
+// H with seven points runs over points (far_p2p.hip): its tiles' origins are
+// not the point form's, and 1/r^3 next to the surface leaves the two roundings
+// of D up to 2e-5 of the result apart, for 770 us in place of 960.
+static bool pts_has(int kernel, int nq) {
+    return kernel >= TCT_U && kernel <= TCT_H &&
+           (nq == 3 || nq == 4 || (nq == 7 && kernel != TCT_H));
+}
+
 static int check_pts(const tct_tri_pts_plan *p, const char *what) {
     TCT_CHECK_ARG(p, "%s: null plan", what);
     TCT_CHECK_ARG(p->kernel >= TCT_U && p->kernel <= TCT_H, "%s: kernel id %d", what, p->kernel);
-    if (p->nq != 3 && p->nq != 4 && p->nq != 7)
-        return set_error(TCT_EUNSUPPORTED, "%s: rule of %d points (3, 4 or 7)", what, p->nq);
+    if (!pts_has(p->kernel, p->nq))
+        return set_error(TCT_EUNSUPPORTED, "%s: rule of %d points (3, 4 or 7; H: 3 or 4)", what,
+                         p->nq);
     TCT_CHECK_ARG(p->n_pts > 0 && p->n_obs_pad % 64 == 0 && p->n_pts <= p->n_obs_pad &&
+                      p->n_pts > p->n_obs_pad - 64 &&
                       p->n_obs_pad < (1LL << 28),
                   "%s: bad sizes n_pts=%lld n_obs_pad=%lld", what, (long long)p->n_pts,
                   (long long)p->n_obs_pad);
@@ -392,7 +416,7 @@ static int check_pts(const tct_tri_pts_plan *p, const char *what) {
     TCT_CHECK_ARG(p->eps2 >= 0.0 && std::isfinite(p->eps2) && !std::isnan(p->group_extent),
                   "%s: eps2 / group_extent", what);
     TCT_CHECK_ARG((p->flags & ~1) == 0, "%s: unknown flags 0x%x", what, (unsigned)p->flags);
-    TCT_CHECK_ARG(p->obs_n && p->obs && p->rec && p->src_org && p->obs_pt && p->src_tri &&
+    TCT_CHECK_ARG(p->obs && p->obs_org && p->rec && p->src_org && p->obs_pt && p->src_tri &&
                       p->src_jac,
                   "%s: null pointer", what);
     return TCT_OK;
@@ -411,7 +435,13 @@ static int check_pts(const tct_tri_pts_plan *p, const char *what) {
     case TCT_U: TCT_PTS_NQ(TCT_U, nq, F) break;   \
     case TCT_T: TCT_PTS_NQ(TCT_T, nq, F) break;   \
     case TCT_A: TCT_PTS_NQ(TCT_A, nq, F) break;   \
-    default: TCT_PTS_NQ(TCT_H, nq, F) break;      \
+    default:                                      \
+        if (nq == 3) {                            \
+            F(TCT_H, 3);                          \
+        } else {                                  \
+            F(TCT_H, 4);                          \
+        }                                         \
+        break;                                    \
     }
 
 }  // namespace tct
@@ -419,7 +449,7 @@ static int check_pts(const tct_tri_pts_plan *p, const char *what) {
 using namespace tct;
 
 extern "C" int tct_tri_pts_words(int kernel, int nq) {
-    if (kernel < TCT_U || kernel > TCT_H || (nq != 3 && nq != 4 && nq != 7)) return 0;
+    if (!pts_has(kernel, nq)) return 0;
     int w = 0;
 #define TCT_W(K, NS) w = tri_words<K, NS>()
     TCT_PTS_SWITCH(kernel, nq, TCT_W)

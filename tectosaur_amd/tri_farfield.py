@@ -205,7 +205,8 @@ class TriToPtFarfield:
         f32 = dict(dtype=torch.float32, device=device)
         words = N.lib().tct_tri_pts_words(kid, nq)
         self.chunks = source_chunks(n_pad // LANES, n_tiles, resident_pts(kid, nq))
-        t = {'obs_n': torch.empty(3 * n_pad, **f32), 'obs': torch.empty(3 * n_pad, **f64),
+        t = {'obs': torch.empty(6 * n_pad, **f32),
+             'obs_org': torch.empty(3 * (n_pad // LANES), **f64),
              'rec': torch.empty(n_tiles * TILE * words, **f32),
              'src_org': torch.empty(3 * n_tiles, **f64),
              'obs_pt': up(np.ascontiguousarray(pt, dtype=np.int32)),
@@ -213,8 +214,8 @@ class TriToPtFarfield:
              'src_jac': up(np.ascontiguousarray(jac, dtype=np.float64)),
              'partial': torch.empty(self.chunks * 3 * n_pad, **f64)}
         self._t = t
-        # rounding bound of a source point against its tile's origin
-        self.group_extent = origin_extent(s_pts, nq * TILE)
+        # rounding bound of one point stored against two different origins
+        self.group_extent = origin_extent(o_pts, LANES) + origin_extent(s_pts, nq * TILE)
         p = N.TriPtsPlan(kernel=kid, nq=nq, n_pts=o_pts.shape[0], n_obs_pad=n_pad,
                          n_src=tri.shape[0], n_tiles=n_tiles, chunks=self.chunks,
                          eps2=(8.0 * 2.0 ** -24 * self.group_extent) ** 2,

@@ -37,7 +37,7 @@ def test_points_match_fp64(K, nq, n_obs, n_src):
     pts, tris, obs, ns, rng = _problem(n_obs, n_src, 10 * n_obs + n_src)
     op = TriToPtDirectFarfieldOp(obs, ns, (pts, tris), K, nq, PARAMS, np.float32,
                                  precisions=('f32', 'f64'))
-    assert op.tri is not None
+    assert (op.tri is None) == (K == 'elasticH3' and nq == 3)
     v = torch.as_tensor(rng.standard_normal(9 * n_src), device='cuda')
     ref = op.dot_dev(v, prec='f64')
     out = op.dot_dev(v)
@@ -83,6 +83,7 @@ def test_forms_without_it_run_over_points():
     pts, tris, obs, ns, rng = _problem(20, 9, 1)
     args = (obs, ns, (pts, tris))
     assert TriToPtDirectFarfieldOp(*args, 'elasticRT3', 2, PARAMS, np.float32).tri is None
+    assert TriToPtDirectFarfieldOp(*args, 'elasticH3', 3, PARAMS, np.float32).tri is None
     assert TriToPtDirectFarfieldOp(*args, 'elasticT3', 4, PARAMS, np.float32).tri is None
     assert TriToPtDirectFarfieldOp(*args, 'elasticT3', 2, PARAMS, np.float64).tri is None
     import ctypes
