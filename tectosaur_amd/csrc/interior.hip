@@ -212,25 +212,35 @@ __global__ __launch_bounds__(256) void interior_corners_kernel(
 }
 
 // y[3 i + d] (+)= sum_{k in row i} sum_j data[k][d][j] x[9 indices[k] + j].
-// One thread per output row (point, component).
+// RL lanes per output row (point, component): lane l takes blocks l, l + RL,
+// ..., whose sums meet in a butterfly.  Most points have no close triangle and
+// those on the surface's trace have dozens, a serial chain of scattered loads
+// when one thread took a row (62,500 rows, 47,492 blocks, at most 56 in a row:
+// 25 us; 4, 8, 16 and 32 lanes 9.6, 9.5, 9.7, 18; 160,000 rows and 246,576 blocks:
+// 50 us; 31, 25, 28, 47).
+constexpr int RL = 8;
 __global__ __launch_bounds__(256) void bsr39_kernel(int64_t n_rows,
                                                     const int32_t *__restrict__ indptr,
                                                     const int32_t *__restrict__ indices,
                                                     const double *__restrict__ data,
                                                     const double *__restrict__ x,
                                                     double *__restrict__ y, int accumulate) {
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= 3 * n_rows) return;
+    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t r = g / RL;
+    if (r >= 3 * n_rows) return;   // a row's lanes leave together
+    const int l = (int)(g % RL);
     const int64_t i = r / 3;
     const int d = (int)(r % 3);
     double s = 0.0;
-    for (int k = indptr[i]; k < indptr[i + 1]; ++k) {
+    for (int k = indptr[i] + l; k < indptr[i + 1]; k += RL) {
         const double *b = data + (size_t)k * 27 + d * 9;
         const double *xv = x + 9 * (size_t)indices[k];
 #pragma unroll
         for (int j = 0; j < 9; ++j) s += b[j] * xv[j];
     }
-    y[r] = accumulate ? y[r] + s : s;
+#pragma unroll
+    for (int off = RL / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (l == 0) y[r] = accumulate ? y[r] + s : s;
 }
 
 __device__ __forceinline__ double dot3(const double *a, const double *b) {
@@ -511,7 +521,7 @@ extern "C" int tct_bsr39_spmv(int64_t n_block_rows, const int32_t *indptr, const
                   (long long)n_block_rows);
     TCT_CHECK_ARG(indptr && x && y && (data || n_block_rows == 0), "bsr39: null pointer");
     if (n_block_rows == 0) return TCT_OK;
-    hipLaunchKernelGGL(bsr39_kernel, dim3((unsigned)ceil_div(3 * n_block_rows, 256)), dim3(256),
+    hipLaunchKernelGGL(bsr39_kernel, dim3((unsigned)ceil_div(3 * RL * n_block_rows, 256)), dim3(256),
                        0, as_stream(stream), n_block_rows, indptr, indices, data, x, y,
                        accumulate);
     TCT_CHECK_LAUNCH("bsr39_spmv");
