@@ -348,6 +348,10 @@ int tct_tree_p2m(int kernel, int prec, int order, int64_t n_src, int64_t n_tiles
  * c_off + 2i and c_off + 2i + 1 (the latter when 2i + 1 < n_child). */
 int tct_tree_m2m(int kernel, int prec, int order, int p_off, int n_par, int c_off, int n_child,
                  const double *node_cr, void *moments, void *stream);
+/* Two upward levels, orders 2-4 (others return TCT_EUNSUPPORTED): parents from
+ * children as tct_tree_m2m, then the level [g_off, g_off + n_g) from them. */
+int tct_tree_m2m_pair(int kernel, int prec, int order, int g_off, int n_g, int p_off, int n_par,
+                      int c_off, int n_child, const double *node_cr, void *moments, void *stream);
 
 /* Evaluation over interaction-list segments: list int32 entries e >= 0
  * (m2p from node e) or e < 0 (p2p with source tile -(e + 1)); seg

@@ -292,6 +292,118 @@ __global__ __launch_bounds__(256) void tree_m2m_kernel(int order, int p_off, int
                      moments);
 }
 
+// Two levels in one launch, for orders P <= 4: a workgroup of 512 forms two
+// parents (of level p_off, from children of level c_off) and from them node i
+// of level g_off.  Latency bounds the upward pass, not its few thousand
+// products: m2m_node's outputs walk nested loops of dependent table reads, and
+// its index arithmetic is as long.  Here every edge child -> parent has its
+// (terms)^2 matrix in LDS, a product of three one-dimensional entries and a
+// power, and an output is an unrolled product with it, all of whose reads are
+// independent.  32,256 triangles, order 3, eight levels: eight launches of
+// 12.1 us -> four of 8.4.
+constexpr int M2M_EDGE = 128;   // threads that form one edge's tables and matrix
+
+// C(a, b) for a, b <= 4
+__device__ __forceinline__ double binom4(int a, int b) {
+    const unsigned row =
+        a == 0 ? 0x1u : (a == 1 ? 0x11u : (a == 2 ? 0x121u : (a == 3 ? 0x1331u : 0x14641u)));
+    return (double)((row >> (4 * b)) & 15u);
+}
+__device__ __forceinline__ double pow4(double x, int n) {
+    double v = 1.0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v = q < n ? v * x : v;
+    return v;
+}
+
+struct M2MEdge {
+    double f[3][25];   // C(a, b) (delta_k / rho_p)^(a - b) at 5 a + b; 0 for b > a
+    double s[5];       // (rho_c / rho_p)^q
+    double delta[3];   // c_child - c_parent
+};
+
+// Thread t of M2M_EDGE.
+__device__ __forceinline__ void m2m_edge(int t, const double *__restrict__ child,
+                                         const double *__restrict__ par, M2MEdge &e) {
+    const int k = t / 32, x = t % 32;
+    const double base = child[k] - (k < 3 ? par[k] : 0.0), r = base / par[3];
+    if (k == 3) {
+        if (x < 5) e.s[x] = pow4(r, x);
+    } else {
+        if (x < 25) e.f[k][x] = binom4(x / 5, x % 5) * pow4(r, x / 5 - x % 5);
+        if (x == 25) e.delta[k] = base;
+    }
+}
+
+template <int KID, typename T, int P>
+__global__ __launch_bounds__(512) void tree_m2m_pair_kernel(
+    int g_off, int p_off, int n_par, int c_off, int n_child, const double *__restrict__ node_cr,
+    T *__restrict__ moments) {
+    constexpr int TT = n_terms(P), M1 = TreeK<KID>::C * TT;
+    __shared__ double mc[4 * M1], mp[2 * M1];
+    __shared__ double mat[4][TT * TT];   // [b][a]
+    __shared__ M2MEdge edge[6];          // four of the children, two of the parents
+    __shared__ int mi[TT];
+    const int tid = threadIdx.x, i = blockIdx.x, par0 = 2 * i;
+    const int np = par0 + 1 < n_par ? 2 : 1;
+    const int nc = min(4, n_child - 2 * par0);   // more than 2 (np - 1)
+    const int e = tid / M2M_EDGE, et = tid % M2M_EDGE;
+    if (tid < TT) {
+        const Mi m = mi_at(tid);
+        mi[tid] = m.a | (m.b << 8) | (m.c << 16);
+    }
+    const double *cr_p = node_cr + 4 * (size_t)(p_off + par0);
+    if (e < nc)
+        m2m_edge(et, node_cr + 4 * (size_t)(c_off + 2 * par0 + e), cr_p + 4 * (e / 2), edge[e]);
+    if (e < np) m2m_edge(et, cr_p + 4 * e, node_cr + 4 * (size_t)(g_off + i), edge[4 + e]);
+    for (int o = tid; o < nc * M1; o += 512)
+        mc[o] = (double)moments[(size_t)(c_off + 2 * par0) * M1 + o];
+    __syncthreads();
+    // the matrices of n edges from e0, and their n nodes m: Psi channels absorb
+    // the shift (they read the unshifted sources)
+    auto prepare = [&](double *m, int n, int e0) {
+        if (e < n) {
+            const M2MEdge &E = edge[e0 + e];
+            for (int x = et; x < TT * TT; x += M2M_EDGE) {
+                const int b = mi[x / TT], a = mi[x % TT];
+                const int b0 = b & 255, b1 = (b >> 8) & 255, b2 = b >> 16;
+                mat[e][x] = E.f[0][5 * (a & 255) + b0] * E.f[1][5 * ((a >> 8) & 255) + b1] *
+                            E.f[2][5 * (a >> 16) + b2] * E.s[b0 + b1 + b2];
+            }
+        }
+        for (int o = tid; o < n * psi_count<KID>() * TT; o += 512) {
+            const int cc = o / (psi_count<KID>() * TT), r = o % (psi_count<KID>() * TT);
+            const int ps = r / TT, bi = r % TT;
+            double add = 0.0;
+            for (int b = 0; b < 3; ++b)
+                add += edge[e0 + cc].delta[b] * m[cc * M1 + psi_source<KID>(ps, b) * TT + bi];
+            m[cc * M1 + psi_channel<KID>(ps) * TT + bi] += add;
+        }
+    };
+    // output r of the parent of n shifted children m (matrices m0..)
+    auto merge = [&](const double *m, int n, int m0, int r) {
+        const int ch = r / TT, a = r % TT;
+        double acc = 0.0;
+        for (int cc = 0; cc < n; ++cc)
+#pragma unroll
+            for (int b = 0; b < TT; ++b)
+                acc = fma(mat[m0 + cc][b * TT + a], m[cc * M1 + ch * TT + b], acc);
+        return (T)acc;
+    };
+    prepare(mc, nc, 0);
+    __syncthreads();
+    for (int o = tid; o < np * M1; o += 512) {
+        const int p = o / M1;
+        const T v = merge(mc + 2 * p * M1, min(2, nc - 2 * p), 2 * p, o % M1);
+        moments[(size_t)(p_off + par0) * M1 + o] = v;
+        mp[o] = (double)v;
+    }
+    __syncthreads();
+    prepare(mp, np, 4);
+    __syncthreads();
+    for (int o = tid; o < M1; o += 512) moments[(size_t)(g_off + i) * M1 + o] = merge(mp, np, 0, o);
+}
+
 // ---------------------------------------------------------------------------
 // One multipole node evaluated at one observation point.  a: derivatives up
 // to order P + 1 at u = (c - x)/rho; Rt = c - x (physical); M: the node's

@@ -103,6 +103,53 @@ extern "C" int tct_tree_m2m(int kernel, int prec, int order, int p_off, int n_pa
     return TCT_OK;
 }
 
+template <int KID, typename T>
+static int m2m_pair(int order, int g_off, int n_g, int p_off, int n_par, int c_off, int n_child,
+                    const double *node_cr, T *moments, hipStream_t st) {
+#define TCT_PAIR(P)                                                                            \
+    hipLaunchKernelGGL((tree_m2m_pair_kernel<KID, T, P>), dim3((unsigned)n_g), dim3(512), 0,   \
+                       st, g_off, p_off, n_par, c_off, n_child, node_cr, moments)
+    switch (order) {
+    case 2: TCT_PAIR(2); break;
+    case 3: TCT_PAIR(3); break;
+    case 4: TCT_PAIR(4); break;
+    default:
+        return set_error(TCT_EUNSUPPORTED, "tree_m2m_pair: order %d not built (2-4)", order);
+    }
+#undef TCT_PAIR
+    return TCT_OK;
+}
+
+extern "C" int tct_tree_m2m_pair(int kernel, int prec, int order, int g_off, int n_g, int p_off,
+                                 int n_par, int c_off, int n_child, const double *node_cr,
+                                 void *moments, void *stream) {
+    TCT_CHECK_ARG(tree_kernel_ok(kernel), "tree_m2m_pair: kernel %d has no treecode form", kernel);
+    TCT_CHECK_ARG(prec == TCT_F32 || prec == TCT_F64, "tree_m2m_pair: precision %d", prec);
+    TCT_CHECK_ARG(n_par > 0 && n_child > 0 && n_child <= 2 * n_par && n_child > 2 * (n_par - 1) &&
+                      n_g > 0 && n_par <= 2 * n_g && n_par > 2 * (n_g - 1) && c_off >= 0 &&
+                      c_off + n_child <= p_off && p_off + n_par <= g_off,
+                  "tree_m2m_pair: bad levels g_off=%d n_g=%d p_off=%d n_par=%d c_off=%d n_child=%d",
+                  g_off, n_g, p_off, n_par, c_off, n_child);
+    TCT_CHECK_ARG(node_cr && moments, "tree_m2m_pair: null pointer");
+    hipStream_t st = as_stream(stream);
+    int rc;
+#define TCT_MP(KID)                                                                             \
+    rc = prec == TCT_F32 ? m2m_pair<KID, float>(order, g_off, n_g, p_off, n_par, c_off,         \
+                                                n_child, node_cr, (float *)moments, st)         \
+                         : m2m_pair<KID, double>(order, g_off, n_g, p_off, n_par, c_off,        \
+                                                 n_child, node_cr, (double *)moments, st)
+    switch (kernel) {
+    case TCT_U: TCT_MP(TCT_U); break;
+    case TCT_RT: TCT_MP(TCT_RT); break;
+    case TCT_RA: TCT_MP(TCT_RA); break;
+    default: TCT_MP(TCT_RH); break;
+    }
+#undef TCT_MP
+    if (rc != TCT_OK) return rc;
+    TCT_CHECK_LAUNCH("tree_m2m_pair");
+    return TCT_OK;
+}
+
 extern "C" int tct_tree_eval(int kernel, int prec, int order, int n_obs_pad, const void *obs,
                              const double *obs_org, const void *rec, const double *src_org,
                              const double *node_cr, const void *moments, int n_seg,

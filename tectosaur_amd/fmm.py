@@ -16,8 +16,8 @@ rest for the GPU (far_tree.h):
     traversal.cpp:124-160); accepted nodes are evaluated from multipoles
     (m2p), the rest refined down to source tiles evaluated directly (p2p);
   * multipoles are Cartesian Taylor moments of 1/r with per-kernel Laplace
-    charges; moments of parents come from children (m2m), one launch per
-    level up to the highest level the lists use.
+    charges; moments of parents come from children (m2m), two levels a launch
+    up to the highest level the lists use.
 
 ``pts_per_cell`` sets the smallest source node evaluated directly: ranges of
 ``max(64, pts_per_cell)`` points rounded up to a power-of-two number of
@@ -233,14 +233,13 @@ class TreeFarfield:
         self.seg = N.upload(seg, None, dev)
         self.seg_off = N.upload(seg_off, None, dev)
         self.chunks = 1  # the reduced output has one chunk
-        # upward pass: one launch per level, only up to the highest level any
-        # list refers to.  Three one-launch forms measured slower at 4k-32k
-        # triangles: the block that finishes a parent's last child going on
-        # to the parent (device-scope fences between levels, 1.4x), one
-        # workgroup forming the small top levels node after node (3x at 4k),
-        # and one workgroup forming them with every node of a level at once
-        # (180 us for the top five levels at 8k against 55 us per level: four
-        # waves cannot hide the translation's LDS and FP64 latency)
+        # upward pass: two levels a launch (one for orders above 4), only up
+        # to the highest level any list refers to.  Forms that put more
+        # levels into one launch measured slower at 4k-32k triangles: the
+        # block that finishes a parent's last child going on to the parent
+        # (device-scope fences between levels, 1.4x), one workgroup forming
+        # the small top levels node after node (3x at 4k), and one workgroup
+        # forming them with every node of a level at once
         used = lst[lst >= 0]
         self.max_level = int(self.tree.level[used].max()) if used.size else 0
         self._moments = {}
@@ -273,11 +272,17 @@ class TreeFarfield:
         rec = e.rec(prec)
         N.call('tct_tree_p2m', e.kid, pid, self.order, e.n_src, self.tree.n_tiles, N.ptr(rec),
                N.ptr(e.src_org), N.ptr(self.node_cr), N.ptr(mom), st)
-        for lvl in range(1, self.max_level + 1):
-            p_off, n_par = self.tree.levels[lvl]
-            c_off, n_child = self.tree.levels[lvl - 1]
-            N.call('tct_tree_m2m', e.kid, pid, self.order, p_off, n_par, c_off, n_child,
-                   N.ptr(self.node_cr), N.ptr(mom), st)
+        lvl = 1
+        while lvl <= self.max_level:
+            par, child = self.tree.levels[lvl], self.tree.levels[lvl - 1]
+            if lvl < self.max_level and 2 <= self.order <= 4:
+                N.call('tct_tree_m2m_pair', e.kid, pid, self.order, *self.tree.levels[lvl + 1],
+                       *par, *child, N.ptr(self.node_cr), N.ptr(mom), st)
+                lvl += 2
+            else:
+                N.call('tct_tree_m2m', e.kid, pid, self.order, *par, *child,
+                       N.ptr(self.node_cr), N.ptr(mom), st)
+                lvl += 1
         obs = e.loc32 if prec == 'f32' else e.obs_soa64
         out = self.partial
         N.call('tct_tree_eval', e.kid, pid, self.order, e.n_obs_pad, N.ptr(obs), N.ptr(e.obs_org),
