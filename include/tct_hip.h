@@ -262,8 +262,8 @@ int tct_tri_matvec(const tct_tri_plan *plan, int prec, const double *v, double *
  * and rules of 3, 4 or (not H) 7 points: one lane holds an observation point
  * and walks whole source triangles (far_tri_pts.hip).
  *   n_pts, n_obs_pad: observation points, padded to a multiple of 64;
- *   n_src, n_tiles, qw, phi, chunks, flags: as tct_tri_plan;
- *   eps2, group_extent: as tct_far_p2p, one origin per 64 points and tile;
+ *   n_src, n_tiles, qw, phi, chunks: as tct_tri_plan;
+ *   eps2:             as tct_far_p2p, one origin per 64 points and tile;
  *   obs [6][n_obs_pad], obs_org [n_obs_pad / 64][3], src_org [n_tiles][3],
  *   rec [n_tiles TCT_TRI_TILE][tct_tri_pts_words(kernel, nq)]: written by
  *                     tct_tri_pts_pack;
@@ -276,8 +276,8 @@ typedef struct {
     double qw[7];
     double phi[21];
     int64_t n_pts, n_obs_pad, n_src, n_tiles;
-    double eps2, group_extent;
-    int32_t chunks, flags;
+    double eps2;
+    int32_t chunks, reserved;
     float *obs;
     double *obs_org;
     float *rec;

@@ -65,8 +65,7 @@ class TriPtsPlan(ctypes.Structure):
                 ('phi', ctypes.c_double * 21), ('n_pts', ctypes.c_int64),
                 ('n_obs_pad', ctypes.c_int64), ('n_src', ctypes.c_int64),
                 ('n_tiles', ctypes.c_int64), ('eps2', ctypes.c_double),
-                ('group_extent', ctypes.c_double), ('chunks', ctypes.c_int32),
-                ('flags', ctypes.c_int32)] + \
+                ('chunks', ctypes.c_int32), ('reserved', ctypes.c_int32)] + \
         [(k, ctypes.c_void_p) for k in ('obs', 'obs_org', 'rec', 'src_org', 'obs_pt', 'src_tri',
                                         'src_jac', 'partial')]
 

@@ -130,6 +130,19 @@ constexpr int tri_fence() {
     return KID == TCT_U || KID == TCT_A || KID == TCT_RA ? 1 : 0;
 }
 
+// Whether every tile runs the body with the r2 test: its two instructions more
+// a pair change which others pair up, for the better with these (147,456
+// triangles, FP32, ms, tiles far from the lane without the test -> all with it):
+//   3 points  T 121.4 -> 95.0, A 103.2 -> 95.2, RT 92.8 -> 88.5
+//   4 points  T 212.9 -> 176, A 201.0 -> 165, RH 171.4 -> 166
+// and for the worse with the others (U 69.3 -> 72.8, RA 83.5 -> 87.9, RH with
+// three points 90.7 -> 99.6, H with four 245.0 -> 253.8) and FP64 (1-2%).
+template <int KID, int NQ, typename T>
+constexpr bool tri_always_masked() {
+    return sizeof(T) == 4 && (KID == TCT_T || KID == TCT_A || (KID == TCT_RT && NQ == 3) ||
+                              (KID == TCT_RH && NQ == 4));
+}
+
 // a += f v
 template <typename T>
 __device__ __forceinline__ void add3(T *a, T f, const T *v) {
@@ -490,7 +503,7 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> 
         tri_head<KID, NQ, T>(tw, h);
         // one triangle per step: two (no register copies between a record's
         // head and the next one's) measured 2-9% slower
-        if (mask) {
+        if (tri_always_masked<KID, NQ, T>() || mask) {
 #pragma unroll 1
             for (int j = 0; j < TT; ++j)
                 tri_pair<KID, NQ, T, true>(x, m, tw + j * RW, tw + min(j + 1, TT - 1) * RW, k, h,

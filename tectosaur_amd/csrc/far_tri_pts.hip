@@ -9,7 +9,9 @@
 // What bounds it: VALU issue, as the triangle-to-triangle N-body of far_tri.h,
 // whose records and tile walk it shares.  A lane holds one observation point
 // and walks whole source triangles: n . D and m . n are formed once per
-// triangle and terms along n are summed as scalars over it.
+// triangle and terms along n are summed as scalars over it.  Every tile runs
+// with the r2 test: a body without it for far tiles was no faster (U 396 us
+// with, 406 without; T 484 and 487; seven points, below).
 // 62,500 points x 2,048 triangles, us, point form (far_p2p.hip, its sums and
 // the permutation of its outputs) -> this:
 //   4 points  U 312 -> 255, T 388 -> 322, A 371 -> 332, H 580 -> 457
@@ -31,7 +33,7 @@ constexpr int pts_acc() { return KID == TCT_U ? 6 : (KID == TCT_A ? 4 : (KID == 
 // in LDS, its head already in h): acc += its terms, h becomes the head of the
 // record `next`.  One fence per source point: without, T with seven rule
 // points takes 520 us in place of 502, U 426 in place of 399.
-template <int KID, int NS, bool MASK>
+template <int KID, int NS>
 __device__ __forceinline__ void pts_pair(const float (&x)[3], const float (&m)[3], const float *r,
                                          const float *next, const TriConst<float> &k,
                                          TriHead<KID, float> &h, float (&acc)[pts_acc<KID>()]) {
@@ -52,7 +54,7 @@ __device__ __forceinline__ void pts_pair(const float (&x)[3], const float (&m)[3
         const T *s = q + 3;
         const T D[3] = {q[0] - x[0], q[1] - x[1], q[2] - x[2]};
         const T r2 = dot3(D[0], D[1], D[2], D[0], D[1], D[2]);
-        const T invr = MASK ? rsq_masked(r2, k.eps2) : rsq_plain(r2);
+        const T invr = rsq_masked(r2, k.eps2);
         const T w = invr * invr;
         const T i3 = invr * w;
         if constexpr (tri_src_normal<KID>())
@@ -136,7 +138,7 @@ template <int KID, int NS>
 __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
     int n_pad, int n_tiles, int chunks, const float *__restrict__ obs,
     const double *__restrict__ obs_org, const float *__restrict__ rec,
-    const double *__restrict__ src_org, double sep2, TriConst<float> kc,
+    const double *__restrict__ src_org, TriConst<float> kc,
     double *__restrict__ partial) {
     typedef float vec __attribute__((ext_vector_type(4)));
     constexpr int RW = tri_words<KID, NS>(), NO = 3;
@@ -191,30 +193,16 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
                 pre[v] = src[e < NVEC ? e : NVEC - 1];
             }
         }
-        double dd[3];
         float x[3], acc[pts_acc<KID>()];
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            dd[d] = src_org[3 * t + d] - oo[d];
-            x[d] = xl[d] - (float)dd[d];
-        }
-        const bool mask =   // the same in every lane
-            t == n_tiles - 1 || dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2] <= sep2;
+        for (int d = 0; d < 3; ++d) x[d] = xl[d] - (float)(src_org[3 * t + d] - oo[d]);
 #pragma unroll
         for (int a = 0; a < pts_acc<KID>(); ++a) acc[a] = 0.0f;
         TriHead<KID, float> h;
         tri_head<KID, NS, float>(tw, h);
-        if (mask) {
 #pragma unroll 1
-            for (int j = 0; j < TT; ++j)
-                pts_pair<KID, NS, true>(x, m, tw + j * RW, tw + min(j + 1, TT - 1) * RW, k, h,
-                                        acc);
-        } else {
-#pragma unroll 1
-            for (int j = 0; j < TT; ++j)
-                pts_pair<KID, NS, false>(x, m, tw + j * RW, tw + min(j + 1, TT - 1) * RW, k, h,
-                                         acc);
-        }
+        for (int j = 0; j < TT; ++j)
+            pts_pair<KID, NS>(x, m, tw + j * RW, tw + min(j + 1, TT - 1) * RW, k, h, acc);
         float o[3];
         pts_fold<KID>(m, k, acc, o);
 #pragma unroll
@@ -347,18 +335,11 @@ template <int KID, int NS>
 static void pts_go(const tct_tri_pts_plan &p, hipStream_t st) {
     const KConst<float> kc = kernel_consts<float>(KID, p.params, 0.0);
     const TriConst<float> k{kc.c0, kc.c1, kc.c2, kc.c3, kc.c4, (float)p.eps2, 1.0f, 1.0f, kc.c0};
-    // beyond sep no pair of a tile can reach r2 <= eps2
-    double sep2 = INFINITY;
-    if (p.eps2 > 0.0 && p.group_extent >= 0.0 && std::isfinite(p.group_extent) &&
-        !(p.flags & 1)) {
-        const double sep = p.group_extent * (1.0 + 1e-3) + 5.0 * std::sqrt(p.eps2);
-        sep2 = sep * sep;
-    }
     const unsigned lds = (unsigned)pts_lds_bytes<KID, NS>();
     hipLaunchKernelGGL((tri_pts_kernel<KID, NS>), dim3((unsigned)(p.n_obs_pad / 64 * p.chunks)),
                        dim3(64 * TRI_WAVES), lds, st, (int)p.n_obs_pad, (int)p.n_tiles, p.chunks,
                        (const float *)p.obs, (const double *)p.obs_org, (const float *)p.rec,
-                       (const double *)p.src_org, sep2, k, p.partial);
+                       (const double *)p.src_org, k, p.partial);
 }
 
 template <int KID, int NS>
@@ -413,9 +394,7 @@ static int check_pts(const tct_tri_pts_plan *p, const char *what) {
                       p->n_src > (p->n_tiles - 1) * TT,
                   "%s: bad sizes n_src=%lld n_tiles=%lld", what, (long long)p->n_src,
                   (long long)p->n_tiles);
-    TCT_CHECK_ARG(p->eps2 >= 0.0 && std::isfinite(p->eps2) && !std::isnan(p->group_extent),
-                  "%s: eps2 / group_extent", what);
-    TCT_CHECK_ARG((p->flags & ~1) == 0, "%s: unknown flags 0x%x", what, (unsigned)p->flags);
+    TCT_CHECK_ARG(p->eps2 >= 0.0 && std::isfinite(p->eps2), "%s: eps2", what);
     TCT_CHECK_ARG(p->obs && p->obs_org && p->rec && p->src_org && p->obs_pt && p->src_tri &&
                       p->src_jac,
                   "%s: null pointer", what);

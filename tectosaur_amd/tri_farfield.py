@@ -218,8 +218,7 @@ class TriToPtFarfield:
         self.group_extent = origin_extent(o_pts, LANES) + origin_extent(s_pts, nq * TILE)
         p = N.TriPtsPlan(kernel=kid, nq=nq, n_pts=o_pts.shape[0], n_obs_pad=n_pad,
                          n_src=tri.shape[0], n_tiles=n_tiles, chunks=self.chunks,
-                         eps2=(8.0 * 2.0 ** -24 * self.group_extent) ** 2,
-                         group_extent=self.group_extent)
+                         eps2=(8.0 * 2.0 ** -24 * self.group_extent) ** 2)
         p.params[:] = [float(x) for x in params][:2]
         p.qw[:nq] = np.asarray(q[1], dtype=np.float64).tolist()
         p.phi[:3 * nq] = np.asarray(phi, dtype=np.float64).reshape(-1).tolist()
