@@ -40,7 +40,7 @@ RH_NEAR_FLOPS_PER_QP = 65
 # runs), read from the profile summary, which records the launch shape and
 # a hash of the kernel sources it was measured on: a figure measured on
 # other sources or another launch shape is not reported.
-TRAFFIC_SOURCE = 'profiles/far_p2p_H_two_surface_442k_pmc_traffic.md'
+TRAFFIC_SOURCE = 'profiles/far_tri_H_two_surface_147k.md'
 TRAFFIC_KERNEL_SOURCES = {
     'far_tri_kernel<H>': ('tectosaur_amd/csrc/far_tri.h', 'tectosaur_amd/csrc/far_pair.h'),
     'bsr9_kernel': ('tectosaur_amd/csrc/sparse.hip',)}

@@ -1,4 +1,5 @@
-"""Launch-shape autotuner for the farfield N-body kernel.
+"""Launch-shape autotuner for the farfield N-body over points (far_p2p.hip);
+the forms over whole triangles choose their source chunks from the sizes.
 
 The tunable shape is ``TileCfg(block, obs_per_lane, src_chunks, flags)``
 with flags 0 or 2 (the XCD chunk order, src_chunks a multiple of 8).  A tuning

@@ -10,7 +10,8 @@
 // ranges, then one pass over the blocks), so results do not depend on
 // timing, and tct_cgs2 uses no library workspace: solves on different
 // streams share nothing (tct_cgs2_noalloc instead uses one static array per
-// device, below).  HBM-bound: each pass reads V[:m] once.
+// device, below).  HBM-bound at large n, latency-bound at small n; bases of up
+// to 400 columns are read once a pass (once_kernel).
 #include <mutex>
 
 #include "tct_common.h"

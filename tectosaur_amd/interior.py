@@ -15,8 +15,10 @@ whatever the argument, :33) and vertex pairs split off by a 1e-9 distance
 test (fast_find_nearfield.cpp:184-215).
 
 On the device:
-  * far(v) is the farfield N-body of far_p2p.hip with the observation points
-    as observers: the gather folds J w phi into per-quadrature-point source
+  * far(v) is, in FP32, an N-body of whole source triangles against the
+    points (far_tri_pts.hip: U, T, A with rules of 3, 4 and 7 points, H with 3
+    and 4), else the farfield N-body of far_p2p.hip with the points as
+    observers: the gather folds J w phi into per-quadrature-point source
     strengths (the surface curls for RT), the kernel sums, and the reduction
     writes one 3-vector per point -- farfield_tris_to_pts{K}
     (tectosaur/matrix_free.cl:109-194) in another order.
@@ -134,7 +136,8 @@ class TriToPtDirectFarfieldOp:
     """out[3i + d] = sum over every source triangle and quadrature point of
     K(y_q - x_i) (J w phi . v), pairs at r2 == 0 skipped: the reference's
     TriToPtDirectFarfieldOp (tectosaur/interior.py:139-185) as gather +
-    N-body + point reduction.  ``dot_dev`` writes a device tensor
+    N-body + point reduction, over whole source triangles (``tri``) or over
+    points (``engine``).  ``dot_dev`` writes a device tensor
     [n_obs * 3] in the caller's point order."""
 
     def __init__(self, obs_pts, obs_ns, src_mesh, K_name, nq, params, float_type,

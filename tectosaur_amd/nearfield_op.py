@@ -13,7 +13,8 @@ Assembly (one-time, per mesh), following nearfield_op.py:95-141:
     covers every pair with that rule, so the difference corrects it);
   * all blocks placed in one 9x9 BSR matrix on the device (the reference
     keeps four BCOO matrices and applies them on the host).
-All integration runs on the device in FP64 (pairs.hip).
+All integration runs on the device in FP64 (pairs.hip, pairs_product.hip),
+sorted pair lists straight into their rows of the matrix.
 """
 import ctypes
 

@@ -3,8 +3,12 @@ drop-in for tectosaur/ops/sparse_farfield_op.py:16-71.
 
 The reference launches one thread per observation triangle that loops over
 every source triangle and every quadrature-point pair
-(farfield_tris_to_tris{K}, tectosaur/matrix_free.cl:19-107).  Here the same
-sum is computed as three device steps per matvec:
+(farfield_tris_to_tris{K}, tectosaur/matrix_free.cl:19-107).  With a rule of
+three or four points the N-body runs over whole triangles (far_tri.h,
+``tri_farfield.TriFarfield``): strengths into the source triangles' records,
+one launch over (observation triangle, source triangle) pairs, and the
+Galerkin scatter.  Other rules, and a caller's launch shape, take the point
+form, the same sum as three device steps per matvec:
 
   1. gather   s_j = J_t w_q sum_b phi_b(q) v[9t+3b+:]  (one value per source
                quadrature point; the factor J_t w_q of matrix_free.cl:83 and
