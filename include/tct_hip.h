@@ -425,10 +425,11 @@ int tct_pairs_product(int kernel, int n_o, const double *qo, const double *wo, i
 
 /* Host: a pair list (int64, width 2 or 5, rows contiguous) into int32 with the
  * ranges checked: triangles in [0, n_tris), clicks in [0, 3), flip 0 or 1;
- * with dofs (int64 [n][2], rows dofs_stride values apart) those into dofs32,
- * in [0, n_rows) and [0, n_cols).  Returns TCT_EARG when a value is out of
- * range; *sorted tells whether the dofs (the pairs without dofs) come in
- * ascending order of (row, column), equal ones allowed. */
+ * with dofs (int64 [n][2], rows dofs_stride values apart) those into dofs32.
+ * The block places -- the dofs, or without dofs the pairs -- must lie in
+ * [0, n_rows) and [0, n_cols).  Returns TCT_EARG when a value is out of
+ * range; *sorted tells whether the places come in ascending order of (row,
+ * column), equal ones allowed. */
 int tct_pairs_pack(int64_t n, int width, const int64_t *pairs, int64_t n_tris,
                    const int64_t *dofs, int64_t dofs_stride, int64_t n_rows, int64_t n_cols,
                    int32_t *pairs32, int32_t *dofs32, int *sorted);
@@ -441,7 +442,8 @@ int tct_pairs_same(int64_t n, int width, const int64_t *pairs, const int64_t *do
  * column), merged: list k has n[k] blocks at dofs[k] (dev, (row, column) at a
  * stride of strides[k] int32).  rank[k][i]: position of its block i in the
  * merged order (earlier lists first where equal); indices: the merged
- * columns; indptr [n_rows + 1]: the row starts. */
+ * columns; indptr [n_rows + 1]: the row starts.  The kernel trusts the places:
+ * the caller has checked them (tct_pairs_pack). */
 int tct_bsr_merge(int n_lists, const int64_t *n, const int32_t *const *dofs, const int *strides,
                   int64_t n_rows, int32_t *const *rank, int32_t *indices, int32_t *indptr,
                   void *stream);

@@ -239,8 +239,8 @@ extern "C" int tct_pairs_pack(int64_t n, int width, const int64_t *pairs, int64_
         o[0] = (int32_t)p[0];
         o[1] = (int32_t)p[1];
         const int64_t *d = dofs ? dofs + i * dofs_stride : p;
+        bad |= d[0] < 0 || d[0] >= n_rows || d[1] < 0 || d[1] >= n_cols;
         if (dofs) {
-            bad |= d[0] < 0 || d[0] >= n_rows || d[1] < 0 || d[1] >= n_cols;
             dofs32[2 * i] = (int32_t)d[0];
             dofs32[2 * i + 1] = (int32_t)d[1];
         }

@@ -121,6 +121,15 @@ def nearfield_plan(pts, tris, obs_subset, src_subset, near_threshold, finder='ho
                 near=(near, near_dofs))
 
 
+def check_places(dofs, shape):
+    """The blocks (dofs [n, 2], n > 0) must lie in a matrix of ``shape``: its
+    product trusts the columns and the rows of blocks."""
+    d = np.asarray(dofs)
+    for k, what in ((0, 'row'), (1, 'column')):
+        if d[:, k].min() < 0 or d[:, k].max() >= shape[k] // 9:
+            raise IndexError('block %s out of range [0, %d)' % (what, shape[k] // 9))
+
+
 class RegularizedNearfieldIntegralOp:
     def __init__(self, pts, tris, obs_subset, src_subset, nq_coincident, nq_edge_adj,
                  nq_vert_adjacent, nq_far, nq_near, near_threshold, K_near_name, K_far_name,
@@ -166,6 +175,7 @@ class RegularizedNearfieldIntegralOp:
             if prs.shape[0] == 0:
                 continue
             check_pairs(prs, tris.shape[0])
+            check_places(dofs, self.shape)
             p_dev = N.upload(prs.astype(np.int32), None, dev)
             acc = pairs_int.pairs_quad_dev(rules[name], p_dev, check0)
             corr = corr_int.pairs_quad_dev(far_q, p_dev[:, :2].contiguous(), corr_check0)
