@@ -262,10 +262,11 @@ int tct_tri_matvec(const tct_tri_plan *plan, int prec, const double *v, double *
  * and rules of 3, 4 or (not H) 7 points: one lane holds an observation point
  * and walks whole source triangles (far_tri_pts.hip).
  *   n_pts, n_obs_pad: observation points, padded to a multiple of 64;
- *   n_src, n_tiles, qw, phi, chunks: as tct_tri_plan;
+ *   n_src, n_tiles:   source triangles, tiles of tct_tri_pts_tile(kernel, nq);
+ *   qw, phi, chunks:  as tct_tri_plan;
  *   eps2:             as tct_far_p2p, one origin per 64 points and tile;
  *   obs [6][n_obs_pad], obs_org [n_obs_pad / 64][3], src_org [n_tiles][3],
- *   rec [n_tiles TCT_TRI_TILE][tct_tri_pts_words(kernel, nq)]: written by
+ *   rec [n_tiles tct_tri_pts_tile][tct_tri_pts_words(kernel, nq)]: written by
  *                     tct_tri_pts_pack;
  *   obs_pt:           caller's point of each packed position;
  *   src_tri, src_jac: DOF-space triangle and Jacobian of each packed one;
@@ -287,9 +288,10 @@ typedef struct {
     double *partial;
 } tct_tri_pts_plan;
 
-/* Words of a source triangle's record (0: no such form), and the N-body's
- * workgroups that a CU holds at once. */
+/* Words of a source triangle's record and triangles of a tile (0: no such
+ * form), and the N-body's workgroups that a CU holds at once. */
 int tct_tri_pts_words(int kernel, int nq);
+int tct_tri_pts_tile(int kernel, int nq);
 int tct_tri_pts_resident(int kernel, int nq, int *blocks);
 /* Geometry into the plan's layout: observation points and normals [n_pts][3],
  * source quadrature points [n_src][nq][3] and unit normals [n_src][3], in

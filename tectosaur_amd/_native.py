@@ -99,6 +99,7 @@ SIGNATURES = {
     'tct_tri_scatter': [_vp, _int, _vp, _vp],
     'tct_tri_matvec': [_vp, _int, _vp, _vp, _vp],
     'tct_tri_pts_words': [_int, _int],
+    'tct_tri_pts_tile': [_int, _int],
     'tct_tri_pts_resident': [_int, _int, _vp],
     'tct_tri_pts_pack': [_vp, _vp, _vp, _vp, _vp, _vp],
     'tct_tri_pts_matvec': [_vp, _vp, _vp, _vp],

@@ -26,6 +26,13 @@ struct PtsRule {
     double qw[7], phi[21];
 };
 
+// Source triangles per tile: as many whole ones as have at most 64 points, up
+// to TCT_TRI_TILE.  A tile has one origin and one FP32 sum, so its size sets the
+// rounding of the points and of the sums; 64 points is the point form's.  (Tiles
+// of 16 triangles with seven points, 112: at points next to a fault of 2,048
+// triangles T's and A's median error grew 1.2 to 1.3 times.)
+constexpr int pts_tile(int nq) { return nq == 7 ? 9 : TT; }
+
 template <int KID>
 constexpr int pts_acc() { return KID == TCT_U ? 6 : (KID == TCT_A ? 4 : (KID == TCT_H ? 5 : 3)); }
 
@@ -120,7 +127,8 @@ __device__ __forceinline__ void pts_fold(const float (&m)[3], const TriConst<flo
 
 template <int KID, int NS>
 constexpr size_t pts_lds_bytes() {
-    return TRI_WAVES * (sizeof(double) * 64 * 3 + sizeof(float) * TT * tri_words<KID, NS>());
+    return TRI_WAVES *
+           (sizeof(double) * 64 * 3 + sizeof(float) * pts_tile(NS) * tri_words<KID, NS>());
 }
 
 // A workgroup of four waves holds 64 observation points (one a lane, the same
@@ -129,7 +137,8 @@ constexpr size_t pts_lds_bytes() {
 // tile, FP64 across them, the four waves' sums added in wave order.  The 64
 // points have one FP64 origin and are moved to a tile's frame as in
 // far_p2p_f32_kernel; with four rule points a tile holds 64 source points, the
-// same as there, and every D is the same bit for bit.  (A point next to the
+// same as there, and every D is the same bit for bit, with three and seven its
+// frame is a little smaller (48 and 63 points).  (A point next to the
 // surface has large far-rule terms that the near blocks take off again: what
 // is left of them is D's rounding.)
 // obs [6][n_pad]: local points, normals; obs_org [n_pad / 64][3];
@@ -141,8 +150,10 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
     const double *__restrict__ src_org, TriConst<float> kc,
     double *__restrict__ partial) {
     typedef float vec __attribute__((ext_vector_type(4)));
+    constexpr int TP = pts_tile(NS);
     constexpr int RW = tri_words<KID, NS>(), NO = 3;
-    constexpr int NVEC = TT * RW / 4, NV = (NVEC + 63) / 64;
+    constexpr int NVEC = TP * RW / 4, NV = (NVEC + 63) / 64;
+    static_assert(TP * RW % 4 == 0 && TP * NS <= 64, "whole vectors, at most 64 points");
     extern __shared__ double lds_raw[];
     const int obs_blocks = n_pad / 64;
     const int ob = (int)blockIdx.x % obs_blocks, ch = (int)blockIdx.x / obs_blocks;
@@ -169,7 +180,7 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
     vec pre[NV];
     {
         const int tf = t0 + wave < t1 ? t0 + wave : t0;      // a chunk holds a tile
-        const vec *src = (const vec *)(rec + (size_t)tf * TT * RW);
+        const vec *src = (const vec *)(rec + (size_t)tf * TP * RW);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const int e = v * 64 + lane;
@@ -186,7 +197,7 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
         }
         {
             const int tn = t + TRI_WAVES < t1 ? t + TRI_WAVES : t;
-            const vec *src = (const vec *)(rec + (size_t)tn * TT * RW);
+            const vec *src = (const vec *)(rec + (size_t)tn * TP * RW);
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
                 const int e = v * 64 + lane;
@@ -201,8 +212,8 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
         TriHead<KID, float> h;
         tri_head<KID, NS, float>(tw, h);
 #pragma unroll 1
-        for (int j = 0; j < TT; ++j)
-            pts_pair<KID, NS>(x, m, tw + j * RW, tw + min(j + 1, TT - 1) * RW, k, h, acc);
+        for (int j = 0; j < TP; ++j)
+            pts_pair<KID, NS>(x, m, tw + j * RW, tw + min(j + 1, TP - 1) * RW, k, h, acc);
         float o[3];
         pts_fold<KID>(m, k, acc, o);
 #pragma unroll
@@ -245,18 +256,19 @@ template <int KID, int NS>
 __global__ void pts_pack_src_kernel(int64_t n, int64_t n_tiles, const double *__restrict__ pts,
                                     const double *__restrict__ ns, float *__restrict__ rec,
                                     double *__restrict__ org) {
+    constexpr int TP = pts_tile(NS);
     constexpr int RW = tri_words<KID, NS>(), SW = tri_sw<KID>();
     const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= n_tiles * 3) return;
     const int64_t t = g / 3;
     const int d = (int)(g % 3);
-    const int64_t k0 = t * TT;
-    const int cnt = (int)(n - k0 < TT ? n - k0 : TT);
+    const int64_t k0 = t * TP;
+    const int cnt = (int)(n - k0 < TP ? n - k0 : TP);
     double o = 0.0;
     for (int e = 0; e < cnt * NS; ++e) o += pts[(k0 * NS + e) * 3 + d];
     o /= cnt * NS;
     org[3 * t + d] = o;
-    for (int u = 0; u < TT; ++u) {
+    for (int u = 0; u < TP; ++u) {
         float *r = rec + (k0 + u) * RW;
         for (int w = d; w < RW; w += 3) {
             // strengths are zero until a gather writes them
@@ -390,8 +402,9 @@ static int check_pts(const tct_tri_pts_plan *p, const char *what) {
                       p->n_obs_pad < (1LL << 28),
                   "%s: bad sizes n_pts=%lld n_obs_pad=%lld", what, (long long)p->n_pts,
                   (long long)p->n_obs_pad);
-    TCT_CHECK_ARG(p->n_src > 0 && p->n_tiles < (1LL << 24) && p->n_src <= p->n_tiles * TT &&
-                      p->n_src > (p->n_tiles - 1) * TT,
+    const int64_t tile = pts_tile(p->nq);
+    TCT_CHECK_ARG(p->n_src > 0 && p->n_tiles < (1LL << 24) && p->n_src <= p->n_tiles * tile &&
+                      p->n_src > (p->n_tiles - 1) * tile,
                   "%s: bad sizes n_src=%lld n_tiles=%lld", what, (long long)p->n_src,
                   (long long)p->n_tiles);
     TCT_CHECK_ARG(p->eps2 >= 0.0 && std::isfinite(p->eps2), "%s: eps2", what);
@@ -434,6 +447,10 @@ extern "C" int tct_tri_pts_words(int kernel, int nq) {
     TCT_PTS_SWITCH(kernel, nq, TCT_W)
 #undef TCT_W
     return w;
+}
+
+extern "C" int tct_tri_pts_tile(int kernel, int nq) {
+    return pts_has(kernel, nq) ? pts_tile(nq) : 0;
 }
 
 extern "C" int tct_tri_pts_resident(int kernel, int nq, int *blocks) {

@@ -198,7 +198,8 @@ class TriToPtFarfield:
         if o_pts.shape[0] == 0 or tri.shape[0] == 0:
             raise N.TctError('empty point set')
         n_pad = -(-o_pts.shape[0] // LANES) * LANES
-        n_tiles = -(-tri.shape[0] // TILE)
+        tile = N.lib().tct_tri_pts_tile(kid, nq)
+        n_tiles = -(-tri.shape[0] // tile)
         self.device = device
         up = lambda a: N.upload(a, None, device)
         f64 = dict(dtype=torch.float64, device=device)
@@ -207,7 +208,7 @@ class TriToPtFarfield:
         self.chunks = source_chunks(n_pad // LANES, n_tiles, resident_pts(kid, nq))
         t = {'obs': torch.empty(6 * n_pad, **f32),
              'obs_org': torch.empty(3 * (n_pad // LANES), **f64),
-             'rec': torch.empty(n_tiles * TILE * words, **f32),
+             'rec': torch.empty(n_tiles * tile * words, **f32),
              'src_org': torch.empty(3 * n_tiles, **f64),
              'obs_pt': up(np.ascontiguousarray(pt, dtype=np.int32)),
              'src_tri': up(np.ascontiguousarray(tri, dtype=np.int32)),
@@ -215,7 +216,7 @@ class TriToPtFarfield:
              'partial': torch.empty(self.chunks * 3 * n_pad, **f64)}
         self._t = t
         # rounding bound of one point stored against two different origins
-        self.group_extent = origin_extent(o_pts, LANES) + origin_extent(s_pts, nq * TILE)
+        self.group_extent = origin_extent(o_pts, LANES) + origin_extent(s_pts, nq * tile)
         p = N.TriPtsPlan(kernel=kid, nq=nq, n_pts=o_pts.shape[0], n_obs_pad=n_pad,
                          n_src=tri.shape[0], n_tiles=n_tiles, chunks=self.chunks,
                          eps2=(8.0 * 2.0 ** -24 * self.group_extent) ** 2)
