@@ -371,7 +371,7 @@ struct TriSeg {
     double *partial;         // [chunks][tri_out][n_obs_pad]
     double sep2;
     float eps2;
-    int n_obs_pad, n_tiles, chunks, blk0;
+    int n_obs_pad, n_src, n_tiles, chunks, blk0;
 };
 constexpr int TRI_SEG_MAX = 16;
 template <typename T>
@@ -381,6 +381,24 @@ struct TriSegTable {
 };
 
 constexpr int TRI_WAVES = 4;   // waves of a workgroup, one source tile each at a time
+
+// What a wave takes of its workgroup's chunk of source tiles [t0, t1): tiles
+// t0 + wave, t0 + wave + 4, ...; of a chunk of one or two tiles, where that
+// would leave waves without work, the tile's triangles in four or two parts.
+// The real triangles only: a tile's padding is never walked.  (Few sources
+// against many observers, FP64, four points, 59,700 x 9 triangles: one wave of
+// four walking 16 triangles took 110 us for H and 52 for T, this 38 and 26, the
+// point form 55 and 42.)
+struct TriShare {
+    int first, step, part, parts;
+    // triangles [j0, j1) of a tile with n real ones
+    __device__ __forceinline__ int j0(int n) const { return n * part / parts; }
+    __device__ __forceinline__ int j1(int n) const { return n * (part + 1) / parts; }
+};
+__device__ __forceinline__ TriShare tri_share(int wave, int t0, int t1) {
+    const int n = t1 - t0, parts = n == 1 ? TRI_WAVES : (n == 2 ? TRI_WAVES / 2 : 1);
+    return {t0 + wave / parts, TRI_WAVES / parts, wave % parts, parts};
+}
 
 // Bytes of LDS: every wave's sums and its current source tile.
 template <int KID, int NQ, typename T>
@@ -400,8 +418,7 @@ constexpr size_t tri_lds_bytes() {
 // FP32: points are stored relative to an FP64 origin, one per observation
 // triangle and one per source tile; a tile's sums are FP32, the sums over
 // tiles FP64.  Tiles whose origin is farther than sqrt(sep2) from every
-// lane's origin hold no pair with r2 <= eps2 and run without the test (the
-// last tile, which holds padding, keeps it).
+// lane's origin hold no pair with r2 <= eps2 and run without the test.
 template <int KID, int NQ, typename T>
 __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> segs,
                                                                TriConst<T> kc) {
@@ -418,7 +435,7 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> 
     int si = 0;
     while (si + 1 < segs.n && L >= segs.s[si + 1].blk0) ++si;
     const TriSeg<T> &g = segs.s[si];
-    const int n_obs_pad = g.n_obs_pad, n_tiles = g.n_tiles, chunks = g.chunks;
+    const int n_obs_pad = g.n_obs_pad, n_src = g.n_src, n_tiles = g.n_tiles, chunks = g.chunks;
     const int obs_blocks = n_obs_pad / 64;
     const int l = L - g.blk0;
     const int ob = l % obs_blocks, ch = l / obs_blocks;
@@ -456,8 +473,9 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> 
     vec *tile = (vec *)(lds_raw + TRI_WAVES * NO * 64) + wave * NVEC;
     const T *tw = (const T *)tile;
     vec pre[NV];
-    const int tf = t0 + wave < t1 ? t0 + wave : t0;      // a chunk holds a tile
+    const TriShare sh = tri_share(wave, t0, t1);
     {
+        const int tf = sh.first < t1 ? sh.first : t0;      // a chunk holds a tile
         const vec *src = (const vec *)(g.rec + (size_t)tf * TT * RW);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
@@ -465,7 +483,9 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> 
             pre[v] = src[e < NVEC ? e : NVEC - 1];
         }
     }
-    for (int t = t0 + wave; t < t1; t += TRI_WAVES) {
+    for (int t = sh.first; t < t1; t += sh.step) {
+        const int real = min(TT, n_src - t * TT), j0 = sh.j0(real), j1 = sh.j1(real);
+        if (j0 == j1) break;   // fewer triangles than parts: nothing for this wave
         // the previous tile's LDS reads were issued before these writes, and
         // a wave's LDS operations complete in order
 #pragma unroll
@@ -474,7 +494,7 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> 
             if (e < NVEC) tile[e] = pre[v];
         }
         {
-            const int tn = t + TRI_WAVES < t1 ? t + TRI_WAVES : t;
+            const int tn = t + sh.step < t1 ? t + sh.step : t;
             const vec *src = (const vec *)(g.rec + (size_t)tn * TT * RW);
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
@@ -490,8 +510,7 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> 
 #pragma unroll
         for (int d = 0; d < 3; ++d)
             dd[d] = g.src_org[3 * t + d] - g.obs_org[(size_t)d * n_obs_pad + ii];
-        const bool close =
-            t == n_tiles - 1 || dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2] <= g.sep2;
+        const bool close = dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2] <= g.sep2;
         if constexpr (F32)
 #pragma unroll
             for (int p = 0; p < NQ; ++p)
@@ -500,19 +519,22 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> 
                     x[p][d] = g.obs[(size_t)(3 * p + d) * n_obs_pad + ii] - (T)dd[d];
         const bool mask = __any(close);
         TriHead<KID, T> h;
-        tri_head<KID, NQ, T>(tw, h);
+        tri_head<KID, NQ, T>(tw + j0 * RW, h);
         // one triangle per step: two (no register copies between a record's
         // head and the next one's) measured 2-9% slower
+        int j = j0;
         if (tri_always_masked<KID, NQ, T>() || mask) {
 #pragma unroll 1
-            for (int j = 0; j < TT; ++j)
+            do
                 tri_pair<KID, NQ, T, true>(x, m, tw + j * RW, tw + min(j + 1, TT - 1) * RW, k, h,
                                            acc);
+            while (++j < j1);
         } else {
 #pragma unroll 1
-            for (int j = 0; j < TT; ++j)
+            do
                 tri_pair<KID, NQ, T, false>(x, m, tw + j * RW, tw + min(j + 1, TT - 1) * RW, k,
                                             h, acc);
+            while (++j < j1);
         }
         if constexpr (F32) {
             T o[NO];

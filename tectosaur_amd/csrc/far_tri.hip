@@ -291,6 +291,7 @@ static void set_seg(TriSeg<T> &g, const tct_tri_plan &p, int blk0) {
     g.sep2 = F32 && p.kernel == TCT_H && p.nq == 3 ? INFINITY : plan_sep2(p);
     g.eps2 = (float)p.eps2;
     g.n_obs_pad = (int)p.n_obs_pad;
+    g.n_src = (int)p.n_src;
     g.n_tiles = (int)p.n_tiles;
     g.chunks = p.chunks[F32 ? TCT_F32 : TCT_F64];
     g.blk0 = blk0;

@@ -145,7 +145,7 @@ constexpr size_t pts_lds_bytes() {
 // partial [chunks][3][n_pad].
 template <int KID, int NS>
 __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
-    int n_pad, int n_tiles, int chunks, const float *__restrict__ obs,
+    int n_pad, int n_src, int n_tiles, int chunks, const float *__restrict__ obs,
     const double *__restrict__ obs_org, const float *__restrict__ rec,
     const double *__restrict__ src_org, TriConst<float> kc,
     double *__restrict__ partial) {
@@ -178,8 +178,9 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
     vec *tile = (vec *)(lds_raw + TRI_WAVES * NO * 64) + wave * NVEC;
     const float *tw = (const float *)tile;
     vec pre[NV];
+    const TriShare sh = tri_share(wave, t0, t1);
     {
-        const int tf = t0 + wave < t1 ? t0 + wave : t0;      // a chunk holds a tile
+        const int tf = sh.first < t1 ? sh.first : t0;      // a chunk holds a tile
         const vec *src = (const vec *)(rec + (size_t)tf * TP * RW);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
@@ -187,7 +188,9 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
             pre[v] = src[e < NVEC ? e : NVEC - 1];
         }
     }
-    for (int t = t0 + wave; t < t1; t += TRI_WAVES) {
+    for (int t = sh.first; t < t1; t += sh.step) {
+        const int real = min(TP, n_src - t * TP), j0 = sh.j0(real), j1 = sh.j1(real);
+        if (j0 == j1) break;   // fewer triangles than parts: nothing for this wave
         // the previous tile's LDS reads were issued before these writes, and
         // a wave's LDS operations complete in order
 #pragma unroll
@@ -196,7 +199,7 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
             if (e < NVEC) tile[e] = pre[v];
         }
         {
-            const int tn = t + TRI_WAVES < t1 ? t + TRI_WAVES : t;
+            const int tn = t + sh.step < t1 ? t + sh.step : t;
             const vec *src = (const vec *)(rec + (size_t)tn * TP * RW);
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
@@ -210,10 +213,12 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
 #pragma unroll
         for (int a = 0; a < pts_acc<KID>(); ++a) acc[a] = 0.0f;
         TriHead<KID, float> h;
-        tri_head<KID, NS, float>(tw, h);
+        tri_head<KID, NS, float>(tw + j0 * RW, h);
+        int j = j0;
 #pragma unroll 1
-        for (int j = 0; j < TP; ++j)
+        do
             pts_pair<KID, NS>(x, m, tw + j * RW, tw + min(j + 1, TP - 1) * RW, k, h, acc);
+        while (++j < j1);
         float o[3];
         pts_fold<KID>(m, k, acc, o);
 #pragma unroll
@@ -349,8 +354,8 @@ static void pts_go(const tct_tri_pts_plan &p, hipStream_t st) {
     const TriConst<float> k{kc.c0, kc.c1, kc.c2, kc.c3, kc.c4, (float)p.eps2, 1.0f, 1.0f, kc.c0};
     const unsigned lds = (unsigned)pts_lds_bytes<KID, NS>();
     hipLaunchKernelGGL((tri_pts_kernel<KID, NS>), dim3((unsigned)(p.n_obs_pad / 64 * p.chunks)),
-                       dim3(64 * TRI_WAVES), lds, st, (int)p.n_obs_pad, (int)p.n_tiles, p.chunks,
-                       (const float *)p.obs, (const double *)p.obs_org, (const float *)p.rec,
+                       dim3(64 * TRI_WAVES), lds, st, (int)p.n_obs_pad, (int)p.n_src, (int)p.n_tiles,
+                       p.chunks, (const float *)p.obs, (const double *)p.obs_org, (const float *)p.rec,
                        (const double *)p.src_org, k, p.partial);
 }
 
