@@ -382,6 +382,19 @@ struct TriSegTable {
 
 constexpr int TRI_WAVES = 4;   // waves of a workgroup, one source tile each at a time
 
+// Chunk ch of a problem's n_tiles source tiles: tiles [t0, t1).  Chunks are made
+// of whole groups of four tiles, one for each wave, where there are groups for
+// all of them, else of pairs or single tiles.
+struct TriChunk {
+    int t0, t1;
+};
+__device__ __forceinline__ TriChunk tri_chunk(int n_tiles, int chunks, int ch) {
+    const int unit = chunks <= (n_tiles + 3) / 4 ? 4 : (chunks <= (n_tiles + 1) / 2 ? 2 : 1);
+    const int64_t units = (n_tiles + unit - 1) / unit;
+    return {unit * (int)(units * ch / chunks),
+            min(n_tiles, unit * (int)(units * (ch + 1) / chunks))};
+}
+
 // What a wave takes of its workgroup's chunk of source tiles [t0, t1): tiles
 // t0 + wave, t0 + wave + 4, ...; of a chunk of one or two tiles, where that
 // would leave waves without work, the tile's triangles in four or two parts.
@@ -441,8 +454,8 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> 
     const int ob = l % obs_blocks, ch = l / obs_blocks;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int lane = (int)threadIdx.x & 63;
-    const int t0 = (int)((int64_t)n_tiles * ch / chunks);
-    const int t1 = (int)((int64_t)n_tiles * (ch + 1) / chunks);
+    const TriChunk tc = tri_chunk(n_tiles, chunks, ch);
+    const int t0 = tc.t0, t1 = tc.t1;
     const int i = ob * 64 + lane;
 
     // FP32 reads its points again for every tile (coalesced, and in cache by

@@ -159,8 +159,8 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
     const int ob = (int)blockIdx.x % obs_blocks, ch = (int)blockIdx.x / obs_blocks;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int lane = (int)threadIdx.x & 63;
-    const int t0 = (int)((int64_t)n_tiles * ch / chunks);
-    const int t1 = (int)((int64_t)n_tiles * (ch + 1) / chunks);
+    const TriChunk tc = tri_chunk(n_tiles, chunks, ch);
+    const int t0 = tc.t0, t1 = tc.t1;
     const int i = ob * 64 + lane;
     TriConst<float> k = kc;
     asm volatile("" : "+v"(k.c0), "+v"(k.c1), "+v"(k.c2), "+v"(k.c4), "+v"(k.eps2));

@@ -41,19 +41,22 @@ def origin_extent(p, counts):
 
 def source_chunks(obs_blocks, n_tiles, resident):
     """Source chunks of a launch of obs_blocks x chunks workgroups, of which
-    the chip holds ``resident`` at once, four waves each.  Sixteen rounds of
-    workgroups, whose loads and sums then overlap others' arithmetic (H FP32,
-    32,256 triangles: 7.97 ms in one round, 7.41 in four, 7.18 in sixteen),
-    but at least two tiles for every wave (RH FP32, 4,982 triangles: 137 us
-    with two, 139 with one, 154 with six); where that leaves part of the chip
-    idle, one tile (U FP32, 2,048 triangles: 33 us) and never a second one for
-    some (A FP32, 264 triangles, 17 tiles: 29 us in five chunks, 44 in four).
-    From the sizes and the compiled kernel alone: the chunks set the
+    the chip holds ``resident`` at once, four waves each.  A chunk lasts as long
+    as its busiest wave, so every wave takes the same number k of tiles and the
+    chunks are groups of 4 k (far_tri.h): k = 1 while that makes at most
+    sixteen rounds of workgroups (of 512 at least), whose loads and sums overlap
+    others' arithmetic (H FP32, 32,256 triangles: 7.97 ms in one round, 7.41 in
+    four, 7.18 in sixteen) and 512 chunks; more where there are more, as every
+    chunk has its sums to write and an observation block adds the sums of its
+    chunks one after another (FP64 H, four points, 100 x 59,700 triangles: 311
+    us with 933 chunks, 262 with 467).  us, chunks of equal size -> this: FP64 H,
+    four points, 1,240 triangles 111 -> 64 (90 over points), 2,640 236 -> 200;
+    FP64 T, four points, 1,900 116 -> 86; RH 1,564 63 -> 47; A FP32, 2,640
+    64 -> 52.  From the sizes and the compiled kernel alone: the chunks set the
     summation order."""
-    c = min(-(-16 * resident // obs_blocks), n_tiles // 8)
-    if c * obs_blocks < resident:
-        c = min(-(-resident // obs_blocks), -(-n_tiles // 4))
-    return max(1, c)
+    groups = -(-n_tiles // 4)
+    k = max(-(-obs_blocks * groups // (16 * max(resident, 512))), -(-groups // 512))
+    return -(-groups // k)
 
 
 _RESIDENT = {}
