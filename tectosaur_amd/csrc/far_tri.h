@@ -127,7 +127,7 @@ __device__ __forceinline__ void tri_head(const T *r, TriHead<KID, T> &h) {
 template <int KID, int NQ, typename T>
 constexpr int tri_fence() {
     if (sizeof(T) == 8) return NQ;
-    return KID == TCT_U || KID == TCT_A || KID == TCT_RA ? 1 : 0;
+    return KID == TCT_U || KID == TCT_A || KID == TCT_RA || (KID == TCT_H && NQ == 3) ? 1 : 0;
 }
 
 // Whether every tile runs the body with the r2 test: its two instructions more
@@ -136,7 +136,8 @@ constexpr int tri_fence() {
 //   3 points  T 121.4 -> 95.0, A 103.2 -> 95.2, RT 92.8 -> 88.5
 //   4 points  T 212.9 -> 176, A 201.0 -> 165, RH 171.4 -> 166
 // and for the worse with the others (U 69.3 -> 72.8, RA 83.5 -> 87.9, RH with
-// three points 90.7 -> 99.6, H with four 245.0 -> 253.8) and FP64 (1-2%).
+// three points 90.7 -> 99.6, H with three 132.5 -> 150, with four 245.0 ->
+// 253.8) and FP64 (1-2%).
 template <int KID, int NQ, typename T>
 constexpr bool tri_always_masked() {
     return sizeof(T) == 4 && (KID == TCT_T || KID == TCT_A || (KID == TCT_RT && NQ == 3) ||
@@ -262,7 +263,21 @@ __device__ __forceinline__ void tri_pair(const T (&x)[NQ][3], const T (&m)[3], c
                 const T ds = dot3(D[0], D[1], D[2], s[0], s[1], s[2]);
                 acc[4 * p + 3] = fma_t(i3, ds, acc[4 * p + 3]);
                 add3(acc + 4 * p, i3 * fma_t(w * bm, ds, sm), D);
+            } else if constexpr (KID == TCT_H && NQ == 3) {
+                const T wa = w * an[p];
+                add3(acc + 5 * p, i3 * fma_t(wa, b4, mn0), s);
+                acc[5 * p + 3] = fma_t(i3, q[6], acc[5 * p + 3]);
+                const T c = dot3(s[0], s[1], s[2], D[0], D[1], D[2]);
+                acc[5 * p + 4] = fma_t(i3, wa * c, acc[5 * p + 4]);
+                const T wbc = (w * bm) * c;
+                const T ni = fma_t(k.c1, wbc, sm);
+                nt[p] = j == 0 ? i3 * ni : fma_t(i3, ni, nt[p]);
+                const T inner = fma_t(T(-15), wbc, sm4);
+                add3(acc + 5 * p, (i3 * w) * fma_t(an[p], inner, fma_t(c, mn1, e1b)), D);
             } else if constexpr (KID == TCT_H) {
+                // the same in the order that is the faster one with four
+                // points (32,256 triangles: 11.85 ms, 13.2 in the order above;
+                // with three points the other way round, 6.84 and 6.58)
                 const T c = dot3(s[0], s[1], s[2], D[0], D[1], D[2]);
                 const T wbc = (w * bm) * c;
                 const T ni = fma_t(k.c1, wbc, sm);

@@ -285,10 +285,7 @@ static void set_seg(TriSeg<T> &g, const tct_tri_plan &p, int blk0) {
     g.obs_org = p.obs_org;
     g.src_org = p.src_org;
     g.partial = p.partial[F32 ? TCT_F32 : TCT_F64];
-    // H with three points in FP32: the body with the test is the faster one for
-    // far tiles too (136.1 ms in place of 141.7 at 147,456 triangles), but only
-    // as the compiler lays it out next to the other (149.4 ms alone)
-    g.sep2 = F32 && p.kernel == TCT_H && p.nq == 3 ? INFINITY : plan_sep2(p);
+    g.sep2 = plan_sep2(p);
     g.eps2 = (float)p.eps2;
     g.n_obs_pad = (int)p.n_obs_pad;
     g.n_src = (int)p.n_src;
