@@ -206,7 +206,7 @@ int tct_far_p2p_batched(int kernel, const double *params_host, int block, int ob
  *                     precision: partial[prec] is [chunks][out][n_obs_pad],
  *                     out = 3 nq (U, T, A, H, RT), 9 (RH) or 3 + 3 nq (RA);
  *   flags:            bit 0 keeps the r2 test on every tile;
- *   obs32/64 [3 nq + 3][n_obs_pad], obs_org [3][n_obs_pad],
+ *   obs [3 nq + 3][n_obs_pad], obs_org [3][n_obs_pad],
  *   rec32/64 [n_tiles TCT_TRI_TILE][words], src_org [n_tiles][3]: written by
  *                     tct_tri_pack (words = tct_tri_words(kernel, nq));
  *   obs_tri, src_tri: DOF-space triangle of each packed position;
@@ -224,8 +224,7 @@ typedef struct {
     double eps2, group_extent;
     int32_t chunks[2];
     int32_t flags, reserved;
-    float *obs32;
-    double *obs64;
+    double *obs;
     double *obs_org;
     float *rec32;
     double *rec64;

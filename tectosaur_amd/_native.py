@@ -54,7 +54,7 @@ class TriPlan(ctypes.Structure):
                 ('group_extent', ctypes.c_double), ('chunks', ctypes.c_int32 * 2),
                 ('flags', ctypes.c_int32), ('reserved', ctypes.c_int32)] + \
         [(k, ctypes.c_void_p) for k in
-         ('obs32', 'obs64', 'obs_org', 'rec32', 'rec64', 'src_org', 'obs_tri', 'src_tri',
+         ('obs', 'obs_org', 'rec32', 'rec64', 'src_org', 'obs_tri', 'src_tri',
           'obs_jac', 'src_jac', 'obs_curl', 'src_curl')] + [('partial', ctypes.c_void_p * 2)]
 
 

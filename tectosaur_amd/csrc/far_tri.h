@@ -379,7 +379,7 @@ __device__ __forceinline__ void tri_fold(const T (&m)[3], const TriConst<T> &k, 
 // blk0), observation block fastest, then chunk).
 template <typename T>
 struct TriSeg {
-    const T *obs;            // [3 NQ + 3][n_obs_pad]: points (FP32: local), normal
+    const double *obs;       // [3 NQ + 3][n_obs_pad]: points, normal
     const double *obs_org;   // [3][n_obs_pad]
     const T *rec;            // [n_tiles * TT][tri_words]
     const double *src_org;   // [n_tiles][3]
@@ -443,9 +443,8 @@ constexpr size_t tri_lds_bytes() {
 // in wave order through LDS, so a chunk has one partial sum whatever its
 // number of waves: a quarter of the partial sums that one wave per chunk
 // would write and the scatter would read.
-// FP32: points are stored relative to an FP64 origin, one per observation
-// triangle and one per source tile; a tile's sums are FP32, the sums over
-// tiles FP64.  Tiles whose origin is farther than sqrt(sep2) from every
+// FP32: points are relative to the source tile's FP64 origin; a tile's sums are
+// FP32, the sums over tiles FP64.  Tiles whose origin is farther than sqrt(sep2) from every
 // lane's origin hold no pair with r2 <= eps2 and run without the test.
 template <int KID, int NQ, typename T>
 __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> segs,
@@ -474,7 +473,14 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> 
     const int i = ob * 64 + lane;
 
     // FP32 reads its points again for every tile (coalesced, and in cache by
-    // then), so they hold registers only in the tile's frame
+    // then) and moves them to the tile's frame in FP64: one rounding, the same
+    // as that of a source point there, so D of a pair and of the pair the other
+    // way round are opposite numbers, as in the point form.  (Points stored in
+    // FP32 against an origin of their triangle were rounded twice more: eight
+    // meshes of 3,000 to 10,000 triangles, relative L2 error over the point
+    // form's, three points T 0.85, A 0.87, H 0.85, RH 1.01, RA 1.16, four points
+    // T 1.13, A 1.22; this 0.68, 0.68, 0.67, 0.90, 1.03, 1.04 and 1.06, and the
+    // same time.)
     T x[NQ][3], m[3];
     if constexpr (!F32)
 #pragma unroll
@@ -483,7 +489,7 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> 
             for (int d = 0; d < 3; ++d) x[p][d] = g.obs[(size_t)(3 * p + d) * n_obs_pad + i];
 #pragma unroll
     for (int d = 0; d < 3; ++d)
-        m[d] = tri_obs_normal<KID>() ? g.obs[(size_t)(3 * NQ + d) * n_obs_pad + i] : T(0);
+        m[d] = tri_obs_normal<KID>() ? (T)g.obs[(size_t)(3 * NQ + d) * n_obs_pad + i] : T(0);
     TriConst<T> k = kc;
     k.eps2 = F32 ? (T)g.eps2 : T(0);
     if constexpr (F32) {
@@ -534,17 +540,19 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> 
         // these loads out of the loop and hold their registers through it
         int ii = i;
         asm volatile("" : "+v"(ii));
-        double dd[3];
+        double org[3], dd[3];
 #pragma unroll
-        for (int d = 0; d < 3; ++d)
-            dd[d] = g.src_org[3 * t + d] - g.obs_org[(size_t)d * n_obs_pad + ii];
+        for (int d = 0; d < 3; ++d) {
+            org[d] = g.src_org[3 * t + d];
+            dd[d] = org[d] - g.obs_org[(size_t)d * n_obs_pad + ii];
+        }
         const bool close = dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2] <= g.sep2;
         if constexpr (F32)
 #pragma unroll
             for (int p = 0; p < NQ; ++p)
 #pragma unroll
                 for (int d = 0; d < 3; ++d)
-                    x[p][d] = g.obs[(size_t)(3 * p + d) * n_obs_pad + ii] - (T)dd[d];
+                    x[p][d] = (T)(g.obs[(size_t)(3 * p + d) * n_obs_pad + ii] - org[d]);
         const bool mask = __any(close);
         TriHead<KID, T> h;
         tri_head<KID, NQ, T>(tw + j0 * RW, h);

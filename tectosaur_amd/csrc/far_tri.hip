@@ -11,11 +11,11 @@ struct TriRule {
     double qw[4], phi[12];
 };
 
-// One thread per observation triangle: origin, local and absolute points.
+// One thread per observation triangle: points, normal and origin.
 template <int NQ>
 __global__ void tri_pack_obs_kernel(int64_t n, int64_t n_pad, const double *__restrict__ pts,
-                                    const double *__restrict__ ns, float *__restrict__ o32,
-                                    double *__restrict__ o64, double *__restrict__ org) {
+                                    const double *__restrict__ ns, double *__restrict__ obs,
+                                    double *__restrict__ org) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_pad) return;
     const bool valid = i < n;
@@ -26,13 +26,8 @@ __global__ void tri_pack_obs_kernel(int64_t n, int64_t n_pad, const double *__re
             o += p[q] / NQ;
         }
         org[d * n_pad + i] = o;
-        for (int q = 0; q < NQ; ++q) {
-            o32[(size_t)(3 * q + d) * n_pad + i] = (float)(p[q] - o);
-            o64[(size_t)(3 * q + d) * n_pad + i] = p[q];
-        }
-        const double nn = valid ? ns[3 * i + d] : 0.0;
-        o32[(size_t)(3 * NQ + d) * n_pad + i] = (float)nn;
-        o64[(size_t)(3 * NQ + d) * n_pad + i] = nn;
+        for (int q = 0; q < NQ; ++q) obs[(size_t)(3 * q + d) * n_pad + i] = p[q];
+        obs[(size_t)(3 * NQ + d) * n_pad + i] = valid ? ns[3 * i + d] : 0.0;
     }
 }
 
@@ -242,7 +237,7 @@ static int check_plan(const tct_tri_plan *p, const char *what) {
     TCT_CHECK_ARG(p->eps2 >= 0.0 && std::isfinite(p->eps2) && !std::isnan(p->group_extent),
                   "%s: eps2 / group_extent", what);
     TCT_CHECK_ARG((p->flags & ~1) == 0, "%s: unknown flags 0x%x", what, (unsigned)p->flags);
-    TCT_CHECK_ARG(p->obs32 && p->obs64 && p->obs_org && p->rec32 && p->rec64 && p->src_org &&
+    TCT_CHECK_ARG(p->obs && p->obs_org && p->rec32 && p->rec64 && p->src_org &&
                       p->obs_tri && p->src_tri && p->obs_jac && p->src_jac,
                   "%s: null pointer", what);
     const bool so = p->kernel == TCT_RA || p->kernel == TCT_RH;
@@ -276,12 +271,11 @@ template <typename T>
 static void set_seg(TriSeg<T> &g, const tct_tri_plan &p, int blk0) {
     constexpr bool F32 = sizeof(T) == 4;
     if constexpr (F32) {
-        g.obs = p.obs32;
         g.rec = p.rec32;
     } else {
-        g.obs = p.obs64;
         g.rec = p.rec64;
     }
+    g.obs = p.obs;
     g.obs_org = p.obs_org;
     g.src_org = p.src_org;
     g.partial = p.partial[F32 ? TCT_F32 : TCT_F64];
@@ -388,7 +382,7 @@ extern "C" int tct_tri_pack(const tct_tri_plan *p, const double *obs_pts, const 
     const unsigned nb = (unsigned)ceil_div(p->n_obs_pad, (int64_t)256);
 #define TCT_PACK(K, NQ)                                                                         \
     hipLaunchKernelGGL((tri_pack_obs_kernel<NQ>), dim3(nb), dim3(256), 0, st, p->n_obs,         \
-                       p->n_obs_pad, obs_pts, obs_ns, p->obs32, p->obs64, p->obs_org);          \
+                       p->n_obs_pad, obs_pts, obs_ns, p->obs, p->obs_org);                      \
     hipLaunchKernelGGL((tri_pack_src_kernel<K, NQ>), dim3((unsigned)p->n_tiles), dim3(64), 0,   \
                        st, p->n_src, src_pts, src_ns, p->rec32, p->rec64, p->src_org)
     if (p->nq == 3) {

@@ -99,8 +99,7 @@ class TriFarfield:
         obs_of = np.empty(self.n_obs, dtype=np.int32)   # packed position -> triangle
         obs_of[plan['pt_of_tri']] = np.arange(self.n_obs, dtype=np.int32)
         jac = lambda wj: np.ascontiguousarray(wj[nq - 1::nq]) / qw[nq - 1]
-        t = {'obs32': torch.empty((3 * nq + 3) * n_pad, **f32),
-             'obs64': torch.empty((3 * nq + 3) * n_pad, **f64),
+        t = {'obs': torch.empty((3 * nq + 3) * n_pad, **f64),
              'obs_org': torch.empty(3 * n_pad, **f64),
              'rec32': torch.empty(n_tiles * TILE * words, **f32),
              'rec64': torch.empty(n_tiles * TILE * words, **f64),
