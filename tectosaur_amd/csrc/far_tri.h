@@ -558,23 +558,41 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> 
         tri_head<KID, NQ, T>(tw + j0 * RW, h);
         // one triangle per step: two (no register copies between a record's
         // head and the next one's) measured 2-9% slower
+        // RA in FP32: the sums that its observation points share, folded after
+        // each triangle pair: through a whole tile they would be 48 and 144
+        // terms long with three points, where the point form adds 64 (median
+        // error 1.33 times its, 1.00 with this; 32,256 triangles 4.12 -> 4.26 ms)
+        T ra[3] = {T(0), T(0), T(0)};
+        auto fold_ra = [&]() {
+            if constexpr (F32 && KID == TCT_RA)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    ra[d] = ra[d] + fma_t(k.c0, acc[d], k.c1 * acc[3 + d]);
+                    acc[d] = acc[3 + d] = T(0);
+                }
+        };
         int j = j0;
         if (tri_always_masked<KID, NQ, T>() || mask) {
 #pragma unroll 1
-            do
+            do {
                 tri_pair<KID, NQ, T, true>(x, m, tw + j * RW, tw + min(j + 1, TT - 1) * RW, k, h,
                                            acc);
-            while (++j < j1);
+                fold_ra();
+            } while (++j < j1);
         } else {
 #pragma unroll 1
-            do
+            do {
                 tri_pair<KID, NQ, T, false>(x, m, tw + j * RW, tw + min(j + 1, TT - 1) * RW, k,
                                             h, acc);
-            while (++j < j1);
+                fold_ra();
+            } while (++j < j1);
         }
         if constexpr (F32) {
             T o[NO];
             tri_fold<KID, NQ, T>(m, k, acc, o);
+            if constexpr (KID == TCT_RA)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) o[d] = ra[d];
 #pragma unroll
             for (int a = 0; a < NO; ++a) out[a * 64] += (double)o[a];
 #pragma unroll

@@ -69,7 +69,7 @@ def test_points_beside_the_surface(K, nq):
 
 @pytest.mark.parametrize('nq', [1, 2])
 @pytest.mark.parametrize('K', ['elasticU3', 'elasticT3', 'elasticA3', 'elasticH3', 'elasticRT3',
-                               'elasticRH3'])
+                               'elasticRA3', 'elasticRH3'])
 def test_triangles_of_curved_meshes(K, nq):
     # mean of the logarithm over meshes of several sizes and orientations: on
     # one mesh alone a tile that reaches across a fold of the Z-curve in one form
