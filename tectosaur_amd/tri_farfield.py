@@ -43,19 +43,22 @@ def source_chunks(obs_blocks, n_tiles, resident):
     """Source chunks of a launch of obs_blocks x chunks workgroups, of which
     the chip holds ``resident`` at once, four waves each.  A chunk lasts as long
     as its busiest wave, so every wave takes the same number k of tiles and the
-    chunks are groups of 4 k (far_tri.h): k = 1 while that makes at most
-    sixteen rounds of workgroups (of 512 at least), whose loads and sums overlap
-    others' arithmetic (H FP32, 32,256 triangles: 7.97 ms in one round, 7.41 in
-    four, 7.18 in sixteen) and 512 chunks; more where there are more, as every
+    chunks are groups of 4 k (far_tri.h).  k = 1 up to 8,192 such workgroups, 2
+    up to 16,384, then 3 while that is at most sixteen rounds of workgroups,
+    whose loads and sums overlap others' arithmetic (H FP32, 32,256 triangles:
+    7.97 ms in one round, 7.41 in four, 7.18 in sixteen); more beyond, as every
     chunk has its sums to write and an observation block adds the sums of its
-    chunks one after another (FP64 H, four points, 100 x 59,700 triangles: 311
-    us with 933 chunks, 262 with 467).  us, chunks of equal size -> this: FP64 H,
-    four points, 1,240 triangles 111 -> 64 (90 over points), 2,640 236 -> 200;
-    FP64 T, four points, 1,900 116 -> 86; RH 1,564 63 -> 47; A FP32, 2,640
-    64 -> 52.  From the sizes and the compiled kernel alone: the chunks set the
-    summation order."""
+    chunks one after another, 512 at most (FP64 H, four points, 100 x 59,700
+    triangles: 311 us with 933 chunks, 262 with 467).  k = 1, 2, 3, us: RH FP32,
+    4,144 triangles 98.7 99.3 100.6, 6,580 235 224 227, 9,130 425 410 406; FP64 T,
+    four points, 306 314 316, 760 749 759, 1436 1418 1413.  Chunks of equal size
+    -> this: FP64 H, four points, 1,240 triangles 111 -> 64 (90 over points),
+    2,640 236 -> 200; FP64 T, four points, 1,900 116 -> 86; A FP32, 2,640 64 -> 52.
+    From the sizes and the compiled kernel alone: the chunks set the summation
+    order."""
     groups = -(-n_tiles // 4)
-    k = max(-(-obs_blocks * groups // (16 * max(resident, 512))), -(-groups // 512))
+    work = obs_blocks * groups
+    k = max(min(3, -(-work // 8192)), -(-work // (16 * max(resident, 1024))), -(-groups // 512))
     return -(-groups // k)
 
 

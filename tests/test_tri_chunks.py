@@ -25,9 +25,9 @@ def test_waves_take_equal_tiles(resident):
         k = -(-int(t.max()) // 4)
         # chunks end between groups of four tiles (the last where the tiles do)
         assert t.sum() == nt and t.min() >= 1 and np.all(t[:-1] % 4 == 0)
-        # one tile a wave unless that is more than 16 rounds or 512 chunks
+        # one tile a wave unless that is more than 8,192 workgroups or 512 chunks
         groups = -(-nt // 4)
-        if groups <= 512 and ob * groups <= 16 * max(resident, 512):
+        if groups <= 512 and ob * groups <= 8192:
             assert k == 1 and c == groups
 
 
