@@ -217,12 +217,20 @@ def run_batched(engines, block=256, obs_per_lane=1):
     constants), each with its own layout and source chunks; every engine's
     partial-sum buffer gets what its own ``run('f32')`` would write.
     Operators on the triangle layout (``tri_farfield.TriFarfield``) share a
-    launch of theirs; ``block`` and ``obs_per_lane`` are the point N-body's.
+    launch of theirs, one per rule; ``block`` and ``obs_per_lane`` shape the
+    point N-body's launch.
     Returns the partial-sum buffers."""
     if not engines:
         return []
     tri = [e for e in engines if not isinstance(e, FarfieldEngine)]
     if tri:
+        # the checks of a point launch, over the whole list
+        consts = {(e.K.kid, float(p[0]), float(p[1])) for e in engines
+                  for p in [e.params if isinstance(e, FarfieldEngine) else e.plan.params]}
+        if len(consts) > 1:
+            raise N.TctError('batched N-body: engines differ in kernel or constants')
+        if block not in (64, 128, 256) or obs_per_lane not in (1, 2, 4):
+            raise N.TctError('batched N-body: block %s, %s points a lane' % (block, obs_per_lane))
         from . import tri_farfield
         done = {}
         for nq in sorted({t.nq for t in tri}):
