@@ -11,6 +11,7 @@ relative to an FP64 origin per group, and its accuracy depends on the group
 extent.
 """
 import ctypes
+import threading
 
 import numpy as np
 import torch
@@ -210,6 +211,51 @@ class FarfieldEngine:
     @property
     def pair_evals(self):
         return self.n_obs * self.n_src
+
+
+class PointLayout:
+    """Mixin of the operators over triangles: their point layout, ``engine``
+    and the arrays beside it (``_POINT_ARRAYS``), made by ``_make_points()`` in
+    the constructor (``_build_points``) where the operator itself runs over
+    points, and else when first asked for, by any thread and on any stream."""
+
+    _POINT_ARRAYS = ()
+
+    def _init_points(self):
+        self._engine = None
+        self._engine_lock = threading.Lock()
+
+    def _build_points(self):
+        """On the current stream, like the rest of the set-up."""
+        with self._engine_lock:
+            if self._engine is None:
+                engine, arrays = self._make_points()
+                self.__dict__.update(arrays)
+                self._engine = engine
+        return self._engine
+
+    @property
+    def engine(self):
+        """The point layout and N-body."""
+        if self._engine is None:
+            if torch.cuda.is_current_stream_capturing():
+                raise N.TctError('the point layout cannot be built during a graph capture: '
+                                 'use .engine once before')
+            with self._engine_lock:
+                if self._engine is None:
+                    engine, arrays = self._make_points()
+                    # whoever asked first may not be on the stream of the next
+                    torch.cuda.current_stream().synchronize()
+                    self.__dict__.update(arrays)
+                    self._engine = engine
+        return self._engine
+
+    def __getattr__(self, name):
+        if name in type(self)._POINT_ARRAYS and '_engine_lock' in self.__dict__:
+            self.engine
+            if name in self.__dict__:
+                return self.__dict__[name]
+        raise AttributeError('%s has no attribute %r' % (type(self).__name__, name))
 
 
 def run_batched(engines, block=256, obs_per_lane=1):

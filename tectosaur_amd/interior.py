@@ -31,7 +31,7 @@ import scipy.sparse
 import torch
 
 from . import _native as N, tri_farfield
-from .farfield import FarfieldEngine, morton_order, prec_of, group_extent
+from .farfield import FarfieldEngine, PointLayout, morton_order, prec_of, group_extent
 from .find_near_adj import find_near_pairs, get_tri_centroids_rs
 from .kernels import kernels as KERNELS
 from .quadrature import gauss2d_tri, gaussxw, map_to
@@ -132,13 +132,15 @@ def interior_pairs_quad(K_name, pairs_list, quad, obs_pts, obs_ns, src_pts, src_
     return out.cpu().numpy().reshape((n, 3, 3, 3)).astype(float_type)
 
 
-class TriToPtDirectFarfieldOp:
+class TriToPtDirectFarfieldOp(PointLayout):
     """out[3i + d] = sum over every source triangle and quadrature point of
     K(y_q - x_i) (J w phi . v), pairs at r2 == 0 skipped: the reference's
     TriToPtDirectFarfieldOp (tectosaur/interior.py:139-185) as gather +
     N-body + point reduction, over whole source triangles (``tri``) or over
     points (``engine``).  ``dot_dev`` writes a device tensor
     [n_obs * 3] in the caller's point order."""
+
+    _POINT_ARRAYS = ('tri_of_pt', 'qphi', 'wj_src', 'po_dev', '_packed')
 
     def __init__(self, obs_pts, obs_ns, src_mesh, K_name, nq, params, float_type,
                  precisions=None, device=None):
@@ -172,8 +174,9 @@ class TriToPtDirectFarfieldOp:
         o_pts = obs_pts[self.po]
         self.device = device if device is not None else N.require_device()
         dev = self.device
-        self._engine = None
-        self._points = (params, precisions or (self.prec,), o_pts, obs_ns[self.po], s_pts, s_ns,
+        self._init_points()
+        precisions = precisions or (self.prec,)
+        self._points = (params, precisions, o_pts, obs_ns[self.po], s_pts, s_ns,
                         s_order, s_wj, phi)
         self.curl_src = None
         if K.surf_curl_src:
@@ -186,34 +189,30 @@ class TriToPtDirectFarfieldOp:
         # FP32 runs over whole source triangles where that form pays; FP64
         # and the rest over points
         self.tri = None
-        if 'f32' in self._points[1] and self._tri_pays(K_name):
+        if 'f32' in precisions and self._tri_pays(K_name):
             self.tri = tri_farfield.TriToPtFarfield(K_name, params, o_pts, obs_ns[self.po],
                                                     self.po, s_pts, s_ns, s_order, jac, self.q,
                                                     phi, dev)
-        else:
-            self.engine
+        if self.tri is None or 'f64' in precisions:
+            self._build_points()
 
     def _tri_pays(self, K_name):
         return tri_farfield.pts_supported(K_name, self.nq)
 
-    @property
-    def engine(self):
-        """The point layout and N-body (built when first used)."""
-        if self._engine is None:
-            params, precisions, o_pts, o_ns, s_pts, s_ns, s_order, s_wj, phi = self._points
-            dev = self.device
-            self._engine = FarfieldEngine(self.K.name, params, o_pts, o_ns, s_pts, s_ns,
-                                          precisions=precisions, device=dev,
-                                          extents=(group_extent(o_pts), group_extent(s_pts)))
-            i32 = dict(dtype=torch.int32, device=dev)
-            f64 = dict(dtype=torch.float64, device=dev)
-            self.tri_of_pt = torch.as_tensor(np.repeat(s_order, self.nq).astype(np.int32), **i32)
-            self.qphi = torch.as_tensor(np.ascontiguousarray(phi), **f64)
-            self.wj_src = torch.as_tensor(s_wj, **f64)
-            # point k of the packed observation set is caller point po[k]
-            self.po_dev = torch.as_tensor(self.po, dtype=torch.int64, device=dev)
-            self._packed = torch.empty((self.n_obs, 3), **f64)
-        return self._engine
+    def _make_points(self):
+        params, precisions, o_pts, o_ns, s_pts, s_ns, s_order, s_wj, phi = self._points
+        dev = self.device
+        engine = FarfieldEngine(self.K.name, params, o_pts, o_ns, s_pts, s_ns,
+                                precisions=precisions, device=dev,
+                                extents=(group_extent(o_pts), group_extent(s_pts)))
+        up = lambda a, dt: torch.as_tensor(np.ascontiguousarray(a), dtype=dt, device=dev)
+        arrays = dict(tri_of_pt=up(np.repeat(s_order, self.nq), torch.int32),
+                      qphi=up(phi, torch.float64), wj_src=up(s_wj, torch.float64),
+                      # point k of the packed observation set is caller point po[k]
+                      po_dev=up(self.po, torch.int64),
+                      _packed=torch.empty((self.n_obs, 3), dtype=torch.float64, device=dev))
+        self._points = None     # nothing reads it any more
+        return engine, arrays
 
     @property
     def pair_evals(self):

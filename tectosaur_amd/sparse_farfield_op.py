@@ -30,7 +30,7 @@ import torch
 
 from . import _native as N
 from . import tri_farfield
-from .farfield import FarfieldEngine, morton_order, prec_of
+from .farfield import FarfieldEngine, PointLayout, morton_order, prec_of
 from .kernels import kernels as KERNELS
 from .quadrature import gauss2d_tri
 
@@ -85,10 +85,11 @@ def farfield_plan(nq_far, pts, tris, obs_subset, src_subset, curl):
     return plan
 
 
-class TriToTriDirectFarfieldOp:
+class TriToTriDirectFarfieldOp(PointLayout):
     # whether the operator itself is evaluated by the direct N-body (the
     # treecode operator only uses the point layout)
     _direct = True
+    _POINT_ARRAYS = ('tri_of_pt', 'pt_of_tri', 'qphi', 'wj_src', 'wj_obs', 'curl_src', 'curl_obs')
 
     def __init__(self, nq_far, K_name, params, pts, tris, float_type, obs_subset, src_subset,
                  tile_cfg=None, precisions=None, plan=None):
@@ -115,7 +116,7 @@ class TriToTriDirectFarfieldOp:
         self._args = (params, precisions, tile_cfg)
         self._plan = plan
         self._plan_pts = (plan['o_pts'], plan['s_pts'])
-        self._engine = None
+        self._init_points()
         self.tri = None
         self.tree = None
         # rules of three and four points run over whole triangles
@@ -123,29 +124,25 @@ class TriToTriDirectFarfieldOp:
         if self._direct and tile_cfg is None and tri_farfield.supports(self.q[1]):
             self.tri = tri_farfield.TriFarfield(K_name, params, plan, dev)
         else:
-            self.engine
+            self._build_points()
 
-    @property
-    def engine(self):
-        """The point layout and N-body of this operator (built when first
-        used: the treecode, rules without a triangle form, and callers that
-        drive the point N-body themselves)."""
-        if self._engine is None:
-            params, precisions, tile_cfg = self._args
-            plan, dev = self._plan, self.device
-            self._engine = FarfieldEngine(self.K_name, params, plan['o_pts'], plan['o_ns'],
-                                          plan['s_pts'], plan['s_ns'], precisions=precisions,
-                                          device=dev, tile_cfg=tile_cfg, extents=plan['extents'])
-            # source point k belongs to DOF-space triangle tri_of_pt[k]
-            self.tri_of_pt = N.upload(plan['tri_of_pt'], torch.int32, dev)
-            self.pt_of_tri = N.upload(plan['pt_of_tri'], torch.int32, dev)
-            self.qphi = N.upload(plan['phi'], torch.float64, dev)
-            self.wj_src = N.upload(plan['s_wj'], torch.float64, dev)
-            self.wj_obs = N.upload(plan['o_wj'], torch.float64, dev)
-            if self.curl:
-                self.curl_src = N.upload(plan['curl_src'], torch.float64, dev)
-                self.curl_obs = N.upload(plan['curl_obs'], torch.float64, dev)
-        return self._engine
+    def _make_points(self):
+        """The point layout: for the treecode, rules without a triangle form, and
+        callers that drive the point N-body themselves."""
+        params, precisions, tile_cfg = self._args
+        plan, dev = self._plan, self.device
+        engine = FarfieldEngine(self.K_name, params, plan['o_pts'], plan['o_ns'],
+                                plan['s_pts'], plan['s_ns'], precisions=precisions,
+                                device=dev, tile_cfg=tile_cfg, extents=plan['extents'])
+        # source point k belongs to DOF-space triangle tri_of_pt[k]
+        arrays = {k: N.upload(plan[k], torch.int32, dev) for k in ('tri_of_pt', 'pt_of_tri')}
+        arrays.update((k, N.upload(plan[f], torch.float64, dev)) for k, f in
+                      (('qphi', 'phi'), ('wj_src', 's_wj'), ('wj_obs', 'o_wj')))
+        if self.curl:
+            arrays.update((k, N.upload(plan[k], torch.float64, dev))
+                          for k in ('curl_src', 'curl_obs'))
+        self._plan = None       # nothing reads it any more
+        return engine, arrays
 
     def attach_tree(self, order=4, mac=3.0, pts_per_cell=64, plan=None, n_waves=None):
         """Add a treecode evaluation of this operator (kernels U3, RT3, RA3,
@@ -154,7 +151,7 @@ class TriToTriDirectFarfieldOp:
         ``plan``: a precomputed ``fmm.tree_plan`` for these point sets;
         ``n_waves``: target number of list segments (wavefronts)."""
         from .fmm import TreeFarfield
-        self.tree = TreeFarfield(self.engine, self._plan_pts[0], self._plan_pts[1], order=order,
+        self.tree = TreeFarfield(self._build_points(), self._plan_pts[0], self._plan_pts[1], order=order,
                                  mac=mac, pts_per_cell=pts_per_cell, plan=plan, n_waves=n_waves)
         return self.tree
 
