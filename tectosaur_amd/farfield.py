@@ -51,15 +51,16 @@ def round_up(n, m):
     return ((n + m - 1) // m) * m
 
 
-def group_extent(p):
-    """Largest distance of a point from the mean of its 64-point group."""
+def group_extent(p, group=GROUP):
+    """Largest distance of a point from the mean of its group of consecutive
+    points (the last group may be shorter), points that are NaN left out."""
     p = np.asarray(p, dtype=np.float64)
     n = p.shape[0]
     if n == 0:
         return 0.0
-    q = np.full((round_up(n, GROUP), 3), np.nan)
+    q = np.full((round_up(n, group), 3), np.nan)
     q[:n] = p
-    q = q.reshape((-1, GROUP, 3))
+    q = q.reshape((-1, group, 3))
     cnt = np.sum(~np.isnan(q[:, :, 0]), axis=1)
     mean = np.nansum(q, axis=1) / cnt[:, None]
     d = np.linalg.norm(q - mean[:, None, :], axis=2)

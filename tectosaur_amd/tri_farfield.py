@@ -13,6 +13,7 @@ import numpy as np
 import torch
 
 from . import _native as N
+from .farfield import group_extent
 from .kernels import kernels as KERNELS
 
 TILE = N.TRI_TILE
@@ -26,17 +27,6 @@ RULE_POINTS = (3, 4)
 def supports(qw):
     """Whether a triangle rule with weights ``qw`` has a triangle form."""
     return qw.shape[0] in RULE_POINTS and bool(np.all(qw[-3:] == qw[-1]))
-
-
-def origin_extent(p, counts):
-    """Largest distance of a point from its group's mean; the points [n, 3]
-    come in consecutive groups of ``counts`` (the last may be shorter)."""
-    n = p.shape[0]
-    start = np.arange(0, n, counts)
-    cnt = np.minimum(start + counts, n) - start
-    mean = np.add.reduceat(p, start, axis=0) / cnt[:, None]
-    d = p - np.repeat(mean, cnt, axis=0)
-    return float(np.sqrt(np.max(np.einsum('ij,ij->i', d, d))))
 
 
 def source_chunks(obs_blocks, n_tiles, resident):
@@ -117,7 +107,7 @@ class TriFarfield:
             t['src_curl'] = t['obs_curl'] if shared else up(plan['curl_src'])
         self._t = t
         # rounding bound of one point stored against two different origins
-        self.group_extent = origin_extent(o_pts, nq) + origin_extent(s_pts, nq * TILE)
+        self.group_extent = group_extent(o_pts, nq) + group_extent(s_pts, nq * TILE)
         p = N.TriPlan(kernel=K.kid, nq=nq, n_obs=self.n_obs, n_obs_pad=n_pad, n_src=self.n_src,
                       n_tiles=n_tiles, eps2=(8.0 * 2.0 ** -24 * self.group_extent) ** 2,
                       group_extent=self.group_extent)
@@ -221,7 +211,7 @@ class TriToPtFarfield:
              'partial': torch.empty(self.chunks * 3 * n_pad, **f64)}
         self._t = t
         # rounding bound of one point stored against two different origins
-        self.group_extent = origin_extent(o_pts, LANES) + origin_extent(s_pts, nq * tile)
+        self.group_extent = group_extent(o_pts, LANES) + group_extent(s_pts, nq * tile)
         p = N.TriPtsPlan(kernel=kid, nq=nq, n_pts=o_pts.shape[0], n_obs_pad=n_pad,
                          n_src=tri.shape[0], n_tiles=n_tiles, chunks=self.chunks,
                          eps2=(8.0 * 2.0 ** -24 * self.group_extent) ** 2)
