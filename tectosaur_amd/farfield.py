@@ -51,6 +51,25 @@ def round_up(n, m):
     return ((n + m - 1) // m) * m
 
 
+def _extent2(q):
+    """Largest squared distance of a point from its group's mean, q [groups,
+    points, 3]; NaN if a point is."""
+    if q.shape[1] > 8:
+        r2 = np.zeros(q.shape[:2])
+        for d in range(3):
+            x = np.array(q[:, :, d])
+            x -= x.mean(axis=1, keepdims=True)
+            x *= x
+            r2 += x
+        return r2.max()
+    r2 = 0.0
+    mean = sum(q[:, i] for i in range(q.shape[1])) / q.shape[1]
+    for i in range(q.shape[1]):
+        d = q[:, i] - mean
+        r2 = np.maximum(r2, np.einsum('ij,ij->i', d, d).max())
+    return r2
+
+
 def group_extent(p, group=GROUP):
     """Largest distance of a point from the mean of its group of consecutive
     points (the last group may be shorter), points that are NaN left out."""
@@ -58,6 +77,12 @@ def group_extent(p, group=GROUP):
     n = p.shape[0]
     if n == 0:
         return 0.0
+    full = n // group * group
+    r2 = max((_extent2(q) for q in (p[:full].reshape((-1, group, 3)),
+                                    p[full:].reshape((1, -1, 3))) if q.size),
+             key=lambda x: np.inf if np.isnan(x) else x)
+    if not np.isnan(r2):
+        return float(np.sqrt(r2))
     q = np.full((round_up(n, group), 3), np.nan)
     q[:n] = p
     q = q.reshape((-1, group, 3))

@@ -75,10 +75,11 @@ def farfield_plan(nq_far, pts, tris, obs_subset, src_subset, curl):
     n_obs = obs_subset.shape[0]
     pt_of_tri = np.empty(n_obs, dtype=np.int32)
     pt_of_tri[o_order] = np.arange(n_obs, dtype=np.int32)
+    extent = group_extent(o_pts)
     plan = dict(nq=nq, q=(qx, qw), phi=np.ascontiguousarray(phi), o_pts=o_pts, o_ns=o_ns,
                 o_wj=o_wj, s_pts=s_pts, s_ns=s_ns, s_wj=s_wj,
                 tri_of_pt=np.repeat(s_order, nq).astype(np.int32), pt_of_tri=pt_of_tri,
-                extents=(group_extent(o_pts), group_extent(s_pts)))
+                extents=(extent, extent if same else group_extent(s_pts)))
     if curl:
         plan['curl_src'] = curls(src_subset)
         plan['curl_obs'] = plan['curl_src'] if same else curls(obs_subset)
