@@ -86,7 +86,9 @@ class TriFarfield:
         self.n_out = N.lib().tct_tri_outputs(K.kid, nq)
         words = N.lib().tct_tri_words(K.kid, nq)
         same = s_pts is o_pts
-        up = lambda a: N.upload(a, None, device)
+        # in the types that the kernels read, whatever a caller's plan holds
+        up = lambda a: N.upload(a, torch.float64, device)
+        up32 = lambda a: N.upload(a, torch.int32, device)
         f64 = dict(dtype=torch.float64, device=device)
         f32 = dict(dtype=torch.float32, device=device)
         obs_of = np.empty(self.n_obs, dtype=np.int32)   # packed position -> triangle
@@ -97,7 +99,7 @@ class TriFarfield:
              'rec32': torch.empty(n_tiles * TILE * words, **f32),
              'rec64': torch.empty(n_tiles * TILE * words, **f64),
              'src_org': torch.empty(3 * n_tiles, **f64),
-             'obs_tri': up(obs_of), 'src_tri': up(plan['tri_of_pt'][::nq]),
+             'obs_tri': up32(obs_of), 'src_tri': up32(plan['tri_of_pt'][::nq]),
              'obs_jac': up(jac(plan['o_wj']))}
         t['src_jac'] = t['obs_jac'] if same else up(jac(plan['s_wj']))
         if K.surf_curl_obs:
