@@ -520,13 +520,13 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void far_tri_kernel(TriSegTable<T> 
     for (int t = sh.first; t < t1; t += sh.step) {
         const int real = min(TT, n_src - t * TT), j0 = sh.j0(real), j1 = sh.j1(real);
         if (j0 == j1) break;   // fewer triangles than parts: nothing for this wave
-        // the previous tile's LDS reads were issued before these writes, and
-        // a wave's LDS operations complete in order
+        wave_lds_order();
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const int e = v * 64 + lane;
             if (e < NVEC) tile[e] = pre[v];
         }
+        wave_lds_order();
         {
             const int tn = t + sh.step < t1 ? t + sh.step : t;
             const vec *src = (const vec *)(g.rec + (size_t)tn * TT * RW);

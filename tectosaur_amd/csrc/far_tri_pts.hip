@@ -191,13 +191,13 @@ __global__ __launch_bounds__(64 * TRI_WAVES) void tri_pts_kernel(
     for (int t = sh.first; t < t1; t += sh.step) {
         const int real = min(TP, n_src - t * TP), j0 = sh.j0(real), j1 = sh.j1(real);
         if (j0 == j1) break;   // fewer triangles than parts: nothing for this wave
-        // the previous tile's LDS reads were issued before these writes, and
-        // a wave's LDS operations complete in order
+        wave_lds_order();
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const int e = v * 64 + lane;
             if (e < NVEC) tile[e] = pre[v];
         }
+        wave_lds_order();
         {
             const int tn = t + sh.step < t1 ? t + sh.step : t;
             const vec *src = (const vec *)(rec + (size_t)tn * TP * RW);

@@ -381,14 +381,12 @@ __device__ __forceinline__ void write_pairs(F &&pack, const PairTable &tab,
     const int lane = (int)threadIdx.x & 63;
 #pragma unroll 1
     for (int h = 0; h < PW / SP; ++h) {
-        // a wave's LDS operations complete in order: no barrier needed
-        // between its writes and reads but the compiler's
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_order();
         if (writer && pl / SP == h) {
             pack(&sg.v[(pl % SP) * ND]);
             sg.row[pl % SP] = row;
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_order();
         int p = 0, i = lane;   // entry i of pair p: element p * 81 + i
 #pragma unroll 2
         for (int e = lane; e < NE; e += 64) {

@@ -40,7 +40,7 @@ __global__ __launch_bounds__(256) void bsr9_kernel(int n_block_rows,
         // on its own index load before its data and x loads can issue
         for (int kb = k0; kb < k1; kb += 9 * NB) {
             scol[wave][lane] = kb + lane < k1 ? indices[kb + lane] : 0;
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_order();
             const int ke = kb + 9 * NB < k1 ? kb + 9 * NB : k1;
             if (lane < NB * 9) {
 #pragma unroll 2
@@ -51,7 +51,7 @@ __global__ __launch_bounds__(256) void bsr9_kernel(int n_block_rows,
                     for (int j = 0; j < 9; ++j) s += (double)A[j] * xc[j];
                 }
             }
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_order();
         }
     }
     if (lane < NB * 9) part[wave][lane] = s;

@@ -71,4 +71,16 @@ inline ElasticConsts elastic_consts(const double *params) {
     return c;
 }
 
+#ifdef __HIPCC__
+// Between LDS writes of a wave and its other lanes' reads of them, and between
+// those and the next writes.  A wave's LDS operations complete in order, so no
+// instruction is needed, but the compiler must not move or forward a lane's own
+// accesses across: nothing else tells it that other lanes read them.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+#endif
+
 }  // namespace tct
