@@ -213,12 +213,13 @@ __global__ __launch_bounds__(256) void interior_corners_kernel(
 
 // y[3 i + d] (+)= sum_{k in row i} sum_j data[k][d][j] x[9 indices[k] + j].
 // RL lanes per output row (point, component): lane l takes blocks l, l + RL,
-// ..., whose sums meet in a butterfly.  Most points have no close triangle and
-// those on the surface's trace have dozens, a serial chain of scattered loads
-// when one thread took a row (62,500 rows, 47,492 blocks, at most 56 in a row:
-// 25 us; 4, 8, 16 and 32 lanes 9.6, 9.5, 9.7, 18; 160,000 rows and 246,576 blocks:
-// 50 us; 31, 25, 28, 47).
-constexpr int RL = 8;
+// ..., whose sums meet in a butterfly.  Points on the surface's trace have dozens
+// of close triangles, a serial chain of scattered loads when one thread takes a
+// row (62,500 rows, 47,492 blocks, at most 56 in a row: 25 us with one lane, 9.6,
+// 9.5, 9.7 and 18 with 4, 8, 16 and 32; 160,000 rows, 121,778 blocks: 44 and, with
+// 8, 19).  Most points have none, and with very many rows their lanes are the
+// cost: see bsr39_lanes.
+template <int RL>
 __global__ __launch_bounds__(256) void bsr39_kernel(int64_t n_rows,
                                                     const int32_t *__restrict__ indptr,
                                                     const int32_t *__restrict__ indices,
@@ -242,6 +243,11 @@ __global__ __launch_bounds__(256) void bsr39_kernel(int64_t n_rows,
     for (int off = RL / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
     if (l == 0) y[r] = accumulate ? y[r] + s : s;
 }
+
+// Eight lanes up to 256k points: there the longest rows decide.  Beyond, one:
+// 1,000,000 points with 0.01 and 0.3 blocks each take 13 and 31 us, and 62 and
+// 110 with eight.
+static int bsr39_lanes(int64_t n_rows) { return n_rows <= 262144 ? 8 : 1; }
 
 __device__ __forceinline__ double dot3(const double *a, const double *b) {
     return a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
@@ -521,9 +527,15 @@ extern "C" int tct_bsr39_spmv(int64_t n_block_rows, const int32_t *indptr, const
                   (long long)n_block_rows);
     TCT_CHECK_ARG(indptr && x && y && (data || n_block_rows == 0), "bsr39: null pointer");
     if (n_block_rows == 0) return TCT_OK;
-    hipLaunchKernelGGL(bsr39_kernel, dim3((unsigned)ceil_div(3 * RL * n_block_rows, 256)), dim3(256),
-                       0, as_stream(stream), n_block_rows, indptr, indices, data, x, y,
-                       accumulate);
+    const int rl = bsr39_lanes(n_block_rows);
+    const dim3 grid((unsigned)ceil_div(3 * rl * n_block_rows, (int64_t)256));
+    hipStream_t st = as_stream(stream);
+    if (rl == 8)
+        hipLaunchKernelGGL(bsr39_kernel<8>, grid, dim3(256), 0, st, n_block_rows, indptr, indices,
+                           data, x, y, accumulate);
+    else
+        hipLaunchKernelGGL(bsr39_kernel<1>, grid, dim3(256), 0, st, n_block_rows, indptr, indices,
+                           data, x, y, accumulate);
     TCT_CHECK_LAUNCH("bsr39_spmv");
     return TCT_OK;
 }
