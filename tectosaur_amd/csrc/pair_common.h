@@ -204,6 +204,10 @@ struct PairTable {
     uint2 off[81];   // six byte-sized offsets per entry
 };
 
+// T, A and H: what is in LDS are the 81 entries themselves; no table.
+template <int KID>
+constexpr bool pair_tensor() { return KID == TCT_T || KID == TCT_A || KID == TCT_H; }
+
 // Doubles of one pair in LDS.
 template <int KID>
 constexpr int pack_size() {
@@ -212,13 +216,13 @@ constexpr int pack_size() {
 // Pairs in LDS at a time (GL lanes a pair).
 template <int KID, int GL>
 constexpr int pack_pairs() {
-    const int pw = 64 / GL, most = KID <= TCT_H ? 8 : 16;
-    return pw < most ? pw : most;
+    return 64 / GL < 16 ? 64 / GL : 16;
 }
 
 // Filled by the first 81 threads of a workgroup (a barrier before its use).
 template <int KID>
 __device__ __forceinline__ void fill_pair_table(PairTable &t) {
+    if constexpr (pair_tensor<KID>()) return;
     for (int i = (int)threadIdx.x; i < 81; i += (int)blockDim.x) {
         const int b = i / 27, d = i / 9 % 3, e = i / 3 % 3, f = i % 3;
         int o[6] = {0, 0, 0, 0, 0, 0};
@@ -361,6 +365,13 @@ __device__ __forceinline__ int out_row(const int32_t *__restrict__ rows, int pai
     return rows ? rows[pair] : pair;
 }
 
+// Entries in flight at a time: as many as leave a kernel's waves per SIMD as
+// they are (T, A and H read one LDS word an entry, the others three to seven).
+template <int KID, int GL>
+constexpr int write_unroll() {
+    return KID == TCT_RH && GL >= 4 ? 7 : (KID == TCT_U || KID > TCT_H ? 2 : 11);
+}
+
 // LDS of one wave.
 template <int KID, int GL>
 struct PairStage {
@@ -371,13 +382,17 @@ struct PairStage {
 // The outputs of the 64 / GL pairs of one wave.  Every lane of the wave
 // calls it; the GL lanes of pair pl, of which `writer` has the sums.
 // pack(p) puts the pair's sums in LDS (pack_pair).  SUB: subtracted from what
-// is there instead of written.
-template <int KID, int GL, bool SUB, typename F>
+// is there instead of written.  UN entries a lane are formed at a time
+// (write_unroll).  Where few waves run this latency is what a launch adds: 8 pairs
+// at a time, an entry after another, made 16 points of T on 1,000 pairs take 29 us;
+// 16 pairs and all their entries in flight 24, with four lanes a pair 15.
+template <int KID, int GL, bool SUB, int UN, typename F>
 __device__ __forceinline__ void write_pairs(F &&pack, const PairTable &tab,
                                             PairStage<KID, GL> &sg, int pl, bool writer, int row,
                                             double *__restrict__ out) {
     constexpr int PW = 64 / GL, SP = pack_pairs<KID, GL>(), ND = pack_size<KID>();
-    constexpr int NE = SP * 81;
+    constexpr unsigned NE = SP * 81;
+    constexpr int NI = (NE + 63) / 64;
     const int lane = (int)threadIdx.x & 63;
 #pragma unroll 1
     for (int h = 0; h < PW / SP; ++h) {
@@ -387,19 +402,35 @@ __device__ __forceinline__ void write_pairs(F &&pack, const PairTable &tab,
             sg.row[pl % SP] = row;
         }
         wave_lds_order();
-        int p = 0, i = lane;   // entry i of pair p: element p * 81 + i
-#pragma unroll 2
-        for (int e = lane; e < NE; e += 64) {
+        auto put = [&](int p, int i, double x) {
             const int r = sg.row[p];
-            const double x = pair_entry<KID>(&sg.v[p * ND], tab.off[i]);
             if (r >= 0) {
                 double *o = out + (size_t)r * 81 + i;
                 *o = SUB ? *o - x : x;
             }
-            i += 64;
-            if (i >= 81) {
-                i -= 81;
-                ++p;
+        };
+        if constexpr (UN > 2) {
+            // entry i of pair p: p * 81 + i = lane + 64 k
+#pragma unroll UN
+            for (int k = 0; k < NI; ++k) {
+                const unsigned e = lane + 64u * k;
+                if (k == NI - 1 && e >= NE) break;
+                const unsigned p = e / 81u, i = e - 81u * p;
+                if constexpr (pair_tensor<KID>())
+                    put(p, i, sg.v[e]);      // the entries themselves
+                else
+                    put(p, i, pair_entry<KID>(&sg.v[p * ND], tab.off[i]));
+            }
+        } else {
+            int p = 0, i = lane;
+#pragma unroll UN
+            for (unsigned e = lane; e < NE; e += 64) {
+                put(p, i, pair_entry<KID>(&sg.v[p * ND], tab.off[i]));
+                i += 64;
+                if (i >= 81) {
+                    i -= 81;
+                    ++p;
+                }
             }
         }
     }

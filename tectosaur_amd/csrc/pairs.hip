@@ -286,7 +286,7 @@ __global__ __launch_bounds__(256) void pairs_kernel(int nq, const double *__rest
         tri_from_edges(ot, oe[0], oe[1]);
         tri_from_edges(st, g.se[0], g.se[1]);
     }
-    write_pairs<KID, GL, false>(
+    write_pairs<KID, GL, false, write_unroll<KID, GL>()>(
         [&](double *p) { pack_pair<KID>(acc, ot, st, c, oc, sc, flip, p); }, table,
         stage[threadIdx.x / 64], (int)(threadIdx.x % 64) / GL, sub == 0,
         live ? out_row(rows, pair) : -1, out);
@@ -370,16 +370,20 @@ __global__ __launch_bounds__(rh_chunk_block(S)) void pairs_rh_chunk_kernel(
     for (int k = 0; k < NA; ++k) o[k] = acc[k];
 }
 
+constexpr int FL = 4;   // lanes a pair of the kernel below
 __global__ __launch_bounds__(256) void pairs_rh_finish_kernel(
     int n_pairs, const double *__restrict__ pts, const int32_t *__restrict__ tris,
     const int32_t *__restrict__ pairs, int pair_width, int nch, ElasticConsts c,
     const int32_t *__restrict__ rows, double *__restrict__ out) {
     constexpr int NA = n_acc<TCT_RH>();
     __shared__ PairTable table;
-    __shared__ PairStage<TCT_RH, 1> stage[4];
+    __shared__ PairStage<TCT_RH, FL> stage[4];
     fill_pair_table<TCT_RH>(table);
     __syncthreads();
-    const int pair = blockIdx.x * blockDim.x + threadIdx.x;
+    // FL lanes a pair, all with its sums: a wave then writes the outputs of
+    // all its pairs in one go (with one lane a pair in four; 1,000 coincident
+    // pairs 48 -> 33 us, 20,000 207 -> 189)
+    const int gid = blockIdx.x * blockDim.x + threadIdx.x, pair = gid / FL;
     const bool live = pair < n_pairs;
     const int pr = live ? pair : n_pairs - 1;
     const int32_t *pp = pairs + (size_t)pr * pair_width;
@@ -403,9 +407,10 @@ __global__ __launch_bounds__(256) void pairs_rh_finish_kernel(
     Tri ot, st;
     load_tri(ot, pts, tris, pp[0], oc, 0);
     load_tri(st, pts, tris, pp[1], sc, flip);
-    write_pairs<TCT_RH, 1, false>(
+    write_pairs<TCT_RH, FL, false, 7>(
         [&](double *p) { pack_pair<TCT_RH>(acc, ot, st, c, oc, sc, flip, p); }, table,
-        stage[threadIdx.x / 64], (int)(threadIdx.x % 64), true, live ? row : -1, out);
+        stage[threadIdx.x / 64], (int)(threadIdx.x % 64) / FL, gid % FL == 0, live ? row : -1,
+        out);
 }
 
 __global__ void sub_f64_kernel(int64_t n, const double *__restrict__ a,
@@ -496,7 +501,11 @@ extern "C" int tct_pairs_integrate_rows(int kernel, int64_t nq, const double *qx
         // it stays ahead down to ~10k wavefronts; the classes with the
         // r = 0 test (coincident, adjacent) keep gaining from more lanes up
         // to ~16k-46k wavefronts (64-180 per CU).
-        const int gmax = nq >= 1024 ? 64 : (nq >= 128 ? 16 : (nq >= 24 ? 4 : 1));
+        int gmax = nq >= 1024 ? 64 : (nq >= 128 ? 16 : (nq >= 24 ? 4 : 1));
+        // few points on few pairs: a wave's outputs leave sixteen pairs at a
+        // time, so four lanes a pair save three of four goes (16 points, T, one
+        // lane and four: 1,000 pairs 22.7 and 14.4 us, 20,000 24.5 and 25.7)
+        if (kernel <= TCT_H && nq >= 8 && gmax == 1 && n_pairs < 16384) gmax = 4;
         const int64_t min_waves = check0 ? 16384 : 4096;
         gl = gmax;
         for (int g = 1; g < gmax; g *= 4)
@@ -559,7 +568,7 @@ extern "C" int tct_pairs_integrate_rows(int kernel, int64_t nq, const double *qx
         else
             TCT_RH_CHUNKS(CK_NONE);
 #undef TCT_RH_CHUNKS
-        hipLaunchKernelGGL(pairs_rh_finish_kernel, dim3((unsigned)ceil_div(n_pairs, (int64_t)256)),
+        hipLaunchKernelGGL(pairs_rh_finish_kernel, dim3((unsigned)ceil_div(n_pairs * FL, (int64_t)256)),
                            dim3(256), 0, st, np, pts, tris, pairs, pair_width, slots, c, rows, out);
         TCT_CHECK_LAUNCH("pairs_integrate");
         return TCT_OK;

@@ -272,7 +272,7 @@ __global__ __launch_bounds__(256) void pairs_product_kernel(
     Tri ot, st;
     tri_from_edges(FS ? st : ot, fe[0], fe[1]);
     tri_from_edges(FS ? ot : st, me[0], me[1]);
-    write_pairs<KID, GL, SUB>(
+    write_pairs<KID, GL, SUB, write_unroll<KID, GL>()>(
         [&](double *p) {
             if constexpr (KID == TCT_U) {
                 // the six D D sums and the 1/r sum to the six entries of K
@@ -304,7 +304,8 @@ __global__ __launch_bounds__(256) void pairs_product_kernel(
 // once, times the waves that the SIMD runs -- whole ones while they are few,
 // and never less than two, which a SIMD needs to issue at its rate.  (19 x 19
 // points, RH, 226,590 pairs: P = 4 with four lanes for five groups 191 us,
-// P = 2 with two lanes for ten 160 us.)
+// P = 2 with two lanes for ten 160 us.)  The outputs of a wave's pairs leave
+// sixteen pairs at a time, 350 slots each time.
 struct Split {
     int P, GL;
 };
@@ -321,8 +322,8 @@ inline Split product_split(int kernel, int nf, int nm, int64_t n_pairs) {
         const int groups = (nf + P - 1) / P;
         for (int gl = 1, lg = 0; gl <= 16 && gl <= groups; gl *= 2, ++lg) {
             if (tensor && (gl == 2 || gl == 8)) continue;
-            const double serial = (double)((groups + gl - 1) / gl) * nm * (6 + 26 * P) + 1500.0 +
-                                  5.0 * na * lg;
+            const double serial = (double)((groups + gl - 1) / gl) * nm * (6 + 26 * P) + 800.0 +
+                                  (gl < 4 ? 1400.0 / gl : 350.0) + 5.0 * na * lg;
             double waves = (double)n_pairs * gl / 64.0 / 1024.0;
             waves = waves < 2.0 ? 2.0 : (waves < 8.0 ? std::ceil(waves) : waves + 0.5);
             if (cost == 0.0 || serial * waves < cost) {
