@@ -274,7 +274,7 @@ class RegularizedNearfieldIntegralOp:
             r_dev = rank[int(s):int(s) + k]
             q = rules[name]
             fused = (same and not keep_uncorrected and w == 2 and check0 == corr_check0 and
-                     pairs_int.product_side(q) is not None)
+                     pairs_int.product_side(q, k) is not None)
             pairs_int.pairs_quad_rows(q, p_dev, check0, r_dev, data,
                                       minus=far_q if fused else None)
             if not fused:

@@ -51,14 +51,22 @@ def rule_has_equal_params(qx):
     return bool(qx.size) and bool(np.any((qx[:, 0] == qx[:, 2]) & (qx[:, 1] == qx[:, 3])))
 
 
-def product_pays(kernel, n):
+def product_pays(kernel, n, n_pairs):
     """Whether a rule that is a product of an n-point triangle rule with
-    itself runs as one: always for the surface-curl kernels, whose sums are
-    few (3 x 3 points, RH3 135 -> 106 us for 710,704 pairs); for U, T, A and H,
-    with 81 sums a pair and a wave less per SIMD, from 19 points (U3, 710,704
-    pairs: 4 x 4 points 142 -> 167 us, 19 x 19 873 -> 626; 13 x 13, 29,128
-    pairs: 56 -> 90; T3, 19 x 19: 1212 -> 1106)."""
-    return kernel in ('elasticRT3', 'elasticRA3', 'elasticRH3') or n >= 19
+    itself runs as one.  The surface-curl kernels, whose sums are few, always
+    (3 x 3 points, RH3 135 -> 106 us for 710,704 pairs); U, T, A and H, with 81
+    sums a pair and a wave less per SIMD, from 19 points (U3, 710,704 pairs:
+    4 x 4 points 142 -> 167 us, 19 x 19 873 -> 626; 13 x 13, 29,128 pairs: 56 -> 90;
+    T3, 19 x 19: 1212 -> 1106), T, A and H with fewer than 28 on 8,192 pairs or
+    more (19 x 19 points, 5,000 pairs, T 41 -> 43; 20,000: 100 -> 67).  A rule of
+    1,024 points and more in all, which has 64 lanes a pair as it stands and at
+    most 16 as a product, only on as many pairs as give every SIMD a wave either
+    way (64 x 64 points, 1,000 pairs: U 39 -> 55 us, H 52 -> 97, RT 28 -> 34, RH 31 ->
+    28; 5,000: 169 -> 104, 235 -> 185, 82 -> 52, 52 -> 44)."""
+    curl = kernel in ('elasticRT3', 'elasticRA3', 'elasticRH3')
+    if not curl and (n < 19 or (n < 28 and kernel != 'elasticU3' and n_pairs < 8192)):
+        return False
+    return n * n < 1024 or n_pairs >= (512 if kernel == 'elasticRH3' else 1536)
 
 
 def r0_test_mode(q, check0):
@@ -118,11 +126,12 @@ class PairsIntegrator:
         o.kid = N.KERNEL_IDS[kernel]
         return o
 
-    def product_side(self, q):
-        """The triangle rule of a product rule that this kernel runs as one,
-        or None."""
+    def product_side(self, q, n_pairs):
+        """The triangle rule of a product rule that this kernel runs as one on
+        so many pairs, or None."""
         side = getattr(q, 'side', None)
-        return side if side is not None and product_pays(self.kernel, side[1].shape[0]) else None
+        pays = side is not None and product_pays(self.kernel, side[1].shape[0], n_pairs)
+        return side if pays else None
 
     def pairs_quad_rows(self, q, pairs_dev, check0, rows, out, minus=None, subtract=False):
         """Pair i's block into row rows[i] (int32 device tensor) of ``out``
@@ -132,8 +141,8 @@ class PairsIntegrator:
         n = pairs_dev.shape[0]
         width = pairs_dev.shape[1]
         side = getattr(q, 'side', None)
-        product = self.product_side(q) is not None or subtract
-        if (minus is not None or subtract) and (side is None or not product):
+        product = self.product_side(q, n) is not None or subtract or minus is not None
+        if (minus is not None or subtract) and side is None:
             raise N.TctError('only product rules subtract')
         mq, mw = (None, None) if minus is None else minus.side
         st = N.stream_ptr()
@@ -161,7 +170,7 @@ class PairsIntegrator:
         st = N.stream_ptr()
         # a rule that is a product runs as one, unless the caller chooses how
         # many lanes share a pair's 4-D rule
-        side = self.product_side(q) if lanes_per_pair == 0 else None
+        side = self.product_side(q, n) if lanes_per_pair == 0 else None
         for s in range(0, n, CALL_SIZE):
             e = min(n, s + CALL_SIZE)
             if side is not None:
