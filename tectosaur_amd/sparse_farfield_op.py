@@ -80,6 +80,8 @@ def farfield_plan(nq_far, pts, tris, obs_subset, src_subset, curl):
                 o_wj=o_wj, s_pts=s_pts, s_ns=s_ns, s_wj=s_wj,
                 tri_of_pt=np.repeat(s_order, nq).astype(np.int32), pt_of_tri=pt_of_tri,
                 extents=(extent, extent if same else group_extent(s_pts)))
+    if tri_farfield.supports(qw):
+        plan['tri_extent'] = tri_farfield.layout_extent(o_pts, s_pts, nq)
     if curl:
         plan['curl_src'] = curls(src_subset)
         plan['curl_obs'] = plan['curl_src'] if same else curls(obs_subset)

@@ -29,6 +29,12 @@ def supports(qw):
     return qw.shape[0] in RULE_POINTS and bool(np.all(qw[-3:] == qw[-1]))
 
 
+def layout_extent(o_pts, s_pts, nq):
+    """Rounding bound of one point stored against two different origins: the
+    extents of an observation triangle and of a source tile."""
+    return group_extent(o_pts, nq) + group_extent(s_pts, nq * TILE)
+
+
 def source_chunks(obs_blocks, n_tiles, resident):
     """Source chunks of a launch of obs_blocks x chunks workgroups, of which
     the chip holds ``resident`` at once, four waves each.  A chunk lasts as long
@@ -108,8 +114,8 @@ class TriFarfield:
             shared = K.surf_curl_obs and plan['curl_src'] is plan['curl_obs']
             t['src_curl'] = t['obs_curl'] if shared else up(plan['curl_src'])
         self._t = t
-        # rounding bound of one point stored against two different origins
-        self.group_extent = group_extent(o_pts, nq) + group_extent(s_pts, nq * TILE)
+        extent = plan.get('tri_extent')
+        self.group_extent = layout_extent(o_pts, s_pts, nq) if extent is None else float(extent)
         p = N.TriPlan(kernel=K.kid, nq=nq, n_obs=self.n_obs, n_obs_pad=n_pad, n_src=self.n_src,
                       n_tiles=n_tiles, eps2=(8.0 * 2.0 ** -24 * self.group_extent) ** 2,
                       group_extent=self.group_extent)

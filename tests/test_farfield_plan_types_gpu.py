@@ -30,3 +30,19 @@ def test_plan_of_other_types(K, nq):
     # points rounded to 1e-7 of their size, an eighth and more apart: r^-3 moves
     # by a few 1e-6 of a pair's term
     assert np.linalg.norm(y - ref) <= 1e-4 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize('K', ['elasticU3', 'elasticRH3'])
+def test_plan_without_the_triangle_extent(K):
+    # a plan made before it held one
+    from tectosaur_amd.sparse_farfield_op import TriToTriDirectFarfieldOp, farfield_plan
+    pts, tris = mesh.make_rect(9, 8, [[-1, 0, 1], [-1, 0, -1], [1, 0, -1], [1, 0, 1]])
+    n = np.arange(tris.shape[0])
+    args = (1, K, [1.0, 0.25], pts, tris, np.float32, n, n)
+    plan = farfield_plan(1, pts, tris, n, n, K == 'elasticRH3')
+    a = TriToTriDirectFarfieldOp(*args, plan=plan)
+    del plan['tri_extent']
+    b = TriToTriDirectFarfieldOp(*args, plan=plan)
+    assert a.tri.group_extent == b.tri.group_extent > 0
+    v = np.random.default_rng(0).standard_normal(9 * n.size)
+    assert np.array_equal(a.dot(v), b.dot(v))
