@@ -19,9 +19,17 @@
 //     pair needs only 7 moments, sum 1/r and sum D_k D_l / r^3, and one
 //     contraction with the source curl (RH); RT's 1/r term likewise;
 //   * U keeps its two terms in separate sums, scaled once per tile.
-// VALU instructions per point pair with a three-point rule, point form ->
-// this: H 54 -> 39, RH 40 -> 23, T 31 -> 25, A 30 -> 24, RT 27 -> 23,
-// RA 26 -> 23, U 20 -> 19.
+// VALU instructions per point pair with a three-point rule in FP32, counted in
+// the compiled loops that far tiles run (T, A and RT with the r2 test, two more),
+// point form -> this: H 54 -> 39, RH 40 -> 23, T 31 -> 28, A 31 -> 28, RT 27 -> 25,
+// RA 26 -> 24, U 20 -> 19; near tiles take two more.
+// FP64: 24 to 47 a pair, and few waves to hide their latency: the registers
+// leave three a SIMD for U, A and RA with three points, two for the others, one
+// for H and RH with four (256 VGPRs and 66 or 44 AGPRs).  It rounds as the point
+// form does except that T, A, RT and RA take one n . D or m . D for all points of
+// the other triangle, whose error then does not average out: relative L2 error
+// against 64-bit formulas 1.05 to 1.15 times the point form's (2,046 triangles, T
+// with four points 1.7e-14 -> 2.0e-14), U, H and RH 0.96 to 1.01 times.
 #pragma once
 #include "far_pair.h"
 
@@ -117,12 +125,12 @@ __device__ __forceinline__ void tri_head(const T *r, TriHead<KID, T> &h) {
 // unit's two-at-once issue (which register numbers may forbid), so only
 // measurement tells.  15,842 triangles, FP32, us, terms in any order and one
 // fence per source point -> the order below and this:
-//   3 points  U 1045 -> 912, T 1337 -> 1213, A 1443 -> 1183, H 1824 -> 1649,
-//             RT 1234 -> 1091, RA 1292 -> 1070, RH 1208 -> 1214
-//   4 points  U 1970 -> 1658, T 2503 -> 2146, A 2602 -> 2025, H 3364 -> 3028,
-//             RT 2383 -> 1927, RA 2345 -> 1879, RH 2201 -> 2017
-// (point form, 3 and 4 points: U 1164 2011, T 1465 2556, A 1377 2458,
-// H 2353 4111, RT 1413 2459, RA 1253 2217, RH 1916 3275).  FP64 issues no pairs
+//   3 points  U 1045 -> 961, T 1337 -> 1188, A 1443 -> 1186, H 1824 -> 1685,
+//             RT 1234 -> 1065, RA 1292 -> 1113, RH 1208 -> 1170
+//   4 points  U 1970 -> 1650, T 2503 -> 2102, A 2602 -> 2014, H 3364 -> 3058,
+//             RT 2383 -> 1936, RA 2345 -> 1924, RH 2201 -> 1990
+// (point form, 3 and 4 points: U 1150 2015, T 1453 2540, A 1354 2426,
+// H 2335 4108, RT 1385 2459, RA 1219 2166, RH 1790 3073).  FP64 issues no pairs
 // and is within 2% either way.
 template <int KID, int NQ, typename T>
 constexpr int tri_fence() {
@@ -133,11 +141,13 @@ constexpr int tri_fence() {
 // Whether every tile runs the body with the r2 test: its two instructions more
 // a pair change which others pair up, for the better with these (147,456
 // triangles, FP32, ms, tiles far from the lane without the test -> all with it):
-//   3 points  T 121.4 -> 95.0, A 103.2 -> 95.2, RT 92.8 -> 88.5
-//   4 points  T 212.9 -> 176, A 201.0 -> 165, RH 171.4 -> 166
-// and for the worse with the others (U 69.3 -> 72.8, RA 83.5 -> 87.9, RH with
-// three points 90.7 -> 99.6, H with three 132.5 -> 150, with four 245.0 ->
-// 253.8) and FP64 (1-2%).
+//   3 points  T 121.0 -> 95.1, A 106.1 -> 96.6, RT 93.0 -> 85.9
+//   4 points  T 212.2 -> 174.8, A 203.9 -> 165.3, RH 175.3 -> 166.1
+// and for the worse with the others (three and four points, U 70.2 -> 73.1, 131.7
+// -> 141.8; H 132.7 -> 142.0, 252.8 -> 257.2; RA 85.7 -> 90.8, 159.6 -> 162.0; RH
+// 89.2 -> 93.7; RT 167.3 -> 178.4).  FP64 keeps both bodies: at 15,842 triangles,
+// where most tiles have the test anyway, one body is 1% faster, with H and RH with
+// four points, which it frees of register moves, 7 and 10%.
 template <int KID, int NQ, typename T>
 constexpr bool tri_always_masked() {
     return sizeof(T) == 4 && (KID == TCT_T || KID == TCT_A || (KID == TCT_RT && NQ == 3) ||

@@ -14,8 +14,9 @@
 // with, 406 without; T 484 and 487; seven points, below).
 // 62,500 points x 2,048 triangles, us, point form (far_p2p.hip, its sums and
 // the permutation of its outputs) -> this:
-//   4 points  U 312 -> 255, T 388 -> 322, A 371 -> 332, H 580 -> 457
-//   7 points  U 492 -> 411, T 622 -> 503, A 586 -> 547
+//   3 points  U 240 -> 177, T 291 -> 224, A 272 -> 238, H 445 -> 336
+//   4 points  U 300 -> 221, T 371 -> 284, A 345 -> 305, H 574 -> 428
+//   7 points  U 482 -> 377, T 615 -> 464, A 570 -> 518
 // Two, three and four points a lane (fewer LDS reads a pair) were slower: U
 // 421, 428 and 438, T 518, 557 and 557 with seven rule points.
 #include "far_tri.h"
@@ -388,9 +389,10 @@ static hipError_t pts_occ(int *blocks) {
         blocks, (const void *)tri_pts_kernel<KID, NS>, 64 * TRI_WAVES, lds);
 }
 
-// H with seven points runs over points (far_p2p.hip): its tiles' origins are
-// not the point form's, and 1/r^3 next to the surface leaves the two roundings
-// of D up to 2e-5 of the result apart, for 770 us in place of 960.
+// H with seven points runs over points (far_p2p.hip): with tiles of 112 points,
+// as they once were, 1/r^3 next to the surface left the roundings of D in the two
+// forms up to 2e-5 of the result apart (770 us in place of 960); with tiles of 63 it
+// has not been measured.
 static bool pts_has(int kernel, int nq) {
     return kernel >= TCT_U && kernel <= TCT_H &&
            (nq == 3 || nq == 4 || (nq == 7 && kernel != TCT_H));

@@ -55,6 +55,8 @@ def _is_identity(subset):
 
 
 def to_tri_space(dof_indices, obs_subset, src_subset):
+    """Positions in the subsets to triangles; where both subsets are the whole
+    mesh, the positions themselves (the same array, not a copy)."""
     di = np.asarray(dof_indices, dtype=np.int64)
     # identity subsets (the whole mesh) map positions to themselves: the
     # array itself where both are

@@ -18,9 +18,11 @@ from .kernels import kernels as KERNELS
 
 TILE = N.TRI_TILE
 LANES = 64
-# points of the rules with a triangle form: a lane keeps every point of its
-# triangle, its accumulators and a source triangle's record in registers,
-# and with seven points they no longer fit; the last three weights are equal
+# points of the rules with a triangle form, whose last three weights are equal:
+# a lane keeps every point of its triangle, its accumulators and a source
+# triangle's record in registers, which seven points exceed (the form with one
+# observation point a lane, TriToPtFarfield, has room for seven source points, but
+# no Galerkin scatter)
 RULE_POINTS = (3, 4)
 
 
