@@ -350,6 +350,8 @@ class InteriorOp:
 
     def dot_dev(self, v_dev, out=None, prec=None):
         out = self.farfield.dot_dev(v_dev, out, prec)
+        if not self.n_blocks:       # no point is close to a triangle
+            return out
         N.call('tct_bsr39_spmv', self.farfield.n_obs, N.ptr(self.indptr), N.ptr(self.indices),
                N.ptr(self.blocks), N.ptr(v_dev), N.ptr(out), 1, N.stream_ptr())
         return out
